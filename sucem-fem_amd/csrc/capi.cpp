@@ -394,11 +394,11 @@ int sucem_assemble(sucem_ctx* ctx, sucem_space* s, unsigned which, sucem_system*
       f.mf = 1; f.L = 0; f.U = 1; f.G = op_grid(c, s->s.ndofs, 8);
       h->s.cfg[0] = f;
       h->s.cfg[1] = f;
-      const int cb32 = 256, cb64 = s->s.order == 2 ? 192 : 256;
+      const int cb32 = pt_default_cb<float>(&s->s), cb64 = pt_default_cb<double>(&s->s);
       if (pt_prepare(c, &h->s, cb32) && pt_fits<float>(&s->s, cb32))
-        h->s.cfg[0] = pt_cfg(&s->s, cb32, op_grid(c, s->s.pt[2].npd, 16));
+        h->s.cfg[0] = pt_cfg(&s->s, cb32, op_grid(c, pt_maps(&s->s, cb32).npd, 16));
       if (pt_prepare(c, &h->s, cb64) && pt_fits<double>(&s->s, cb64))
-        h->s.cfg[1] = pt_cfg(&s->s, cb64, op_grid(c, s->s.pt[cb64 == 192 ? 1 : 2].npd, 16));
+        h->s.cfg[1] = pt_cfg(&s->s, cb64, op_grid(c, pt_maps(&s->s, cb64).npd, 16));
     }
   } catch (...) {
     delete h;
@@ -523,7 +523,7 @@ int sucem_system_patch_info(sucem_ctx* ctx, sucem_system* sys, int cb, int64_t* 
   c->use();
   SUCEM_CHECK(pt_prepare(c, &sys->s, cb), SUCEM_ERR_UNSUPPORTED,
               "patch operator: orders 1 and 2, patches of at most 65535 products");
-  const PatchMaps& m = sys->s.space->pt[cb == 128 ? 0 : (cb == 192 ? 1 : 2)];
+  const PatchMaps& m = pt_maps(sys->s.space, cb);
   info6_h[0] = m.np; info6_h[1] = m.nu; info6_h[2] = m.npd; info6_h[3] = m.npe;
   info6_h[4] = m.lds; info6_h[5] = m.maxfr;
   API_END

@@ -108,7 +108,7 @@ struct Space {
   int pt_state = 0;                     // 0 not built, 1 built, -1 space unsuited
   int pt_max_lds = 0;                   // LDS bytes per workgroup of the device
   DBuf<int32_t> pt_cell, pt_face, pt_fmeta;
-  PatchMaps pt[3];                      // patches of 128, 192, 256 cells
+  PatchMaps pt[4];                      // patches of 128, 192, 256 and 64 cells
 };
 
 // SpMV launch configuration: lanes per row, loads per lane, blocks (0 = heuristic).

@@ -79,6 +79,35 @@ __device__ __forceinline__ void element_product(const R* a, const typename C2<R>
   (pair_step<R, ORDER, P>(a, xl, acc, std::make_integer_sequence<int, 12>{}), ...);
 }
 
+// Rows [I0, I1) of the element product (all of their columns), for a group of waves that
+// splits a cell's rows: the entries that couple two groups are formed in both.
+template <int NLOC>
+constexpr int pair_of(int i, int j) {
+  return i <= j ? i * NLOC - i * (i - 1) / 2 + (j - i) : j * NLOC - j * (j - 1) / 2 + (i - j);
+}
+
+template <typename R, int ORDER, int I, int J, int I0, int... K>
+__device__ __forceinline__ void row_step(const R* a, const typename C2<R>::T* xl,
+                                         typename C2<R>::T* acc,
+                                         std::integer_sequence<int, K...> ks) {
+  constexpr int P = pair_of<MfTab<ORDER>::NLOC>(I, J);
+  if constexpr (pair_nonzero<ORDER, P>(ks)) {
+    R kij = R(0);
+    (k_term<R, ORDER, P, K>(kij, a), ...);
+    acc[I - I0].x += kij * xl[J].x;
+    acc[I - I0].y += kij * xl[J].y;
+  }
+}
+
+template <typename R, int ORDER, int I0, int... E>
+__device__ __forceinline__ void element_rows(const R* a, const typename C2<R>::T* xl,
+                                             typename C2<R>::T* acc,
+                                             std::integer_sequence<int, E...>) {
+  constexpr int N = MfTab<ORDER>::NLOC;
+  (row_step<R, ORDER, I0 + E / N, E % N, I0>(a, xl, acc,
+                                             std::make_integer_sequence<int, 12>{}), ...);
+}
+
 // Half of the rows at a time (HALF 0: rows i < N/2, HALF 1: rows >= N/2): only that
 // half's accumulators are live, which lowers the register count (more waves per SIMD)
 // at the price of forming the K entries that couple the halves twice.

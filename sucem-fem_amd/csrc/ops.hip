@@ -439,10 +439,10 @@ SpmvCfg sys_cfg(Context* c, const System* sys) {
   // (FP64 order 2: 192 cells, else 256), when the space suits it; the choice is kept on
   // the system (its maps and coefficients are lazily built caches of the system).
   System* ms = const_cast<System*>(sys);
-  const int cb = (sys->space->order == 2 && sizeof(R) == 8) ? 192 : 256;
+  const int cb = pt_default_cb<R>(sys->space);
   if (sys->space->nloc == 6 || sys->space->nloc == 20) {
     if (pt_prepare(c, ms, cb) && pt_fits<R>(sys->space, cb)) {
-      const int64_t npd = sys->space->pt[cb == 192 ? 1 : 2].npd;
+      const int64_t npd = pt_maps(sys->space, cb).npd;
       SpmvCfg f = pt_cfg(sys->space, cb, op_grid(c, std::max<int64_t>(npd, 1), 16));
       ms->cfg[sizeof(R) == 4 ? 0 : 1] = f;
       return f;
@@ -523,7 +523,7 @@ SpmvCfg tune_sys(Context* c, System* sys, int reps) {
     // patch operator: element products summed per patch of cells in LDS + shared-DOF sums
     for (int cb : {128, 192, 256}) {
       if ((s->order == 1 && cb != 256) || !pt_prepare(c, sys, cb) || !pt_fits<R>(s, cb)) continue;
-      const int64_t npd = s->pt[cb == 128 ? 0 : (cb == 192 ? 1 : 2)].npd;
+      const int64_t npd = pt_maps(s, cb).npd;
       for (int pc : {4, 16}) {
         SpmvCfg f = pt_cfg(s, cb, op_grid(c, std::max<int64_t>(npd, 1), pc));
         try {

@@ -29,7 +29,7 @@ template <typename R>
 void mf_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const void* x, void* y,
               const void* w, int epi, const RedSite& rs, const SpmvCfg& f);
 
-// patch operator (patch.hip) with patches of cb cells (128, 192, 256): pt_prepare before
+// patch operator (patch.hip) with patches of cb cells (64, 128, 192, 256): pt_prepare before
 // the first pt_apply with that cb on a system; false when the space does not suit it
 bool pt_prepare(Context* c, System* sys, int cb);
 template <typename R>
@@ -50,6 +50,11 @@ const void* pt_partials(const System* sys);
 // whether the patch kernel's LDS need in precision R fits the device
 template <typename R>
 bool pt_fits(const Space* s, int cb);
+// cells per patch of the patch operator where none was set or tuned
+template <typename R>
+int pt_default_cb(const Space* s);
+// the maps of patches of cb cells (prepared)
+const PatchMaps& pt_maps(const Space* s, int cb);
 // the cfg of the (prepared) patch operator with a partial-sum grid of G blocks
 SpmvCfg pt_cfg(const Space* s, int cb, int G);
 

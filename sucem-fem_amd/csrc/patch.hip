@@ -3,14 +3,14 @@
 // The per-cell form (matfree.hip) writes every element product to HBM and reads it back
 // in a second kernel that sums each DOF's products.  Here the cells are ordered along a
 // Morton curve of their centroids and cut into patches of CB consecutive cells (compact
-// clusters of the mesh; CB = 128, 192 or 256, chosen by the autotuner), one workgroup
-// per patch:
+// clusters of the mesh; CB = 128, 192 or 256, chosen by the autotuner, or 64 on small
+// meshes), one workgroup per patch:
 //
 //  1. the patch's DOFs ("patch DOFs": the union of its cells' DOFs, ~1.4 per DOF of the
 //     mesh) are gathered from x into LDS once;
 //  2. each thread forms its cell's element product from the LDS copy (the same
 //     instruction-folded element matrix as the per-cell form), the boundary faces of the
-//     patch their ABC products;
+//     patch their ABC products (64-cell patches: four threads per cell, five rows each);
 //  3. every product is stored in LDS at its place in the patch's DOF-sorted order, and
 //     each patch DOF's segment is summed in that fixed order.  A DOF that lies in this
 //     patch only (about two thirds of them) is finished: its row of y is written (PEC row
@@ -38,15 +38,7 @@ namespace sucem {
 namespace {
 
 constexpr int TB = 256;    // threads of the set-up kernels and of k_mf_psum
-// patch DOFs per thread and batch in k_mf_patch: of the x gather (UB) and of the segment
-// sums (UD).  Patches of 256 cells hold about 2,300 DOFs at order 2, so 10 per thread
-// takes them in one batch; measured per FP32 application at 40^3, order 2: 8 / 10 / 12 /
-// 14 / 16 -> 64.6 / 59.9 / 60.5 / 60.5 / 62.0 us.
-constexpr int UB = 10;
-constexpr int UD = 10;
-constexpr int kCbs[3] = {128, 192, 256};   // cells per patch = threads of k_mf_patch
-
-int cb_slot(int cb) { return cb == 128 ? 0 : (cb == 192 ? 1 : (cb == 256 ? 2 : -1)); }
+int cb_slot(int cb) { return cb == 128 ? 0 : (cb == 192 ? 1 : (cb == 256 ? 2 : (cb == 64 ? 3 : -1))); }
 
 __device__ __forceinline__ uint32_t spread10(uint32_t v) {
   v &= 0x3ffu;
@@ -282,12 +274,46 @@ __device__ __forceinline__ void epilogue(double2& d1, double2& d2, C v, C wv) {
   d2.x += yd.x * yd.x + yd.y * yd.y;
 }
 
+// Threads of a patch of CB cells: one per cell, or (64-cell patches, order 2, for meshes too
+// small to fill the device) one per cell and quarter of its rows.
+constexpr int patch_slabs(int cb) { return cb == 64 ? 4 : 1; }
+constexpr int patch_threads(int cb) { return cb * patch_slabs(cb); }
+// Patch DOFs per thread and batch (see k_mf_patch): enough for one batch on the Kuhn
+// meshes, where patches of 64 / 128 / 192 / 256 cells hold at most about 810 / 1,410 /
+// 1,970 / 2,560 DOFs at order 2 and patches of 256 cells 610 at order 1.
+constexpr int patch_batch(int order, int cb) {
+  return order == 1 ? 3 : (cb == 64 ? 4 : (cb == 256 ? 10 : 11));
+}
+
+// Waves per SIMD that the registers have to allow (512 / waves registers per lane).
+constexpr int patch_waves(int order, bool fp32) {
+  return order == 1 ? 4 : (fp32 ? 3 : 2);
+}
+
+// T[idx] by a 32-bit byte offset from a uniform base (idx * sizeof(T) below 2^32)
+template <typename T>
+__device__ __forceinline__ T at32(const T* base, uint32_t idx) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) +
+                                     (uint32_t)(idx * (uint32_t)sizeof(T)));
+}
+
 // One workgroup per patch (XCD-aware order: consecutive patches share x entries and
 // should share an L2); Gp = grid (a multiple of 8), Gt = all block partials of the
 // operator (Gp + the grid of k_mf_psum).  EPI 3 (COCG, shared rows left as partial sums)
 // reduces p.Ap; EPI 4 is EPI 3 for two paired real systems (per-part products).
+//
+// The kernel is bound by the latency of its chain of dependent loads (DOF ids -> x -> LDS
+// -> products -> LDS -> rows), so every phase issues all of its loads before it uses the
+// first of them: indexes past the end are clamped instead of branched around (a
+// predicated load costs a branch, and the loads behind it wait for it), the segment
+// bounds, destinations, epilogue operands and mask bytes of a whole batch are in flight
+// together, and the first two products of every segment are read before any is summed.
+// Per application in the solve at 40^3 order 2: FP32 60.9 -> 54.8 us, FP64 111 -> 97.8 us
+// (there the places that are read again instead of held also take the kernel from 274 to
+// 246 registers, one wave per SIMD to two); 17 x 22 x 13 boxes with the 64-cell patches
+// 24.4 -> 14.7 and 26.7 -> 17.2 us.
 template <typename R, int ORDER, int NFD, int EPI, int CB>
-__global__ __launch_bounds__(CB) void k_mf_patch(
+__global__ __launch_bounds__(patch_threads(CB), patch_waves(ORDER, sizeof(R) == 4)) void k_mf_patch(
     int64_t np, int Gp, int Gt, int64_t nc, int64_t nbf, int lds_main, const R* __restrict__ coef,
     const uint32_t* __restrict__ lp, const int32_t* __restrict__ uptr,
     const int32_t* __restrict__ pdof, const uint16_t* __restrict__ pseg,
@@ -303,168 +329,215 @@ __global__ __launch_bounds__(CB) void k_mf_patch(
   constexpr bool PR = EPI == 4;
   constexpr int NLOC = MfTab<ORDER>::NLOC;
   constexpr int KK = NFD * NFD;
+  constexpr int SL = patch_slabs(CB), ROWS = NLOC / SL, NT = CB * SL;
+  static_assert(ROWS * SL == NLOC, "whole rows per slab");
+  constexpr int UB = patch_batch(ORDER, CB);
+  // w.y over the finished rows and the partial sums; FP64 COCG takes the element quadratic
+  // forms instead (in FP32 their registers cost a wave per SIMD)
+  constexpr bool QF = E3 && sizeof(R) == 8;
+  constexpr bool WY = EPI != 0 && !QF;
   extern __shared__ double2 smem_[];
   C* sm = reinterpret_cast<C*>(smem_);
   const int lb = xcd_block(Gp);
   const int64_t p = lb;
+  const int tid = threadIdx.x;
   double2 d1 = make_double2(0.0, 0.0), d2 = make_double2(0.0, 0.0);
   if (p < np) {   // uniform over the workgroup
     const int u0 = uptr[p], nu = uptr[p + 1] - u0;
-    const int64_t r = p * CB + threadIdx.x;
+    const int slab = SL == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / CB);
+    const int64_t r = p * CB + (SL == 1 ? tid : tid % CB);
     const bool has = r < nc;
+    const uint32_t rc = (uint32_t)(has ? r : nc - 1);   // a cell of this patch in any case
+    const int32_t* pd = pdof + u0;
     // FP32: the cell's coefficients and LDS places do not depend on x, so their loads go
     // out with the x gather below and the two round trips overlap (in FP64 the held
     // registers would cost a wave per SIMD)
-    constexpr bool PF = sizeof(R) == 4;
+    constexpr bool PF = sizeof(R) == 4 || SL > 1 || ORDER == 1;
     R pa[12];
     uint32_t pli[NLOC];
-    if (PF && has) {
+    auto load_cell = [&] {
 #pragma unroll
-      for (int k = 0; k < 12; ++k) pa[k] = coef[k * nc + r];
+      for (int k = 0; k < 12; ++k) pa[k] = at32(coef + k * nc, rc);
 #pragma unroll
-      for (int i = 0; i < NLOC; ++i) pli[i] = lp[(int64_t)i * nc + r];
-    }
-    // batches of UB entries per thread: all id loads, then all x loads, in flight together
-    for (int j0 = 0; j0 < nu; j0 += UB * CB) {
-      int dv[UB];
+      for (int i = 0; i < NLOC; ++i) pli[i] = at32(lp + i * nc, rc);
+    };
+    int dv[UB];
+    auto load_dofs = [&](int j0) {
 #pragma unroll
-      for (int q = 0; q < UB; ++q) {
-        const int j = j0 + q * CB + threadIdx.x;
-        dv[q] = j < nu ? pdof[u0 + j] : -1;
-      }
+      for (int q = 0; q < UB; ++q) dv[q] = at32(pd, (uint32_t)min(j0 + q * NT + tid, nu - 1));
+    };
+    load_dofs(0);
+    if constexpr (PF) load_cell();
+    for (int j0 = 0; j0 < nu; j0 += UB * NT) {
+      if (j0) load_dofs(j0);
       C xv[UB];
 #pragma unroll
-      for (int q = 0; q < UB; ++q) xv[q] = dv[q] >= 0 ? x[dv[q]] : mk(R(0), R(0));
+      for (int q = 0; q < UB; ++q) xv[q] = x[dv[q]];
 #pragma unroll
       for (int q = 0; q < UB; ++q) {
-        const int j = j0 + q * CB + threadIdx.x;
+        const int j = j0 + q * NT + tid;
         if (j < nu) sm[j] = xv[q];
       }
     }
     __syncthreads();
-    C acc[NLOC];
-    if (has) {
-      R a[12];
-      C xl[NLOC];
-      if constexpr (PF) {
-#pragma unroll
-        for (int k = 0; k < 12; ++k) a[k] = pa[k] * (k < 6 ? ct : cs) * R(1.0 / MfTab<ORDER>::den);
-#pragma unroll
-        for (int i = 0; i < NLOC; ++i) xl[i] = sm[pli[i] & 0xffffu];
-      } else {
-#pragma unroll
-        for (int k = 0; k < 12; ++k)
-          a[k] = coef[k * nc + r] * (k < 6 ? ct : cs) * R(1.0 / MfTab<ORDER>::den);
-#pragma unroll
-        for (int i = 0; i < NLOC; ++i) xl[i] = sm[lp[(int64_t)i * nc + r] & 0xffffu];
-      }
-#pragma unroll
-      for (int i = 0; i < NLOC; ++i) acc[i] = mk(R(0), R(0));
-      element_product<R, ORDER>(a, xl, acc, std::make_integer_sequence<int, MfTab<ORDER>::NP>{});
-      if constexpr (E3 && sizeof(R) == 8) {
-        // p.Ap as the sum of the element quadratic forms x_c^T K_c x_c (w = x in COCG;
-        // x is zero on masked rows there, so the masked rows add nothing either way).
-        // FP64 only: in FP32 the extra registers cost a wave per SIMD, and the sums of
-        // the finished rows and partial sums below are cheaper.
-#pragma unroll
-        for (int i = 0; i < NLOC; ++i) {
-          const double2 xd = to_d(xl[i]), yd = to_d(acc[i]);
-          if constexpr (PR) {
-            d1.x += xd.x * yd.x;
-            d1.y += xd.y * yd.y;
-          } else {
-            d1.x += xd.x * yd.x - xd.y * yd.y;
-            d1.y += xd.x * yd.y + xd.y * yd.x;
-          }
-        }
-      }
-    }
     // the patch's boundary faces, one (face, row) pair per thread and pass, staged in LDS
     // behind the x copy (stage[id]) until the x copy may be overwritten
     const int f0 = fptr[p], nfr = (fptr[p + 1] - f0) * NFD;
     C* stage = sm + lds_main;
-    for (int id = threadIdx.x; id < nfr; id += CB) {
-      {
-        const int64_t fp = f0 + id / NFD;
-        const int a = id % NFD;
-        const int mt = fmeta[fp];
-        const int64_t rk = mt >> 2;
-        const int lf = mt & 3;
-        R hk[6];
+    for (int id = tid; id < nfr; id += NT) {
+      if (c0 == R(0)) {   // no ABC term: the faces' products are zero
+        stage[id] = mk(R(0), R(0));
+        continue;
+      }
+      const int64_t fp = f0 + id / NFD;
+      const int a = id % NFD;
+      const int mt = fmeta[fp];
+      const uint32_t rk = (uint32_t)(mt >> 2);
+      const int lf = mt & 3;
+      R hk[6];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) hk[k] = hf[k * nbf + fp];
-        const double* rf = ref_face + lf * 6 * KK + a * NFD;
-        C v = mk(R(0), R(0));
+      for (int k = 0; k < 6; ++k) hk[k] = hf[k * nbf + fp];
+      const double* rf = ref_face + lf * 6 * KK + a * NFD;
+      const int32_t* fd = face_dofs + lf * NFD;
+      uint32_t li[NFD];
 #pragma unroll
-        for (int b = 0; b < NFD; ++b) {
-          R m = R(0);
+      for (int b = 0; b < NFD; ++b) li[b] = lp[(int64_t)fd[b] * nc + rk] & 0xffffu;
+      C v = mk(R(0), R(0));
 #pragma unroll
-          for (int k = 0; k < 6; ++k) m += hk[k] * (R)rf[k * KK + b];
-          const uint32_t li = lp[(int64_t)face_dofs[lf * NFD + b] * nc + rk] & 0xffffu;
-          const C xb = sm[li];
-          v.x += m * xb.x;
-          v.y += m * xb.y;
-        }
-        stage[id] = mk(-c0 * v.y, c0 * v.x);
-        if constexpr (E3 && sizeof(R) == 8) {
-          const C xa = sm[lp[(int64_t)face_dofs[lf * NFD + a] * nc + rk] & 0xffffu];
-          const double2 xd = to_d(xa), yd = to_d(stage[id]);
-          if constexpr (PR) {
-            d1.x += xd.x * yd.x;
-            d1.y += xd.y * yd.y;
-          } else {
-            d1.x += xd.x * yd.x - xd.y * yd.y;
-            d1.y += xd.x * yd.y + xd.y * yd.x;
-          }
-        }
+      for (int b = 0; b < NFD; ++b) {
+        R m = R(0);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) m += hk[k] * (R)rf[k * KK + b];
+        const C xb = sm[li[b]];
+        v.x += m * xb.x;
+        v.y += m * xb.y;
+      }
+      const C sv = mk(-c0 * v.y, c0 * v.x);
+      stage[id] = sv;
+      if constexpr (QF) {
+        const C xa = sm[lp[(int64_t)fd[a] * nc + rk] & 0xffffu];
+        dot_acc(d1, to_d(xa), to_d(sv), PR);
       }
     }
+    C acc[ROWS];
+    if (has) {
+      if constexpr (!PF) load_cell();
+#pragma unroll
+      for (int k = 0; k < 12; ++k) pa[k] *= (k < 6 ? ct : cs) * R(1.0 / MfTab<ORDER>::den);
+      C xl[NLOC];
+#pragma unroll
+      for (int i = 0; i < NLOC; ++i) xl[i] = sm[pli[i] & 0xffffu];
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i) acc[i] = mk(R(0), R(0));
+      auto rows = [&](auto s_) {
+        constexpr int S = decltype(s_)::value;
+        if constexpr (SL == 1)
+          element_product<R, ORDER>(pa, xl, acc,
+                                    std::make_integer_sequence<int, MfTab<ORDER>::NP>{});
+        else
+          element_rows<R, ORDER, S * ROWS>(pa, xl, acc,
+                                           std::make_integer_sequence<int, ROWS * NLOC>{});
+      };
+      if constexpr (SL == 1) {
+        rows(std::integral_constant<int, 0>{});
+      } else {
+        if (slab == 0) rows(std::integral_constant<int, 0>{});
+        else if (slab == 1) rows(std::integral_constant<int, 1>{});
+        else if (slab == 2) rows(std::integral_constant<int, 2>{});
+        else rows(std::integral_constant<int, 3>{});
+      }
+    }
+
+    // where this thread's products go: read again, from an offset the compiler does not
+    // know to be rc, so that the places are not held over the element product
+    uint32_t rq = rc;
+    asm volatile("" : "+v"(rq));
+    uint32_t pl[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) pl[i] = at32(lp + (slab * ROWS + i) * nc, rq);
+    if constexpr (QF) {
+      // p.Ap as the sum of the element quadratic forms x_c^T K_c x_c (w = x in COCG; x is
+      // zero on masked rows there, so the masked rows add nothing either way), x from the
+      // LDS copy again
+      if (has) {
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i)
+          dot_acc(d1, to_d(sm[pl[i] & 0xffffu]), to_d(acc[i]), PR);
+      }
+    }
+    int lo[UB], hi[UB], out[UB];
+    int tq = tid;   // (likewise: the ids of the gather are not held either)
+    asm volatile("" : "+v"(tq));
+    auto load_ids = [&](int j0) {
+#pragma unroll
+      for (int q = 0; q < UB; ++q) {
+        const uint32_t j = (uint32_t)min(j0 + q * NT + tq, nu - 1);
+        hi[q] = (int)at32(pseg + u0, j);
+        lo[q] = (int)at32(pseg + u0, j ? j - 1 : 0);
+        out[q] = at32(pout + u0, j);
+        dv[q] = at32(pd, j);
+      }
+    };
     __syncthreads();   // every read of the x copy is done: the products overwrite it
     if (has) {
 #pragma unroll
-      for (int i = 0; i < NLOC; ++i) sm[lp[(int64_t)i * nc + r] >> 16] = acc[i];
+      for (int i = 0; i < ROWS; ++i) sm[pl[i] >> 16] = acc[i];
     }
-    int lo[UD], hi[UD], out[UD], dv[UD];
-    auto load_ids = [&](int j0) {
-#pragma unroll
-      for (int q = 0; q < UD; ++q) {
-        const int j = j0 + q * CB + threadIdx.x;
-        const bool in = j < nu;
-        lo[q] = (in && j) ? (int)pseg[u0 + j - 1] : 0;
-        hi[q] = in ? (int)pseg[u0 + j] : 0;
-        out[q] = in ? pout[u0 + j] : 0;
-        dv[q] = in ? pdof[u0 + j] : 0;
-      }
-    };
-    if constexpr (PF) load_ids(0);   // before the barrier: the loads overlap the wait
-    for (int id = threadIdx.x; id < nfr; id += CB) sm[fpos[(int64_t)f0 * NFD + id]] = stage[id];
+    load_ids(0);   // in flight over the barrier
+    for (int id = tid; id < nfr; id += NT) sm[at32(fpos + (int64_t)f0 * NFD, (uint32_t)id)] = stage[id];
     __syncthreads();
-    for (int j0 = 0; j0 < nu; j0 += UD * CB) {
-      if (!PF || j0) load_ids(j0);
+    for (int j0 = 0; j0 < nu; j0 += UB * NT) {
+      if (j0) load_ids(j0);
+      C wv[UB];
+      if constexpr (WY) {
 #pragma unroll
-      for (int q = 0; q < UD; ++q) {
-        C v = mk(R(0), R(0));
-        for (int t = lo[q]; t < hi[q]; ++t) {
+        for (int q = 0; q < UB; ++q) wv[q] = w[dv[q]];
+      }
+      uint8_t off[UB];
+#pragma unroll
+      for (int q = 0; q < UB; ++q) off[q] = 0;
+      if (mask) {
+#pragma unroll
+        for (int q = 0; q < UB; ++q) off[q] = mask[dv[q]];
+      }
+      C va[UB], vb[UB];
+#pragma unroll
+      for (int q = 0; q < UB; ++q) {
+        if (j0 + q * NT + tq == 0) lo[q] = 0;
+        va[q] = sm[lo[q]];
+        vb[q] = sm[min(lo[q] + 1, hi[q] - 1)];
+      }
+#pragma unroll
+      for (int q = 0; q < UB; ++q) {
+        C v = va[q];
+        if (lo[q] + 1 < hi[q]) {
+          v.x += vb[q].x;
+          v.y += vb[q].y;
+        }
+        for (int t = lo[q] + 2; t < hi[q]; ++t) {
           const C a = sm[t];
           v.x += a.x;
           v.y += a.y;
         }
-        if (hi[q] > 0) {   // an entry of this patch (segments are never empty)
-          if (out[q] >= 0) {
-            part[out[q]] = v;
-            // FP32: x.y over the partial sums (linear in y; x is zero on masked rows)
-            if constexpr (E3 && sizeof(R) == 4) epilogue<PR ? 4 : 1>(d1, d2, v, w[dv[q]]);
-          } else {
-            if (mask && mask[dv[q]]) v = mk(R(0), R(0));
-            y[dv[q]] = v;
-            if constexpr (EPI == 1 || EPI == 2) epilogue<EPI>(d1, d2, v, w[dv[q]]);
-            else if constexpr (E3 && sizeof(R) == 4) epilogue<PR ? 4 : 1>(d1, d2, v, w[dv[q]]);
+        if (j0 + q * NT + tq < nu) {
+          const bool own = out[q] < 0;
+          if (own && off[q]) v = mk(R(0), R(0));
+          C* dst = own ? y + dv[q] : part + out[q];
+          *dst = v;
+          // FP32 COCG: w.y over the partial sums too (linear in y; w is zero on masked rows)
+          if constexpr (WY) {
+            if (own || E3) epilogue<E3 ? (PR ? 4 : 1) : EPI>(d1, d2, v, wv[q]);
           }
         }
       }
     }
   }
-  if (EPI) block_partials<CB>(rs, Gt, lb, d1, d2);
+  if constexpr (E3) {
+    d1 = block_sum<NT>(d1);
+    if (tid == 0) rs.part[lb] = d1;
+  } else if constexpr (EPI != 0) {
+    block_partials<NT>(rs, Gt, lb, d1, d2);
+  }
 }
 
 // Shared DOFs: y_d = sum of the partial sums of its patches, in patch order.
@@ -782,15 +855,16 @@ void launch_patch(Context* c, const System* sys, const PatchMaps& pm, Coef k,
   }
   const R c0 = (sys->which & SUCEM_MAT_S0) ? (R)k.s0 : R(0);
   const size_t lds = (size_t)(pm.lds + pm.maxfr) * sizeof(C);
+  constexpr int nt = patch_threads(CB);
 #define PT_ARGS pm.np, Gp, Gt, s->mesh->nc, s->nbf, pm.lds, coef, pm.lp.p, pm.uptr.p, pm.dof.p, \
                 pm.seg.p, pm.out.p, pm.fptr.p, s->pt_fmeta.p, pm.fpos.p, hf, s->ref_face_dofs.p, \
                 s->ref_face.p, (R)k.s, (R)k.t, c0, mask, (const C*)x, (C*)y, (C*)sys->pt_part.p, \
                 (const C*)w, rs
-  if (epi == 0) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 0, CB>), Gp, CB, lds, c->stream, PT_ARGS);
-  else if (epi == 1) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 1, CB>), Gp, CB, lds, c->stream, PT_ARGS);
-  else if (epi == 2) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 2, CB>), Gp, CB, lds, c->stream, PT_ARGS);
-  else if (epi == 3) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 3, CB>), Gp, CB, lds, c->stream, PT_ARGS);
-  else SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 4, CB>), Gp, CB, lds, c->stream, PT_ARGS);
+  if (epi == 0) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 0, CB>), Gp, nt, lds, c->stream, PT_ARGS);
+  else if (epi == 1) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 1, CB>), Gp, nt, lds, c->stream, PT_ARGS);
+  else if (epi == 2) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 2, CB>), Gp, nt, lds, c->stream, PT_ARGS);
+  else if (epi == 3) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 3, CB>), Gp, nt, lds, c->stream, PT_ARGS);
+  else SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 4, CB>), Gp, nt, lds, c->stream, PT_ARGS);
 #undef PT_ARGS
 }
 
@@ -799,7 +873,7 @@ void launch_patch(Context* c, const System* sys, const PatchMaps& pm, Coef k,
 bool pt_prepare(Context* c, System* sys, int cb) {
   Space* s = sys->space;
   const int slot = cb_slot(cb);
-  SUCEM_CHECK(slot >= 0, SUCEM_ERR_INVALID, "cells per patch must be 128, 192 or 256");
+  SUCEM_CHECK(slot >= 0, SUCEM_ERR_INVALID, "cells per patch must be 64, 128, 192 or 256");
   {
     std::lock_guard<std::mutex> hold(s->lazy);
     if (s->pt_state == 0) pt_build_order(c, s);
@@ -845,6 +919,28 @@ bool pt_fits(const Space* s, int cb) {
 template bool pt_fits<float>(const Space*, int);
 template bool pt_fits<double>(const Space*, int);
 
+// Order-2 meshes of up to this many cells run on 64-cell patches with four waves per patch
+// (a quarter of the cells' rows each): with 192 or 256 cells they would fill less than one
+// workgroup per CU, and the operator is then one workgroup's chain of loads.  Operator in
+// the solve, 256 / 192 cells (FP32 / FP64) against 64, us: 6,468 cells 19.8 / 22.8 -> 12.5 /
+// 13.9; 29,172 cells 20.9 / 24.5 -> 14.7 / 17.2; 82,944 cells 24.6 / 29.9 against 23.8 /
+// 34.3; 162,000 cells 30.3 / 48.0 against 34.7 / 52.2.  Order 1 gains nothing (48,000
+// cells: 9.8 / 10.3 against 10.5 / 11.1).
+constexpr int64_t kSmallCells = 50000;
+template <typename R>
+int pt_default_cb(const Space* s) {
+  if (s->order == 2 && s->mesh->nc <= kSmallCells) return 64;
+  return (s->order == 2 && sizeof(R) == 8) ? 192 : 256;
+}
+template int pt_default_cb<float>(const Space*);
+template int pt_default_cb<double>(const Space*);
+
+const PatchMaps& pt_maps(const Space* s, int cb) {
+  const int slot = cb_slot(cb);
+  SUCEM_CHECK(slot >= 0 && s->pt[slot].cb == cb, SUCEM_ERR_INVALID, "patch operator not prepared");
+  return s->pt[slot];
+}
+
 SpmvCfg pt_cfg(const Space* s, int cb, int G) {
   SpmvCfg f;
   f.mf = 2;
@@ -873,7 +969,8 @@ void pt_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const 
               "the patch operator needs more LDS per workgroup than the device has");
   SUCEM_CHECK((int64_t)sys->pt_part.n >= pm.npe, SUCEM_ERR_INVALID, "patch operator not prepared");
   if (s->order == 2) {
-    if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
+    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
+    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
     else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
     else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
   } else {
@@ -910,7 +1007,8 @@ void pt_apply_deferred(Context* c, const System* sys, Coef k, const uint8_t* mas
   const PatchMaps& pm = sys->space->pt[cb_slot(f.U)];
   const int epi = rs.paired ? 4 : 3;
   if (sys->space->order == 2) {
-    if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
+    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
+    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
     else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
     else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
   } else {
