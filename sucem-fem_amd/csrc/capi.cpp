@@ -35,6 +35,9 @@ void export_lhs(Context* c, const System* sys, double k0, double2* out_d);
 
 using namespace sucem;
 
+// workspace slots of the point entry points: points, their cells, values, DOFs / indexes
+constexpr int kWsPoints = 80;
+
 #define API_BEGIN try {
 #define API_END                                        \
   return SUCEM_OK;                                     \
@@ -553,8 +556,8 @@ int sucem_locate_points(sucem_ctx* ctx, sucem_space* s, int64_t n, const double*
   Context* c = &ctx->c;
   c->use();
   if (n == 0) return SUCEM_OK;
-  DBuf<double> pts(n * 3);
-  DBuf<int32_t> cell(n);
+  const Scratch<double> pts(c, kWsPoints, n * 3);
+  const Scratch<int32_t> cell(c, kWsPoints + 1, n);
   h2d(c, pts.p, pts_h, n * 3);
   locate_points(c, &s->s, n, pts.p, cell.p);
   std::vector<int32_t> h(n);
@@ -578,8 +581,10 @@ int sucem_basis_at_points(sucem_ctx* ctx, sucem_space* s, int64_t n, const doubl
   c->use();
   if (n == 0) return SUCEM_OK;
   const int nloc = s->s.nloc;
-  DBuf<double> pts(n * 3), vals(n * nloc * 3);
-  DBuf<int32_t> cell(n);
+  const Scratch<double> pts(c, kWsPoints, n * 3);
+  const Scratch<int32_t> cell(c, kWsPoints + 1, n);
+  const Scratch<double> vals(c, kWsPoints + 2, n * nloc * 3);
+  const Scratch<int64_t> dofs(c, kWsPoints + 3, dofs_h ? n * nloc : 0);
   h2d(c, pts.p, pts_h, n * 3);
   locate_points(c, &s->s, n, pts.p, cell.p);
   std::vector<int32_t> h(n);
@@ -587,16 +592,9 @@ int sucem_basis_at_points(sucem_ctx* ctx, sucem_space* s, int64_t n, const doubl
   c->sync();
   for (int64_t i = 0; i < n; ++i)
     SUCEM_CHECK(h[i] != 0x7fffffff, SUCEM_ERR_OUTSIDE, "point is outside the mesh");
-  basis_at_points(c, &s->s, n, pts.p, cell.p, vals.p);
-  d2h(c, vals_h, vals.p, vals.n);
-  if (dofs_h) {
-    std::vector<int32_t> cd(s->s.mesh->nc * 0 + nloc);
-    for (int64_t i = 0; i < n; ++i) {
-      d2h(c, cd.data(), s->s.cell_dofs.p + (int64_t)h[i] * nloc, nloc);
-      c->sync();
-      for (int k = 0; k < nloc; ++k) dofs_h[i * nloc + k] = cd[k];
-    }
-  }
+  basis_at_points(c, &s->s, n, pts.p, cell.p, vals.p, dofs.p);
+  d2h(c, vals_h, vals.p, (size_t)n * nloc * 3);
+  if (dofs_h) d2h(c, dofs_h, dofs.p, (size_t)n * nloc);
   c->sync();
   API_END
 }
@@ -616,9 +614,10 @@ int sucem_rhs_point_sources(sucem_ctx* ctx, sucem_space* s, int64_t nsrc, const 
     SUCEM_CHECK(r >= 0 && r < nrhs, SUCEM_ERR_INVALID, "source rhs index out of range");
     rhs[i] = (int32_t)r;
   }
-  DBuf<double> pos(nsrc * 3);
-  DBuf<double2> val(nsrc * 3);
-  DBuf<int32_t> rhs_d(nsrc), cell(nsrc);
+  const Scratch<double> pos(c, kWsPoints, nsrc * 3);
+  const Scratch<int32_t> cell(c, kWsPoints + 1, nsrc);
+  const Scratch<double2> val(c, kWsPoints + 2, nsrc * 3);
+  const Scratch<int32_t> rhs_d(c, kWsPoints + 3, nsrc);
   h2d(c, pos.p, pos_h, nsrc * 3);
   h2d(c, val.p, (const double2*)val_h, nsrc * 3);
   h2d(c, rhs_d.p, rhs.data(), nsrc);
@@ -628,8 +627,8 @@ int sucem_rhs_point_sources(sucem_ctx* ctx, sucem_space* s, int64_t nsrc, const 
   c->sync();
   for (int64_t i = 0; i < nsrc; ++i)
     SUCEM_CHECK(h[i] != 0x7fffffff, SUCEM_ERR_OUTSIDE, "point source is outside the mesh");
-  rhs_point_sources(c, &s->s, nsrc, pos.p, val.p, rhs_d.p, cell.p, nrhs,
-                    make_double2(scale_re, scale_im), (double2*)b_d);
+  rhs_point_sources(c, &s->s, nsrc, pos.p, val.p, rhs_d.p, cell.p, nrhs, make_double2(scale_re, scale_im),
+                    (double2*)b_d);
   c->sync();
   API_END
 }

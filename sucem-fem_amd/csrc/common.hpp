@@ -68,8 +68,8 @@ struct DBuf {
 // call and grow when a call needs more, so repeated solves on one context allocate (and
 // free, which synchronises the device) nothing after the first.  A slot is used by one
 // routine at a time: the Krylov solver takes slots [0, 32), the eigen solver [32, 48) (it
-// calls the Krylov solver, so their ranges differ), the batched solver [48, 80).  Calls on
-// one context run one at a time (one host thread per context).
+// calls the Krylov solver, so their ranges differ), the batched solver [48, 80), the point entry
+// points [80, 84).  Calls on one context run one at a time (one host thread per context).
 struct Workspace {
   std::vector<DBuf<unsigned char>> slot;
   // device memory of at least `bytes` bytes in slot k (nullptr for 0 bytes); the contents
@@ -117,6 +117,22 @@ template <typename T>
 inline T* ws_take(Context* c, int k, int64_t count) {
   return (T*)c->ws.get(k, count > 0 ? sizeof(T) * (size_t)count : 0);
 }
+
+// `count` elements for one call: workspace slot k up to 32 MB, beyond that an allocation
+// that is given back with the call (the workspace is not to hold an occasional large call)
+template <typename T>
+struct Scratch {
+  DBuf<T> own;
+  T* p = nullptr;
+  Scratch(Context* c, int k, int64_t count) {
+    if (count > 0 && sizeof(T) * (size_t)count <= (size_t(32) << 20)) {
+      p = ws_take<T>(c, k, count);
+    } else {
+      own.alloc(count > 0 ? (size_t)count : 0);
+      p = own.p;
+    }
+  }
+};
 
 template <typename T>
 inline void h2d(Context* c, T* d, const T* h, size_t n) {

@@ -201,7 +201,7 @@ void rhs_point_sources(Context* c, const Space* s, int64_t nsrc, const double* p
                        const double2* val_d, const int32_t* rhs_d, const int32_t* cell_d,
                        int64_t nrhs, double2 scale, double2* b_d);
 void basis_at_points(Context* c, const Space* s, int64_t n, const double* pts_d,
-                     const int32_t* cell_d, double* vals_d);
+                     const int32_t* cell_d, double* vals_d, int64_t* dofs_d);
 // allocation-free variant of the point-source RHS: staging in a fixed device array
 // (noalloc_init once per device with that device current, at context creation)
 constexpr int64_t kNoAllocSources = 4096;

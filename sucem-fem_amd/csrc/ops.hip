@@ -197,17 +197,42 @@ __global__ void k_csr_identity_dinv(int64_t n, const uint8_t* mask, typename C2<
     dinv[r] = (mask && mask[r]) ? mk(R(0), R(0)) : mk(R(1), R(0));
 }
 
-__global__ void k_locate(int64_t nc, const double* xyz, const int32_t* cells, int64_t n,
-                         const double* pts, double tol, int32_t* out) {
-  for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nc;
-       c += (int64_t)gridDim.x * blockDim.x) {
+// out[p] = the lowest-index cell holding point p (initialised to "not found").  A wave
+// takes 64 consecutive cells and tests 64 points at a time against the cells' common
+// bounding box, so that only points in it meet the cells themselves: one box test per 64
+// cell-point pairs instead of 64 tetrahedron tests (which bound this kernel by FP64
+// arithmetic).  The box is enlarged far beyond the tolerance and the rounding of the
+// tetrahedron test.  51,840 cells, 1,200 to 4,000 points: 586 -> 113 us.
+__global__ __launch_bounds__(TB) void k_locate(int64_t nc, const double* xyz, const int32_t* cells,
+                                               int64_t n, const double* pts, double tol,
+                                               int32_t* out) {
+  const int lane = threadIdx.x & 63;
+  const int64_t wave = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
+  const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
+  for (int64_t c0 = wave * 64; c0 < nc; c0 += nwaves * 64) {
+    const bool live = c0 + lane < nc;
+    const int64_t c = live ? c0 + lane : nc - 1;
     const int32_t* cell = cells + 4 * c;
     const double* x0 = xyz + 3 * (int64_t)cell[0];
-    double J[3][3];
+    double J[3][3], lo[3], hi[3];
+    for (int r = 0; r < 3; ++r) lo[r] = hi[r] = x0[r];
     for (int k = 0; k < 3; ++k) {
       const double* xk = xyz + 3 * (int64_t)cell[k + 1];
-      for (int r = 0; r < 3; ++r) J[r][k] = xk[r] - x0[r];
+      for (int r = 0; r < 3; ++r) {
+        J[r][k] = xk[r] - x0[r];
+        lo[r] = fmin(lo[r], xk[r]);
+        hi[r] = fmax(hi[r], xk[r]);
+      }
     }
+    for (int o = 32; o > 0; o >>= 1)
+      for (int r = 0; r < 3; ++r) {
+        lo[r] = fmin(lo[r], __shfl_xor(lo[r], o));
+        hi[r] = fmax(hi[r], __shfl_xor(hi[r], o));
+      }
+    double grow = 0.0;
+    for (int r = 0; r < 3; ++r)
+      grow = fmax(grow, 1e-6 * (hi[r] - lo[r]) + 1e-9 * fmax(fabs(lo[r]), fabs(hi[r])));
+    for (int r = 0; r < 3; ++r) { lo[r] -= grow; hi[r] += grow; }
     double c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
     double c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
     double c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
@@ -219,20 +244,38 @@ __global__ void k_locate(int64_t nc, const double* xyz, const int32_t* cells, in
                         (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id},
                        {c02 * id, (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id,
                         (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id}};
-    for (int64_t p = 0; p < n; ++p) {
-      double d[3] = {pts[3 * p] - x0[0], pts[3 * p + 1] - x0[1], pts[3 * p + 2] - x0[2]};
-      double l1 = Ji[0][0] * d[0] + Ji[0][1] * d[1] + Ji[0][2] * d[2];
-      double l2 = Ji[1][0] * d[0] + Ji[1][1] * d[1] + Ji[1][2] * d[2];
-      double l3 = Ji[2][0] * d[0] + Ji[2][1] * d[1] + Ji[2][2] * d[2];
-      double l0 = 1.0 - l1 - l2 - l3;
-      if (l0 >= -tol && l1 >= -tol && l2 >= -tol && l3 >= -tol) atomicMin(&out[p], (int32_t)c);
+    const double o0 = x0[0], o1 = x0[1], o2 = x0[2];
+    for (int64_t p0 = 0; p0 < n; p0 += 64) {
+      const int64_t pl = p0 + lane < n ? p0 + lane : n - 1;
+      const double px = pts[3 * pl], py = pts[3 * pl + 1], pz = pts[3 * pl + 2];
+      const bool off = p0 + lane >= n || px < lo[0] || px > hi[0] || py < lo[1] || py > hi[1] ||
+                       pz < lo[2] || pz > hi[2];
+      unsigned long long near = __ballot(!off);
+      while (near) {   // uniform over the wave
+        const int b = __ffsll((long long)near) - 1;
+        near &= near - 1;
+        const double d[3] = {__shfl(px, b) - o0, __shfl(py, b) - o1, __shfl(pz, b) - o2};
+        double l1 = Ji[0][0] * d[0] + Ji[0][1] * d[1] + Ji[0][2] * d[2];
+        double l2 = Ji[1][0] * d[0] + Ji[1][1] * d[1] + Ji[1][2] * d[2];
+        double l3 = Ji[2][0] * d[0] + Ji[2][1] * d[1] + Ji[2][2] * d[2];
+        double l0 = 1.0 - l1 - l2 - l3;
+        if (live && l0 >= -tol && l1 >= -tol && l2 >= -tol && l3 >= -tol)
+          atomicMin(&out[p0 + b], (int32_t)c);
+      }
     }
   }
 }
 
-// Physical basis values N_i(x) = J^-T N^_i(x^) of the cell containing x.
-__device__ void basis_values(const double* xyz, const int32_t* cell, const double* ref_basis,
-                             int nloc, const double* p, double out[20][3]) {
+__global__ void k_fill_i32(int64_t n, int32_t v, int32_t* a) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    a[i] = v;
+}
+
+// Physical value of basis function i, N_i(x) = J^-T N^_i(x^), in the cell containing x.
+__device__ __forceinline__ void basis_value(const double* xyz, const int32_t* cell,
+                                            const double* ref_basis, int i, const double* p,
+                                            double out[3]) {
   const double* x0 = xyz + 3 * (int64_t)cell[0];
   double J[3][3];
   for (int k = 0; k < 3; ++k) {
@@ -256,54 +299,108 @@ __device__ void basis_values(const double* xyz, const int32_t* cell, const doubl
   const double mono[10] = {1.0,           xh[0],         xh[1],         xh[2],
                            xh[0] * xh[0], xh[0] * xh[1], xh[0] * xh[2], xh[1] * xh[1],
                            xh[1] * xh[2], xh[2] * xh[2]};
-  for (int i = 0; i < nloc; ++i) {
-    double nh[3];
-    for (int dd = 0; dd < 3; ++dd) {
-      double s = 0;
-      for (int m = 0; m < 10; ++m) s += ref_basis[(i * 3 + dd) * 10 + m] * mono[m];
-      nh[dd] = s;
-    }
-    for (int a = 0; a < 3; ++a) out[i][a] = Ji[0][a] * nh[0] + Ji[1][a] * nh[1] + Ji[2][a] * nh[2];
+  double nh[3];
+  for (int dd = 0; dd < 3; ++dd) {
+    double s = 0;
+    for (int m = 0; m < 10; ++m) s += ref_basis[(i * 3 + dd) * 10 + m] * mono[m];
+    nh[dd] = s;
   }
+  for (int a = 0; a < 3; ++a) out[a] = Ji[0][a] * nh[0] + Ji[1][a] * nh[1] + Ji[2][a] * nh[2];
 }
 
+// One thread per (point, basis function); dofs (nullable): the cell's DOFs.
 __global__ void k_basis_at(int64_t n, const double* pts, const int32_t* cellid, const double* xyz,
-                           const int32_t* cells, const double* ref_basis, int nloc, double* vals) {
-  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < n;
-       p += (int64_t)gridDim.x * blockDim.x) {
-    double v[20][3];
-    basis_values(xyz, cells + 4 * (int64_t)cellid[p], ref_basis, nloc, pts + 3 * p, v);
-    for (int i = 0; i < nloc; ++i)
-      for (int a = 0; a < 3; ++a) vals[(p * nloc + i) * 3 + a] = v[i][a];
+                           const int32_t* cells, const double* ref_basis, int nloc,
+                           const int32_t* cell_dofs, double* vals, int64_t* dofs) {
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n * nloc;
+       t += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t p = t / nloc;
+    const int i = (int)(t - p * nloc);
+    const int64_t c = cellid[p];
+    double v[3];
+    basis_value(xyz, cells + 4 * c, ref_basis, i, pts + 3 * p, v);
+    for (int a = 0; a < 3; ++a) vals[3 * t + a] = v[a];
+    if (dofs) dofs[t] = cell_dofs[c * nloc + i];
   }
 }
 
-// One wavefront per right-hand side; its sources are added in input order
-// (b[dof] += scale * N_dof(x_s) . value_s), so accumulation is deterministic.
-__global__ __launch_bounds__(64) void k_rhs(int64_t nsrc, const double* pos, const double2* val,
-                                            const int32_t* rhs, const int32_t* cellid,
-                                            int64_t nrhs, double2 scale, const double* xyz,
-                                            const int32_t* cells, const int32_t* cell_dofs,
-                                            const double* ref_basis, int nloc, int64_t ndofs,
-                                            double2* b) {
+// One workgroup per right-hand side; b[dof] += scale * N_dof(x_s) . value_s with the
+// sources of a DOF added in input order, so accumulation is deterministic.  The sources go
+// in tiles of 64: every (source, basis function) contribution is formed in parallel into
+// LDS; a hash table of the tile's DOFs collects, per DOF, the set of its sources as a
+// 64-bit mask (the set does not depend on the order of insertion; a cell holds a DOF once);
+// each table entry then adds its sources in ascending order to b.  One source at a time,
+// as the sum's order suggests, each waits for the previous one's memory round trip: 1,200
+// sources on one right-hand side 12.1 ms, by tiles 0.50 ms.
+constexpr int RHS_TB = 512, RHS_TILE = 64, RHS_HASH = 2048, RHS_NLOC = 20;
+static_assert(RHS_TILE * RHS_NLOC < RHS_HASH, "every DOF of a tile finds a free slot");
+__global__ __launch_bounds__(RHS_TB) void k_rhs(int64_t nsrc, const double* pos, const double2* val,
+                                                const int32_t* rhs, const int32_t* cellid,
+                                                int64_t nrhs, double2 scale, const double* xyz,
+                                                const int32_t* cells, const int32_t* cell_dofs,
+                                                const double* ref_basis, int nloc, int64_t ndofs,
+                                                double2* b) {
+  __shared__ double2 add[RHS_TILE * RHS_NLOC];
+  __shared__ int32_t dof[RHS_TILE * RHS_NLOC];   // -1: not a source of this right-hand side
+  __shared__ int32_t key[RHS_HASH];
+  __shared__ unsigned long long who[RHS_HASH];
+  __shared__ double rb[RHS_NLOC * 30];
+  for (int k = threadIdx.x; k < nloc * 30; k += RHS_TB) rb[k] = ref_basis[k];
   for (int64_t r = blockIdx.x; r < nrhs; r += gridDim.x) {
-    for (int64_t s = 0; s < nsrc; ++s) {
-      if (rhs[s] != r) continue;
-      const int32_t c = cellid[s];
-      if (threadIdx.x < nloc) {
-        double v[20][3];
-        basis_values(xyz, cells + 4 * (int64_t)c, ref_basis, nloc, pos + 3 * s, v);
-        const int i = threadIdx.x;
+    double2* br = b + r * ndofs;
+    for (int64_t s0 = 0; s0 < nsrc; s0 += RHS_TILE) {
+      const int ts = (int)(nsrc - s0 < RHS_TILE ? nsrc - s0 : RHS_TILE);
+      const int mine = threadIdx.x < ts && rhs[s0 + threadIdx.x] == r;
+      if (!__syncthreads_or(mine)) continue;   // (uniform) none of the tile's sources
+      for (int h = threadIdx.x; h < RHS_HASH; h += RHS_TB) {
+        key[h] = -1;
+        who[h] = 0;
+      }
+      for (int e = threadIdx.x; e < ts * nloc; e += RHS_TB) {
+        const int t = e / nloc, i = e - t * nloc;
+        const int64_t s = s0 + t;
+        if (rhs[s] != r) {
+          dof[e] = -1;
+          continue;
+        }
+        const int64_t c = cellid[s];
+        double v[3];
+        basis_value(xyz, cells + 4 * c, rb, i, pos + 3 * s, v);
         double2 acc = make_double2(0, 0);
         for (int a = 0; a < 3; ++a) {
-          acc.x += v[i][a] * val[3 * s + a].x;
-          acc.y += v[i][a] * val[3 * s + a].y;
+          acc.x += v[a] * val[3 * s + a].x;
+          acc.y += v[a] * val[3 * s + a].y;
         }
-        const int64_t dof = cell_dofs[(int64_t)c * nloc + i];
-        double2 add = make_double2(scale.x * acc.x - scale.y * acc.y,
-                                   scale.x * acc.y + scale.y * acc.x);
-        double2 old = b[r * ndofs + dof];
-        b[r * ndofs + dof] = make_double2(old.x + add.x, old.y + add.y);
+        add[e] = make_double2(scale.x * acc.x - scale.y * acc.y,
+                              scale.x * acc.y + scale.y * acc.x);
+        dof[e] = cell_dofs[c * nloc + i];
+      }
+      __syncthreads();
+      for (int e = threadIdx.x; e < ts * nloc; e += RHS_TB) {
+        const int32_t d = dof[e];
+        if (d < 0) continue;
+        unsigned h = ((uint32_t)d * 2654435761u) >> 21;   // 11 bits
+        while (true) {   // ends: fewer DOFs than slots
+          const int32_t k = atomicCAS(&key[h], -1, d);
+          if (k == -1 || k == d) break;
+          h = (h + 1) & (RHS_HASH - 1);
+        }
+        atomicOr(&who[h], 1ull << (e / nloc));
+      }
+      __syncthreads();
+      for (int h = threadIdx.x; h < RHS_HASH; h += RHS_TB) {
+        const int32_t d = key[h];
+        if (d < 0) continue;
+        double2 v = br[d];
+        int i = 0;
+        for (unsigned long long m = who[h]; m; m &= m - 1) {
+          // the source's cell holds d, mostly where the previous source's cell did
+          const int* row = dof + (__ffsll((long long)m) - 1) * nloc;
+          while (row[i] != d) i = i + 1 < nloc ? i + 1 : 0;
+          const double2 a = add[(row - dof) + i];
+          v = make_double2(v.x + a.x, v.y + a.y);
+        }
+        br[d] = v;
       }
       __syncthreads();
     }
@@ -598,12 +695,10 @@ void csr_apply64(Context* c, const Csr* A, const double2* x, double2* y) {
 
 void locate_points(Context* c, const Space* s, int64_t n, const double* pts_d, int32_t* cell_d) {
   const Mesh* m = s->mesh;
-  // initialise to "not found"
-  std::vector<int32_t> init(n, 0x7fffffff);
-  h2d(c, cell_d, init.data(), n);
+  if (n == 0) return;
+  SUCEM_LAUNCH(k_fill_i32, grid_for(n, TB), TB, 0, c->stream, n, 0x7fffffff, cell_d);
   SUCEM_LAUNCH(k_locate, grid_for(m->nc, TB), TB, 0, c->stream, m->nc, m->xyz.p, m->cells.p, n,
                pts_d, 1e-12, cell_d);
-  c->sync();
 }
 
 void rhs_point_sources(Context* c, const Space* s, int64_t nsrc, const double* pos_d,
@@ -612,16 +707,17 @@ void rhs_point_sources(Context* c, const Space* s, int64_t nsrc, const double* p
   const Mesh* m = s->mesh;
   unsigned g = (unsigned)(nrhs < 65535 ? nrhs : 65535);
   if (g == 0 || nsrc == 0) return;
-  SUCEM_LAUNCH(k_rhs, g, 64, 0, c->stream, nsrc, pos_d, val_d, rhs_d, cell_d, nrhs, scale,
+  SUCEM_CHECK(s->nloc <= RHS_NLOC, SUCEM_ERR_UNSUPPORTED, "at most 20 DOFs per cell");
+  SUCEM_LAUNCH(k_rhs, g, RHS_TB, 0, c->stream, nsrc, pos_d, val_d, rhs_d, cell_d, nrhs, scale,
                m->xyz.p, m->cells.p, s->cell_dofs.p, s->ref_basis.p, s->nloc, s->ndofs, b_d);
 }
 
 void basis_at_points(Context* c, const Space* s, int64_t n, const double* pts_d,
-                     const int32_t* cell_d, double* vals_d) {
+                     const int32_t* cell_d, double* vals_d, int64_t* dofs_d) {
   const Mesh* m = s->mesh;
   if (n == 0) return;
-  SUCEM_LAUNCH(k_basis_at, grid_for(n, 64), 64, 0, c->stream, n, pts_d, cell_d, m->xyz.p,
-               m->cells.p, s->ref_basis.p, s->nloc, vals_d);
+  SUCEM_LAUNCH(k_basis_at, grid_for(n * s->nloc, TB), TB, 0, c->stream, n, pts_d, cell_d,
+               m->xyz.p, m->cells.p, s->ref_basis.p, s->nloc, s->cell_dofs.p, vals_d, dofs_d);
 }
 
 // ---- allocation-free point-source right-hand sides -----------------------------------
