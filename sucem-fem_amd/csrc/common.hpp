@@ -67,7 +67,7 @@ struct DBuf {
 // Device workspace of a context: numbered slots that keep their allocation from call to
 // call and grow when a call needs more, so repeated solves on one context allocate (and
 // free, which synchronises the device) nothing after the first.  A slot is used by one
-// routine at a time: the Krylov solver takes slots [0, 32), the eigen solver [32, 48) (it
+// routine at a time: the Krylov solver takes slots [0, 32) and 84, the eigen solver [32, 48) (it
 // calls the Krylov solver, so their ranges differ), the batched solver [48, 80), the point entry
 // points [80, 84).  Calls on one context run one at a time (one host thread per context).
 struct Workspace {

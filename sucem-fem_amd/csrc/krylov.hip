@@ -397,7 +397,9 @@ struct Op {
   virtual void vinv_lo(void* vinv) {}
   // operator form that leaves shared rows as partial sums (COCG): block partials, or 0
   virtual int deferred_parts() { return 0; }
-  virtual void apply_deferred(const void* x, void* y, const void* w, const RedSite& rs) {}
+  virtual void apply_deferred(const void* x, void* y, const void* w, const RedSite& rs,
+                              const PtUpdate* up) {}
+  virtual bool updates() { return false; }   // it can form the next search direction
   virtual const int32_t* qcode() { return nullptr; }
   virtual const void* partials() { return nullptr; }
   virtual ~Op() {}
@@ -440,9 +442,11 @@ struct SysOp : Op {
     nodal_winv<R>(c, const_cast<System*>(sys), kp, mask != nullptr, vinv);
   }
   int deferred_parts() override { return pt_deferred_parts(sys, flo); }
-  void apply_deferred(const void* x, void* y, const void* w, const RedSite& rs) override {
-    pt_apply_deferred<R>(c, sys, k, mask, x, y, w, rs, flo);
+  void apply_deferred(const void* x, void* y, const void* w, const RedSite& rs,
+                      const PtUpdate* up) override {
+    pt_apply_deferred<R>(c, sys, k, mask, x, y, w, rs, flo, up);
   }
+  bool updates() override { return pt_updates<R>(sys, flo); }
   const int32_t* qcode() override { return pt_qcode(sys, flo); }
   const void* partials() override { return pt_partials(sys); }
 };
@@ -567,6 +571,10 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
   C* xlo = lo ? xlo_buf.p : (C*)x;
   const Slot<C> z = vec(16, grad ? n : 0), w = vec(17, nl), winv = vec(18, nl),
                 u = vec(19, nn), vinv = vec(20, nn);
+  // the search direction alternates between two buffers where the operator forms the next
+  // one (below)
+  const bool fuse_p = Gd > 0 && op.updates();
+  const Slot<C> p2 = vec(84, fuse_p ? n : 0);
   // z = M^-1 r, reducing r.z / |r|^2 into the site's scalars
   auto precondition = [&](const RedSite& rs) {
     op.precond_lo(winv.p, dinv.p, r.p, w.p, z.p, G, rs, aux ? vinv.p : nullptr, u.p);
@@ -648,18 +656,38 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
   // 24.7 us per FP32 application with the 8 of the other vector kernels, which lose more
   // at 4: the x/r update 34.3 against 28.5 us)
   const int Gz = op_grid(c, n, 4);
+  // With fuse_p that loop leaves p = z + beta p to the next iteration's operator, except
+  // before a host check (a check may restart the recursion, and reads the history entry that
+  // the update writes): `pending` says that it is due, `due` its operands.
+  bool pending = false;
+  PtUpdate due{};
+  C* pc = p.p;   // the current search direction
   for (it = 0; it < o.max_iter; ++it) {
     if (cocg && grad && Gd > 0) {
       const RedSite ra = site(SITE_SPMV1, FIN_COCG_ALPHA);
       const bool sample = it >= o.check_every && it % o.check_every == 0;
       if (sample) timer.start(c);
-      op.apply_deferred(p.p, q.p, p.p, ra);
+      if (pending) {
+        C* pn = pc == p.p ? p2.p : p.p;
+        due.p = pn;
+        op.apply_deferred(pc, q.p, nullptr, ra, &due);
+        pc = pn;
+      } else {
+        op.apply_deferred(pc, q.p, pc, ra, nullptr);
+      }
       if (sample) timer.stop(c);
-      SUCEM_LAUNCH((k_cocg_xr_def_a<C>), G, TB, 0, c->stream, n, G, Gd, ra, xlo, r.p, p.p, q.p,
+      SUCEM_LAUNCH((k_cocg_xr_def_a<C>), G, TB, 0, c->stream, n, G, Gd, ra, xlo, r.p, pc, q.p,
                    op.qcode(), (const C*)op.partials(), op.mask);
       const RedSite rb = site(SITE_UPDATE, FIN_DEFER, it);
       op.precond_lo(winv.p, dinv.p, r.p, w.p, z.p, Gz, rb, aux ? vinv.p : nullptr, u.p);
-      SUCEM_LAUNCH((k_cocg_pz_b<C>), G, TB, 0, c->stream, n, G, Gz, rb, z.p, p.p);
+      pending = fuse_p && (it + 1) % o.check_every != 0 && it + 1 != o.max_iter;
+      if (pending) {
+        due.z = z.p;
+        due.Gr = Gz;
+        due.rb = rb;
+      } else {
+        SUCEM_LAUNCH((k_cocg_pz_b<C>), G, TB, 0, c->stream, n, G, Gz, rb, z.p, pc);
+      }
       st.spmv_lo += 1;
     } else if (cocg && grad) {
       apply_epi(p.p, q.p, p.p, 1, site(SITE_SPMV1, FIN_COCG_ALPHA));
@@ -780,7 +808,7 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
     // the old direction after a residual replacement stalls these indefinite systems
     if (grad) {
       precondition(site(SITE_UPDATE, FIN_SET_RHO));
-      SUCEM_LAUNCH((k_copy<C>), G, TB, 0, c->stream, n, G, z.p, p.p);
+      SUCEM_LAUNCH((k_copy<C>), G, TB, 0, c->stream, n, G, z.p, pc);
     } else if (cocg) {
       SUCEM_LAUNCH((k_cocg_start<C>), G, TB, 0, c->stream, n, G, dinv.p, r.p, p.p);
     } else {

@@ -42,9 +42,22 @@ void pt_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const 
 // zero on masked rows; rs gets pt_deferred_parts(sys, f) block partials (0: the form is
 // not available for f).
 int pt_deferred_parts(const System* sys, const SpmvCfg& f);
+//
+// With `up` (where pt_updates says so), x is the previous search direction and the operator is applied to the next one,
+// p = z + beta x, written to up->p (another buffer than x); beta from the Gr block partials
+// of the preconditioner's site up->rb, whose scalars it stores (w is not used).
+template <typename R>
+bool pt_updates(const System* sys, const SpmvCfg& f);
+struct PtUpdate {
+  const void* z;
+  void* p;
+  int Gr;
+  RedSite rb;
+};
 template <typename R>
 void pt_apply_deferred(Context* c, const System* sys, Coef k, const uint8_t* mask, const void* x,
-                       void* y, const void* w, const RedSite& rs, const SpmvCfg& f);
+                       void* y, const void* w, const RedSite& rs, const SpmvCfg& f,
+                       const PtUpdate* up = nullptr);
 const int32_t* pt_qcode(const System* sys, const SpmvCfg& f);
 const void* pt_partials(const System* sys);
 // whether the patch kernel's LDS need in precision R fits the device

@@ -290,6 +290,49 @@ constexpr int patch_waves(int order, bool fp32) {
   return order == 1 ? 4 : (fp32 ? 3 : 2);
 }
 
+// Whether the operator of COCG forms the next search direction itself (PU below).  Not in
+// FP32 at order 2 with 128 cells or more, where the kernel is bound by its memory traffic
+// and the two gathers cost more than the separate update saves.  Iteration of the solve,
+// separate against fused, us, FP32 / FP64: order 2, 6,468 cells 30.5 / 33.2 -> 29.4 / 32.2;
+// 29,172 cells 39.3 / 45.8 -> 36.6 / 42.3; 384,000 cells 150.7 / 253.3 -> 156.2 / 247.5;
+// order 1, 48,000 cells 27.2 / 28.4 -> 26.2 / 27.4; 178,002 cells 36.1 / 41.8 -> 32.7 /
+// 37.9; 384,000 cells 49.2 / 61.6 -> 47.2 / 59.0.
+constexpr bool patch_updates(int order, int cb, bool fp32) {
+  return order == 1 || cb == 64 || !fp32;
+}
+
+// beta = (r.z) / rho of COCG from the preconditioner's Gr block partials, the same in every
+// block; block 0 stores the scalars of the step (rho for the next alpha in S_RHO_NEXT:
+// S_RHO, the previous rho, is read by all blocks).  Contains barriers.
+template <int NT, bool PR>
+__device__ __forceinline__ double2 next_beta(const RedSite& rb, int Gr) {
+  double2 s0 = make_double2(0, 0), s1 = make_double2(0, 0);
+  for (int k = threadIdx.x; k < Gr; k += NT) {
+    const double2 t = rb.part[k];
+    s0.x += t.x;
+    s0.y += t.y;
+  }
+  const double2 rho = scal2(rb.scal, S_RHO);
+  s0 = block_sum<NT>(s0);
+  const double2 be = PR ? pdiv0(s0, rho) : cdiv0(s0, rho);
+  if (blockIdx.x == 0) {
+    for (int k = threadIdx.x; k < Gr; k += NT) {
+      const double2 t = rb.part[Gr + k];
+      s1.x += t.x;
+      s1.y += t.y;
+    }
+    s1 = block_sum<NT>(s1);
+    if (threadIdx.x == 0) {
+      double* sc = rb.scal;
+      sc[S_BETA] = be.x; sc[S_BETA + 1] = be.y;
+      sc[S_RHO_NEXT] = s0.x; sc[S_RHO_NEXT + 1] = s0.y;
+      sc[S_RR] = PR ? prel2(sc, s1) : s1.x;   // paired: see prel2
+      if (rb.hist) rb.hist[rb.it] = sqrt(sc[S_RR]);
+    }
+  }
+  return be;
+}
+
 // T[idx] by a 32-bit byte offset from a uniform base (idx * sizeof(T) below 2^32)
 template <typename T>
 __device__ __forceinline__ T at32(const T* base, uint32_t idx) {
@@ -312,7 +355,16 @@ __device__ __forceinline__ T at32(const T* base, uint32_t idx) {
 // (there the places that are read again instead of held also take the kernel from 274 to
 // 246 registers, one wave per SIMD to two); 17 x 22 x 13 boxes with the 64-cell patches
 // 24.4 -> 14.7 and 26.7 -> 17.2 us.
-template <typename R, int ORDER, int NFD, int EPI, int CB>
+//
+// PU (COCG forms only): x is the previous search direction and the kernel applies A to the
+// next one, p = z + beta x, formed as it is gathered; beta = (r.z) / rho comes from the
+// preconditioner's Gr block partials in rb (r.z at part[0, Gr), |r|^2 at part[Gr, 2 Gr)),
+// which every block sums in one fixed order, as k_cocg_pz_b does.  p goes to pnew (not x:
+// other patches still read it), a shared DOF's from each of its patches with the same
+// value, so that a thread reads its own stores in the epilogue.  Block 0 stores beta, the
+// new rho, |r|^2 and the residual history entry.  This saves the separate update's pass
+// over z and p and one launch per iteration.
+template <typename R, int ORDER, int NFD, int EPI, int CB, bool PU>
 __global__ __launch_bounds__(patch_threads(CB), patch_waves(ORDER, sizeof(R) == 4)) void k_mf_patch(
     int64_t np, int Gp, int Gt, int64_t nc, int64_t nbf, int lds_main, const R* __restrict__ coef,
     const uint32_t* __restrict__ lp, const int32_t* __restrict__ uptr,
@@ -322,11 +374,12 @@ __global__ __launch_bounds__(patch_threads(CB), patch_waves(ORDER, sizeof(R) == 
     const R* __restrict__ hf, const int32_t* __restrict__ face_dofs,
     const double* __restrict__ ref_face, R cs, R ct, R c0, const uint8_t* __restrict__ mask,
     const typename C2<R>::T* __restrict__ x, typename C2<R>::T* __restrict__ y,
-    typename C2<R>::T* __restrict__ part, const typename C2<R>::T* __restrict__ w,
-    RedSite rs) {
+    typename C2<R>::T* __restrict__ part, const typename C2<R>::T* w, RedSite rs,
+    const typename C2<R>::T* __restrict__ z, typename C2<R>::T* pnew, int Gr, RedSite rb) {
   using C = typename C2<R>::T;
   constexpr bool E3 = EPI == 3 || EPI == 4;   // COCG form (EPI 4: paired systems)
   constexpr bool PR = EPI == 4;
+  static_assert(E3 || !PU, "the p update belongs to the COCG forms");
   constexpr int NLOC = MfTab<ORDER>::NLOC;
   constexpr int KK = NFD * NFD;
   constexpr int SL = patch_slabs(CB), ROWS = NLOC / SL, NT = CB * SL;
@@ -368,14 +421,25 @@ __global__ __launch_bounds__(patch_threads(CB), patch_waves(ORDER, sizeof(R) == 
     };
     load_dofs(0);
     if constexpr (PF) load_cell();
+    C be = mk(R(0), R(0));
     for (int j0 = 0; j0 < nu; j0 += UB * NT) {
       if (j0) load_dofs(j0);
-      C xv[UB];
+      C xv[UB], zv[PU ? UB : 1];
 #pragma unroll
       for (int q = 0; q < UB; ++q) xv[q] = x[dv[q]];
+      if constexpr (PU) {
+#pragma unroll
+        for (int q = 0; q < UB; ++q) zv[q] = z[dv[q]];
+        if (j0 == 0) be = from_d<C>(next_beta<NT, PR>(rb, Gr));   // while x and z arrive
+      }
 #pragma unroll
       for (int q = 0; q < UB; ++q) {
         const int j = j0 + q * NT + tid;
+        if constexpr (PU) {
+          const C bp = PR ? pmul(be, xv[q]) : cmul(be, xv[q]);
+          xv[q] = mk(zv[q].x + bp.x, zv[q].y + bp.y);
+          if (j < nu) pnew[dv[q]] = xv[q];
+        }
         if (j < nu) sm[j] = xv[q];
       }
     }
@@ -491,7 +555,7 @@ __global__ __launch_bounds__(patch_threads(CB), patch_waves(ORDER, sizeof(R) == 
       C wv[UB];
       if constexpr (WY) {
 #pragma unroll
-        for (int q = 0; q < UB; ++q) wv[q] = w[dv[q]];
+        for (int q = 0; q < UB; ++q) wv[q] = PU ? pnew[dv[q]] : w[dv[q]];
       }
       uint8_t off[UB];
 #pragma unroll
@@ -843,7 +907,7 @@ void pt_validate(Context* c, const Space* s, const PatchMaps& pm, const std::vec
 template <typename R, int ORDER, int NFD, int CB>
 void launch_patch(Context* c, const System* sys, const PatchMaps& pm, Coef k,
                   const uint8_t* mask, const void* x, void* y, const void* w, int epi,
-                  const RedSite& rs, int Gp, int Gt) {
+                  const RedSite& rs, int Gp, int Gt, const PtUpdate* up = nullptr) {
   using C = typename C2<R>::T;
   const Space* s = sys->space;
   const R* coef;
@@ -856,15 +920,26 @@ void launch_patch(Context* c, const System* sys, const PatchMaps& pm, Coef k,
   const R c0 = (sys->which & SUCEM_MAT_S0) ? (R)k.s0 : R(0);
   const size_t lds = (size_t)(pm.lds + pm.maxfr) * sizeof(C);
   constexpr int nt = patch_threads(CB);
+  const C* z = up ? (const C*)up->z : nullptr;
+  C* pnew = up ? (C*)up->p : nullptr;
+  const int Gr = up ? up->Gr : 0;
+  const RedSite rb = up ? up->rb : RedSite{};
 #define PT_ARGS pm.np, Gp, Gt, s->mesh->nc, s->nbf, pm.lds, coef, pm.lp.p, pm.uptr.p, pm.dof.p, \
                 pm.seg.p, pm.out.p, pm.fptr.p, s->pt_fmeta.p, pm.fpos.p, hf, s->ref_face_dofs.p, \
                 s->ref_face.p, (R)k.s, (R)k.t, c0, mask, (const C*)x, (C*)y, (C*)sys->pt_part.p, \
-                (const C*)w, rs
-  if (epi == 0) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 0, CB>), Gp, nt, lds, c->stream, PT_ARGS);
-  else if (epi == 1) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 1, CB>), Gp, nt, lds, c->stream, PT_ARGS);
-  else if (epi == 2) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 2, CB>), Gp, nt, lds, c->stream, PT_ARGS);
-  else if (epi == 3) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 3, CB>), Gp, nt, lds, c->stream, PT_ARGS);
-  else SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 4, CB>), Gp, nt, lds, c->stream, PT_ARGS);
+                (const C*)w, rs, z, pnew, Gr, rb
+  if (up) {
+    SUCEM_CHECK((epi == 3 || epi == 4) && patch_updates(ORDER, CB, sizeof(R) == 4),
+                SUCEM_ERR_INTERNAL, "p update not available in this form");
+    if constexpr (patch_updates(ORDER, CB, sizeof(R) == 4)) {
+      if (epi == 3) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 3, CB, true>), Gp, nt, lds, c->stream, PT_ARGS);
+      else SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 4, CB, true>), Gp, nt, lds, c->stream, PT_ARGS);
+    }
+  } else if (epi == 0) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 0, CB, false>), Gp, nt, lds, c->stream, PT_ARGS);
+  else if (epi == 1) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 1, CB, false>), Gp, nt, lds, c->stream, PT_ARGS);
+  else if (epi == 2) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 2, CB, false>), Gp, nt, lds, c->stream, PT_ARGS);
+  else if (epi == 3) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 3, CB, false>), Gp, nt, lds, c->stream, PT_ARGS);
+  else SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 4, CB, false>), Gp, nt, lds, c->stream, PT_ARGS);
 #undef PT_ARGS
 }
 
@@ -999,7 +1074,8 @@ int pt_deferred_parts(const System* sys, const SpmvCfg& f) {
 
 template <typename R>
 void pt_apply_deferred(Context* c, const System* sys, Coef k, const uint8_t* mask, const void* x,
-                       void* y, const void* w, const RedSite& rs, const SpmvCfg& f) {
+                       void* y, const void* w, const RedSite& rs, const SpmvCfg& f,
+                       const PtUpdate* up) {
   const int Gp = pt_deferred_parts(sys, f);
   SUCEM_CHECK(Gp > 0, SUCEM_ERR_INVALID, "deferred patch operator not available");
   SUCEM_CHECK(pt_fits<R>(sys->space, f.U), SUCEM_ERR_UNSUPPORTED,
@@ -1007,20 +1083,27 @@ void pt_apply_deferred(Context* c, const System* sys, Coef k, const uint8_t* mas
   const PatchMaps& pm = sys->space->pt[cb_slot(f.U)];
   const int epi = rs.paired ? 4 : 3;
   if (sys->space->order == 2) {
-    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
-    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
-    else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
-    else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
+    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
+    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
+    else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
+    else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
   } else {
-    launch_patch<R, 1, 3, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp);
+    launch_patch<R, 1, 3, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
   }
 }
 template void pt_apply_deferred<float>(Context*, const System*, Coef, const uint8_t*,
                                        const void*, void*, const void*, const RedSite&,
-                                       const SpmvCfg&);
+                                       const SpmvCfg&, const PtUpdate*);
 template void pt_apply_deferred<double>(Context*, const System*, Coef, const uint8_t*,
                                         const void*, void*, const void*, const RedSite&,
-                                        const SpmvCfg&);
+                                        const SpmvCfg&, const PtUpdate*);
+
+template <typename R>
+bool pt_updates(const System* sys, const SpmvCfg& f) {
+  return f.mf == 2 && patch_updates(sys->space->order, f.U, sizeof(R) == 4);
+}
+template bool pt_updates<float>(const System*, const SpmvCfg&);
+template bool pt_updates<double>(const System*, const SpmvCfg&);
 
 const int32_t* pt_qcode(const System* sys, const SpmvCfg& f) {
   return sys->space->pt[cb_slot(f.U)].qcode.p;
