@@ -27,6 +27,113 @@ double* Context::host_scratch(size_t count) {
   return pinned;
 }
 
+// ---- device memory pools (common.hpp) ---------------------------------------------------
+namespace {
+
+// every pool that may hold unused blocks (never destroyed: buffers may outlive main)
+struct PoolList {
+  std::mutex mu;
+  std::vector<std::weak_ptr<MemPool>> all;
+};
+PoolList& pool_list() {
+  static PoolList* l = new PoolList();
+  return *l;
+}
+
+// sizes are rounded up by at most an eighth, so that buffers of slightly different meshes
+// share blocks
+size_t block_size(size_t bytes) {
+  size_t step = 512;
+  while (step * 8 < bytes) step *= 2;
+  return (bytes + step - 1) / step * step;
+}
+
+}  // namespace
+
+std::shared_ptr<MemPool>& current_pool() {
+  static thread_local std::shared_ptr<MemPool> p;
+  return p;
+}
+
+std::shared_ptr<MemPool> new_pool() {
+  auto p = std::make_shared<MemPool>();
+  PoolList& l = pool_list();
+  std::lock_guard<std::mutex> hold(l.mu);
+  l.all.erase(std::remove_if(l.all.begin(), l.all.end(), [](auto& w) { return w.expired(); }),
+              l.all.end());
+  l.all.push_back(p);
+  return p;
+}
+
+void* device_alloc(size_t bytes) {
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  std::vector<std::shared_ptr<MemPool>> pools;
+  {
+    PoolList& l = pool_list();
+    std::lock_guard<std::mutex> hold(l.mu);
+    for (auto& w : l.all)
+      if (auto q = w.lock()) pools.push_back(q);
+  }
+  for (auto& q : pools) q->trim();
+  SUCEM_HIP(hipMalloc(&p, bytes));
+  return p;
+}
+
+MemPool::~MemPool() { trim(); }
+
+void* MemPool::take(size_t bytes, size_t& got) {
+  const size_t want = block_size(bytes);
+  {
+    std::lock_guard<std::mutex> hold(mu_);
+    auto it = free_.lower_bound(want);
+    if (it != free_.end() && it->first <= want + want / 8) {
+      void* p = it->second;
+      got = it->first;
+      unused_ -= got;
+      free_.erase(it);
+      return p;
+    }
+  }
+  void* p = device_alloc(want);
+  got = want;
+  return p;
+}
+
+void MemPool::put(void* p, size_t size) {
+  {
+    std::lock_guard<std::mutex> hold(mu_);
+    if (!closed_ && unused_ + size <= kMax) {
+      try {
+        free_.emplace(size, p);
+        unused_ += size;
+        return;
+      } catch (const std::bad_alloc&) {   // (destructors call this) back to the device
+      }
+    }
+  }
+  (void)hipFree(p);
+}
+
+void MemPool::trim() {
+  std::multimap<size_t, void*> old;
+  {
+    std::lock_guard<std::mutex> hold(mu_);
+    old.swap(free_);
+    unused_ = 0;
+  }
+  for (auto& e : old) (void)hipFree(e.second);   // waits for the work that may still use it
+}
+
+void MemPool::close() {
+  {
+    std::lock_guard<std::mutex> hold(mu_);
+    closed_ = true;
+  }
+  trim();
+}
+
 // export (AssemblyExport) helpers defined in assemble.hip / mesh_space.hip
 void mesh_translate(Context* c, Mesh* m, const double shift[3]);
 void export_lhs(Context* c, const System* sys, double k0, double2* out_d);
@@ -112,6 +219,8 @@ int sucem_ctx_destroy(sucem_ctx* ctx) {
   }
   if (c.pinned) (void)hipHostFree(c.pinned);
   if (c.own_stream) (void)hipStreamDestroy(c.stream);
+  c.pool->close();
+  if (current_pool() == c.pool) current_pool().reset();
   delete ctx;
   API_END
 }
@@ -137,6 +246,7 @@ int sucem_ctx_release_workspace(sucem_ctx* ctx) {
   ctx->c.use();
   ctx->c.sync();
   ctx->c.ws.release();
+  ctx->c.pool->trim();
   API_END
 }
 
@@ -272,6 +382,8 @@ int sucem_mesh_set_cell_materials(sucem_mesh* m, const double* eps_r_h,
   for (int64_t i = 0; i < nc; ++i)
     SUCEM_CHECK(std::isfinite(eps_r_h[i]) && std::isfinite(inv_mu_r_h[i]), SUCEM_ERR_INVALID,
                 "cell materials must be finite");
+  m->m.eps_r.release_synced();   // an earlier table may still be read
+  m->m.inv_mu_r.release_synced();
   m->m.eps_r.alloc(nc);
   m->m.inv_mu_r.alloc(nc);
   h2d(c, m->m.eps_r.p, eps_r_h, nc);
@@ -284,7 +396,7 @@ int sucem_mesh_destroy(sucem_mesh* m) {
   API_BEGIN
   if (!m) return SUCEM_OK;
   (void)hipSetDevice(m->m.ctx->device);
-  (void)hipStreamSynchronize(m->m.ctx->stream);
+  (void)hipDeviceSynchronize();   // other contexts' streams may still read it
   delete m;
   API_END
 }
@@ -371,7 +483,7 @@ int sucem_space_destroy(sucem_space* s) {
   API_BEGIN
   if (!s) return SUCEM_OK;
   (void)hipSetDevice(s->s.ctx->device);
-  (void)hipStreamSynchronize(s->s.ctx->stream);
+  (void)hipDeviceSynchronize();   // other contexts' streams may still read it
   delete s;
   API_END
 }
@@ -439,7 +551,7 @@ int sucem_system_destroy(sucem_system* sys) {
   API_BEGIN
   if (!sys) return SUCEM_OK;
   (void)hipSetDevice(sys->s.ctx->device);
-  (void)hipStreamSynchronize(sys->s.ctx->stream);
+  (void)hipDeviceSynchronize();   // other contexts' streams may still read it
   delete sys;
   API_END
 }
@@ -965,7 +1077,7 @@ int sucem_csr_destroy(sucem_csr* A) {
   API_BEGIN
   if (!A) return SUCEM_OK;
   (void)hipSetDevice(A->a.ctx->device);
-  (void)hipStreamSynchronize(A->a.ctx->stream);
+  (void)hipDeviceSynchronize();   // other contexts' streams may still read it
   delete A;
   API_END
 }

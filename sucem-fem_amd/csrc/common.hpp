@@ -5,6 +5,9 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <map>
+#include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -36,30 +39,88 @@ void set_last_error(const std::string& msg);
     if (!(cond)) throw ::sucem::Error((code), (msg));   \
   } while (0)
 
+// Device memory that a context's finished buffers leave for its next ones.  Building a mesh,
+// a space and a system takes some 250 buffers, most of them for one step; allocated and
+// freed one by one they cost 15 of the 25 ms of an order-2 set-up of 32,400 cells (hipFree
+// also waits for the whole device).
+//
+// A block that is put back may still be in use by work queued on its context's stream, so it
+// is only handed out to that context (whose stream orders the new use behind the old one).
+// Whoever frees memory that other streams may use waits for the device first, as hipFree
+// does: the destroy entry points, and members replaced while their owner lives (see
+// DBuf::release_synced).  At most kMax bytes stay unused in one pool; blocks go back to the
+// device beyond that, when the context's workspace is released, when an allocation fails
+// (all pools give way), and with the context (buffers that outlive it free directly).
+class MemPool {
+ public:
+  static constexpr size_t kMax = size_t(4) << 30;
+  ~MemPool();
+  // a block of at least `bytes` (its size in `got`), or throws SUCEM_ERR_OOM
+  void* take(size_t bytes, size_t& got);
+  void put(void* p, size_t size);
+  void trim();    // everything unused back to the device
+  void close();   // trim, and keep nothing from now on
+
+ private:
+  std::mutex mu_;
+  std::multimap<size_t, void*> free_;
+  size_t unused_ = 0;
+  bool closed_ = false;
+};
+// The pool of the context that this thread's current entry point runs on (Context::use).
+std::shared_ptr<MemPool>& current_pool();
+std::shared_ptr<MemPool> new_pool();
+// hipMalloc; when it fails, once more after every pool has given its unused blocks back
+void* device_alloc(size_t bytes);
+
 // Owning device allocation.
 template <typename T>
 struct DBuf {
   T* p = nullptr;
   size_t n = 0;
+  size_t size = 0;                  // of the block
+  std::shared_ptr<MemPool> pool;    // where the block goes back to (null: to the device)
   DBuf() = default;
   explicit DBuf(size_t count) { alloc(count); }
   DBuf(const DBuf&) = delete;
   DBuf& operator=(const DBuf&) = delete;
-  DBuf(DBuf&& o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+  DBuf(DBuf&& o) noexcept : p(o.p), n(o.n), size(o.size), pool(std::move(o.pool)) {
+    o.p = nullptr;
+    o.n = o.size = 0;
+  }
   DBuf& operator=(DBuf&& o) noexcept {
-    if (this != &o) { release(); p = o.p; n = o.n; o.p = nullptr; o.n = 0; }
+    if (this != &o) {
+      release();
+      p = o.p; n = o.n; size = o.size; pool = std::move(o.pool);
+      o.p = nullptr;
+      o.n = o.size = 0;
+    }
     return *this;
   }
   ~DBuf() { release(); }
-  void alloc(size_t count) {
+  void alloc(size_t count, bool pooled = true) {
     release();
+    if (count) {
+      std::shared_ptr<MemPool> from = pooled ? current_pool() : nullptr;
+      size = count * sizeof(T);
+      p = (T*)(from ? from->take(size, size) : device_alloc(size));
+      pool = std::move(from);
+    }
     n = count;
-    if (count) SUCEM_HIP(hipMalloc(&p, count * sizeof(T)));
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p) {
+      if (pool) pool->put(p, size);
+      else (void)hipFree(p);
+    }
     p = nullptr;
-    n = 0;
+    n = size = 0;
+    pool.reset();
+  }
+  // release of memory that work on another context's stream may still use
+  void release_synced() {
+    if (p && pool) (void)hipDeviceSynchronize();
+    release();
   }
   size_t bytes() const { return n * sizeof(T); }
 };
@@ -79,7 +140,9 @@ struct Workspace {
     if ((size_t)k >= slot.size()) slot.resize(k + 1);
     if (slot[k].n < bytes) {
       slot[k].release();
-      slot[k].alloc(bytes + (bytes >> 3));   // 1/8 headroom for a slightly larger next call
+      // 1/8 headroom for a slightly larger next call; not from the pool, which is for
+      // buffers that come and go
+      slot[k].alloc(bytes + (bytes >> 3), false);
     }
     return slot[k].p;
   }
@@ -100,6 +163,7 @@ struct Context {
   double* pinned = nullptr;
   size_t pinned_n = 0;
   Workspace ws;
+  std::shared_ptr<MemPool> pool = new_pool();
   // library-owned stream (non-blocking, default priority) for work captured in hipGraphs:
   // the caller's stream may be the null stream, which cannot be captured
   hipStream_t aux_stream = nullptr;
@@ -108,7 +172,10 @@ struct Context {
     return aux_stream;
   }
   void sync() { SUCEM_HIP(hipStreamSynchronize(stream)); }
-  void use() { SUCEM_HIP(hipSetDevice(device)); }
+  void use() {
+    SUCEM_HIP(hipSetDevice(device));
+    current_pool() = pool;
+  }
   double* host_scratch(size_t n);
 };
 

@@ -762,7 +762,7 @@ const double* nodal_diag(Context* c, System* sys, bool masked) {
   Space* s = sys->space;
   ensure_nodal(c, s);
   DBuf<double>& d = sys->ndiag[masked ? 1 : 0];
-  if (masked && sys->ndiag_pec_version != s->pec_version) d.release();
+  if (masked && sys->ndiag_pec_version != s->pec_version) d.release_synced();
   if (!d.p) {
     if (masked) sys->ndiag_pec_version = s->pec_version;
     SUCEM_CHECK(sys->st64.p, SUCEM_ERR_INVALID, "S and T must be assembled");
@@ -863,7 +863,7 @@ const double* gradient_diag(Context* c, System* sys, bool masked) {
   Space* s = sys->space;
   ensure_gradient(c, s);
   DBuf<double>& d = sys->gdiag[masked ? 1 : 0];
-  if (masked && sys->gdiag_pec_version != s->pec_version) d.release();   // PEC mask changed
+  if (masked && sys->gdiag_pec_version != s->pec_version) d.release_synced();   // PEC mask changed
   if (!d.p) {
     if (masked) sys->gdiag_pec_version = s->pec_version;
     SUCEM_CHECK(sys->st64.p, SUCEM_ERR_INVALID, "S and T must be assembled");

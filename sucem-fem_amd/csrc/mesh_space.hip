@@ -534,6 +534,8 @@ int64_t mesh_set_materials(Context* c, Mesh* m, const int32_t* region_d, int64_t
   h2d(c, ids.p, ids_h, nreg);
   h2d(c, eps.p, eps_h, nreg);
   h2d(c, mu.p, mu_h, nreg);
+  m->eps_r.release_synced();   // an earlier table may still be read
+  m->inv_mu_r.release_synced();
   m->eps_r.alloc(m->nc);
   m->inv_mu_r.alloc(m->nc);
   DBuf<unsigned long long> bad(1);

@@ -977,7 +977,7 @@ bool pt_prepare(Context* c, System* sys, int cb) {
     sys->pt_ready = true;
   }
   if ((int64_t)sys->pt_part.n < std::max<int64_t>(s->pt[slot].npe, 1)) {
-    c->sync();
+    sys->pt_part.release_synced();
     sys->pt_part.alloc(std::max<int64_t>(s->pt[slot].npe, 1));
   }
   return true;

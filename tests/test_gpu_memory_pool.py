@@ -1,0 +1,80 @@
+"""Buffers of finished objects are used again by the context's next ones: bounded, given back
+with the workspace, and never before the work that uses them is done."""
+import ctypes
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _free(ctx):
+    from sucemfem import _hip
+    f, t = ctypes.c_int64(), ctypes.c_int64()
+    _hip.call("sucem_ctx_mem_info", ctx.handle, ctypes.byref(f), ctypes.byref(t))
+    return f.value
+
+
+def _solve(ctx, n, order, seed):
+    import torch
+    from sucemfem.Utilities.Workloads import DeviceProblem
+    p = DeviceProblem(n, np.array(n) * 0.03, order, 7, (1.0, 2.2, 4.4), seed, ctx=ctx)
+    c = np.array(n) * 0.015 + 1e-3
+    b = p.rhs_dipoles(c[None], np.array([[0.3, 1.0, -0.2]]), 9.0)
+    x = torch.zeros_like(b)
+    st = p.solve(9.0, b, x, precision=64, tol=1e-10)
+    ctx.synchronize()
+    assert st["status"] == 0
+    return x.cpu().numpy()
+
+
+def test_repeated_meshes_do_not_grow_and_release_gives_back():
+    import torch
+    from sucemfem import _hip
+    from sucemfem.runtime import Context
+    torch.cuda.set_device(0)
+    ctx = Context()
+    ref = _solve(ctx, (9, 8, 7), 2, 0)
+    after = _free(ctx)
+    for n, order, seed in (((9, 8, 7), 2, 0), ((8, 8, 8), 2, 1), ((12, 9, 10), 1, 2)) * 4:
+        x = _solve(ctx, n, order, seed)
+        if (n, order, seed) == ((9, 8, 7), 2, 0):
+            assert np.array_equal(x, ref)       # reused memory changes nothing
+    # a second and third size add at most their own buffers, not one set per repetition
+    assert after - _free(ctx) < (1 << 30)
+    held = _free(ctx)
+    _hip.call("sucem_ctx_release_workspace", ctx.handle)
+    assert _free(ctx) > held
+
+
+def test_threads_with_contexts_of_their_own():
+    """Four threads build, solve and drop problems at once, each on its own stream and context,
+    and drop each other's objects: results equal the ones computed alone."""
+    import torch
+    from sucemfem.runtime import Context
+    torch.cuda.set_device(0)
+    sizes = [((6, 5, 4), 2), ((9, 8, 7), 1), ((5, 6, 7), 2), ((7, 7, 7), 1)]
+    alone = [_solve(Context(), n, o, 5) for n, o in sizes]
+    got, errs = [[] for _ in sizes], []
+
+    def work(i):
+        try:
+            torch.cuda.set_device(0)
+            s = torch.cuda.Stream()
+            with torch.cuda.stream(s):
+                ctx = Context(stream=s)
+                for _ in range(4):
+                    got[i].append(_solve(ctx, sizes[i][0], sizes[i][1], 5))
+        except Exception as e:  # noqa: BLE001 - reported below
+            errs.append(e)
+
+    ths = [threading.Thread(target=work, args=(i,)) for i in range(len(sizes))]
+    for t in ths:
+        t.start()
+    for t in ths:
+        t.join()
+    assert not errs, errs
+    for a, g in zip(alone, got):
+        for x in g:
+            assert np.array_equal(x, a)
