@@ -173,6 +173,8 @@ int64_t build_csr_from_pairs(Context* c, int64_t n, DBuf<uint64_t>& keys, DBuf<u
                              int B, int64_t nrows, DBuf<int32_t>& row_ptr, DBuf<int32_t>& col,
                              DBuf<int32_t>& seg, DBuf<uint32_t>& perm);
 int key_bits(int64_t n);
+// out = exclusive prefix sums of in
+void exclusive_scan_i32(Context* c, const int32_t* in, int32_t* out, size_t n);
 // PEC DOFs = closure of the facets with facet_flag_h[f] != 0 (nF flags; null = the
 // boundary facets); union_mode ORs into the current mask instead of replacing it.
 void space_mark_pec(Context* c, Space* s, const uint8_t* facet_flag_h, bool union_mode);

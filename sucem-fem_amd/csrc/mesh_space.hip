@@ -48,6 +48,8 @@ void inclusive_scan_i32(Context* c, const int32_t* in, int32_t* out, size_t n) {
                                     c->stream));
 }
 
+}  // namespace
+
 void exclusive_scan_i32(Context* c, const int32_t* in, int32_t* out, size_t n) {
   size_t bytes = 0;
   SUCEM_HIP(rocprim::exclusive_scan(nullptr, bytes, in, out, int32_t(0), n,
@@ -56,6 +58,8 @@ void exclusive_scan_i32(Context* c, const int32_t* in, int32_t* out, size_t n) {
   SUCEM_HIP(rocprim::exclusive_scan(tmp.p, bytes, in, out, int32_t(0), n,
                                     rocprim::plus<int32_t>(), c->stream));
 }
+
+namespace {
 
 template <typename T>
 T read_scalar(Context* c, const T* d) {
