@@ -441,19 +441,10 @@ __device__ __forceinline__ void aux_vertex_rows(int64_t blk, int nv, int nE, R i
       }
     }
   }
-#pragma unroll
-  for (int o = L / 2; o > 0; o >>= 1) {
-    g.x += __shfl_xor(g.x, o);
-    g.y += __shfl_xor(g.y, o);
-  }
+  g = mk(group_sum<L>(g.x), group_sum<L>(g.y));
   if constexpr (NODAL) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-#pragma unroll
-      for (int o = L / 2; o > 0; o >>= 1) {
-        acc[d].x += __shfl_xor(acc[d].x, o);
-        acc[d].y += __shfl_xor(acc[d].y, o);
-      }
+    for (int d = 0; d < 3; ++d) acc[d] = mk(group_sum<L>(acc[d].x), group_sum<L>(acc[d].y));
   }
   if (lane == 0 && v < nv) {
     w[v] = cmul(winv[v], mk(inv_den * g.x, inv_den * g.y));
@@ -490,11 +481,7 @@ __device__ __forceinline__ void aux_edge_rows(int64_t blk, int nv, int nE, R inv
       else { g.x += R(4) * (r0.x + r1.x); g.y += R(4) * (r0.y + r1.y); }
     }
   }
-#pragma unroll
-  for (int o = L / 2; o > 0; o >>= 1) {
-    g.x += __shfl_xor(g.x, o);
-    g.y += __shfl_xor(g.y, o);
-  }
+  g = mk(group_sum<L>(g.x), group_sum<L>(g.y));
   if (lane == 0 && e < nE) w[nv + e] = cmul(winv[nv + e], mk(inv_den * g.x, inv_den * g.y));
 }
 

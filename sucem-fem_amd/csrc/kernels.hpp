@@ -70,22 +70,81 @@ __device__ __forceinline__ void sq_acc(double2& d, double2 a, bool paired) {
   }
 }
 
-// Wavefront-then-block sum of a double2; every thread of the block gets the result.
-// Deterministic: fixed reduction tree.
-template <int TB>
-__device__ __forceinline__ double2 block_sum(double2 v) {
-  __shared__ double2 red[TB / 64];
-  for (int o = 32; o > 0; o >>= 1) {
-    v.x += __shfl_xor(v.x, o);
-    v.y += __shfl_xor(v.y, o);
+// x of lane ^ M for M = 1 ... 32 by DPP moves and (M = 16, 32) row swaps, in the vector ALU:
+// a shuffle goes through the LDS crossbar and back, and six of them in a row were most of a
+// small reduction kernel's time.  Every lane of the wave has to be active.
+template <int CTRL>
+__device__ __forceinline__ int dpp_move(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+}
+template <int M>
+__device__ __forceinline__ int lane_xor(int x) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8 || M == 16 || M == 32, "one bit");
+  if constexpr (M == 1) return dpp_move<0xB1>(x);          // quad permutation [1, 0, 3, 2]
+  if constexpr (M == 2) return dpp_move<0x4E>(x);          // quad permutation [2, 3, 0, 1]
+  if constexpr (M == 4) return dpp_move<0x1B>(dpp_move<0x141>(x));   // 7 - i, then 3 - i in quads
+  if constexpr (M == 8) return dpp_move<0x128>(x);         // row rotation by 8 of 16
+  const bool high = (__lane_id() & M) != 0;
+  if constexpr (M == 16) {
+    // the odd rows of 16 of the one operand change places with the even rows of the other
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return high ? r[0] : r[1];
+  }
+  if constexpr (M == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return high ? r[0] : r[1];
+  }
+}
+template <int M>
+__device__ __forceinline__ float lane_xor(float x) {
+  return __int_as_float(lane_xor<M>(__float_as_int(x)));
+}
+template <int M>
+__device__ __forceinline__ double lane_xor(double x) {
+  return __hiloint2double(lane_xor<M>(__double2hiint(x)), lane_xor<M>(__double2loint(x)));
+}
+// Sum over aligned groups of L lanes, the same in every lane of a group; the order of a
+// butterfly from distance L / 2 down to 1.
+template <int L, typename R>
+__device__ __forceinline__ R group_sum(R x) {
+  if constexpr (L >= 64) x += lane_xor<32>(x);
+  if constexpr (L >= 32) x += lane_xor<16>(x);
+  if constexpr (L >= 16) x += lane_xor<8>(x);
+  if constexpr (L >= 8) x += lane_xor<4>(x);
+  if constexpr (L >= 4) x += lane_xor<2>(x);
+  if constexpr (L >= 2) x += lane_xor<1>(x);
+  return x;
+}
+
+// Wavefront-then-block sums of NV double2 at once (one pair of barriers); every thread of
+// the block gets the results.  Deterministic: fixed reduction tree.
+template <int TB, int NV>
+__device__ __forceinline__ void block_sums(double2 (&v)[NV]) {
+  __shared__ double2 red[TB / 64][NV];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    v[k].x = group_sum<64>(v[k].x);
+    v[k].y = group_sum<64>(v[k].y);
   }
   const int w = threadIdx.x >> 6;
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[w] = v;
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) red[w][k] = v[k];
+  }
   __syncthreads();
-  double2 s = red[0];
-  for (int i = 1; i < TB / 64; ++i) { s.x += red[i].x; s.y += red[i].y; }
-  return s;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    double2 s = red[0][k];
+    for (int i = 1; i < TB / 64; ++i) { s.x += red[i][k].x; s.y += red[i][k].y; }
+    v[k] = s;
+  }
+}
+template <int TB>
+__device__ __forceinline__ double2 block_sum(double2 v) {
+  double2 a[1] = {v};
+  block_sums<TB, 1>(a);
+  return a[0];
 }
 
 // Logical block index that gives each XCD a contiguous share of the rows
@@ -214,12 +273,12 @@ __device__ __forceinline__ void finalize(const RedSite& rs, double2 s0, double2 
 // such fence writes back the XCD's L2).  Must be called by every thread of every block.
 template <int TB>
 __device__ __forceinline__ void reduce_finalize(const RedSite& rs, int G, double2 v0, double2 v1) {
-  v0 = block_sum<TB>(v0);
-  v1 = block_sum<TB>(v1);
+  double2 v[2] = {v0, v1};
+  block_sums<TB, 2>(v);
   if (threadIdx.x == 0) {
     const int lb = xcd_block(G);
-    rs.part[lb] = v0;
-    rs.part[G + lb] = v1;
+    rs.part[lb] = v[0];
+    rs.part[G + lb] = v[1];
   }
 }
 

@@ -373,9 +373,9 @@ __global__ __launch_bounds__(FIN_TB) void k_finalize(RedSite rs, int G) {
       b.x += q[k].x; b.y += q[k].y;
     }
   }
-  a = block_sum<FIN_TB>(a);
-  b = block_sum<FIN_TB>(b);
-  if (threadIdx.x == 0) finalize(rs, a, b);
+  double2 s[2] = {a, b};
+  block_sums<FIN_TB, 2>(s);
+  if (threadIdx.x == 0) finalize(rs, s[0], s[1]);
 }
 
 struct Op {

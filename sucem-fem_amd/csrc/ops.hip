@@ -74,12 +74,9 @@ __global__ __launch_bounds__(TB) void k_sys_spmv(
         }
       }
     }
-#pragma unroll
-    for (int o = L / 2; o > 0; o >>= 1) {
-      as.x += __shfl_xor(as.x, o); as.y += __shfl_xor(as.y, o);
-      at.x += __shfl_xor(at.x, o); at.y += __shfl_xor(at.y, o);
-      a0.x += __shfl_xor(a0.x, o); a0.y += __shfl_xor(a0.y, o);
-    }
+    as = mk(group_sum<L>(as.x), group_sum<L>(as.y));
+    at = mk(group_sum<L>(at.x), group_sum<L>(at.y));
+    a0 = mk(group_sum<L>(a0.x), group_sum<L>(a0.y));
     if (lane == 0 && r < end) {
       C yr = mk(cs * as.x + ct * at.x - c0 * a0.y, cs * as.y + ct * at.y + c0 * a0.x);
       if (mask && mask[r]) yr = mk(R(0), R(0));
@@ -139,11 +136,7 @@ __global__ __launch_bounds__(TB) void k_csr_spmv(int n, int G, const int32_t* __
         }
       }
     }
-#pragma unroll
-    for (int o = L / 2; o > 0; o >>= 1) {
-      acc.x += __shfl_xor(acc.x, o);
-      acc.y += __shfl_xor(acc.y, o);
-    }
+    acc = mk(group_sum<L>(acc.x), group_sum<L>(acc.y));
     if (lane == 0 && r < end) {
       if (mask && mask[r]) acc = mk(R(0), R(0));
       y[r] = acc;

@@ -250,11 +250,11 @@ __global__ void k_pt_permute(int64_t n, int k, const int32_t* from, const T* src
 template <int NT>
 __device__ __forceinline__ void block_partials(const RedSite& rs, int Gt, int at, double2 d1,
                                                double2 d2) {
-  d1 = block_sum<NT>(d1);
-  d2 = block_sum<NT>(d2);
+  double2 d[2] = {d1, d2};
+  block_sums<NT, 2>(d);
   if (threadIdx.x == 0) {
-    rs.part[at] = d1;
-    rs.part[Gt + at] = d2;
+    rs.part[at] = d[0];
+    rs.part[Gt + at] = d[1];
   }
 }
 
