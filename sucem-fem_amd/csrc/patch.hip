@@ -375,7 +375,8 @@ __global__ __launch_bounds__(patch_threads(CB), patch_waves(ORDER, sizeof(R) == 
     const double* __restrict__ ref_face, R cs, R ct, R c0, const uint8_t* __restrict__ mask,
     const typename C2<R>::T* __restrict__ x, typename C2<R>::T* __restrict__ y,
     typename C2<R>::T* __restrict__ part, const typename C2<R>::T* w, RedSite rs,
-    const typename C2<R>::T* __restrict__ z, typename C2<R>::T* pnew, int Gr, RedSite rb) {
+    const typename C2<R>::T* __restrict__ z, typename C2<R>::T* pnew, int Gr, RedSite rb,
+    int64_t vec_stride, int64_t part_stride) {
   using C = typename C2<R>::T;
   constexpr bool E3 = EPI == 3 || EPI == 4;   // COCG form (EPI 4: paired systems)
   constexpr bool PR = EPI == 4;
@@ -389,6 +390,11 @@ __global__ __launch_bounds__(patch_threads(CB), patch_waves(ORDER, sizeof(R) == 
   // forms instead (in FP32 their registers cost a wave per SIMD)
   constexpr bool QF = E3 && sizeof(R) == 8;
   constexpr bool WY = EPI != 0 && !QF;
+  if constexpr (EPI == 0) {   // one grid row per vector
+    x += blockIdx.y * vec_stride;
+    y += blockIdx.y * vec_stride;
+    part += blockIdx.y * part_stride;
+  }
   extern __shared__ double2 smem_[];
   C* sm = reinterpret_cast<C*>(smem_);
   const int lb = xcd_block(Gp);
@@ -613,8 +619,13 @@ __global__ __launch_bounds__(TB) void k_mf_psum(int npd, int Gg, int Gt, int at0
                                                 const uint8_t* __restrict__ mask,
                                                 typename C2<R>::T* __restrict__ y,
                                                 const typename C2<R>::T* __restrict__ w,
-                                                RedSite rs) {
+                                                RedSite rs, int64_t vec_stride,
+                                                int64_t part_stride) {
   using C = typename C2<R>::T;
+  if constexpr (EPI == 0) {   // one grid row per vector
+    y += blockIdx.y * vec_stride;
+    part += blockIdx.y * part_stride;
+  }
   const int lb = xcd_block(Gg);
   int chunk = (npd + Gg - 1) / Gg;
   chunk = (chunk + TB - 1) / TB * TB;
@@ -907,7 +918,7 @@ void pt_validate(Context* c, const Space* s, const PatchMaps& pm, const std::vec
 template <typename R, int ORDER, int NFD, int CB>
 void launch_patch(Context* c, const System* sys, const PatchMaps& pm, Coef k,
                   const uint8_t* mask, const void* x, void* y, const void* w, int epi,
-                  const RedSite& rs, int Gp, int Gt, const PtUpdate* up = nullptr) {
+                  const RedSite& rs, int Gp, int Gt, const PtUpdate* up = nullptr, int nvec = 1) {
   using C = typename C2<R>::T;
   const Space* s = sys->space;
   const R* coef;
@@ -927,7 +938,7 @@ void launch_patch(Context* c, const System* sys, const PatchMaps& pm, Coef k,
 #define PT_ARGS pm.np, Gp, Gt, s->mesh->nc, s->nbf, pm.lds, coef, pm.lp.p, pm.uptr.p, pm.dof.p, \
                 pm.seg.p, pm.out.p, pm.fptr.p, s->pt_fmeta.p, pm.fpos.p, hf, s->ref_face_dofs.p, \
                 s->ref_face.p, (R)k.s, (R)k.t, c0, mask, (const C*)x, (C*)y, (C*)sys->pt_part.p, \
-                (const C*)w, rs, z, pnew, Gr, rb
+                (const C*)w, rs, z, pnew, Gr, rb, s->ndofs, pm.npe
   if (up) {
     SUCEM_CHECK((epi == 3 || epi == 4) && patch_updates(ORDER, CB, sizeof(R) == 4),
                 SUCEM_ERR_INTERNAL, "p update not available in this form");
@@ -935,7 +946,7 @@ void launch_patch(Context* c, const System* sys, const PatchMaps& pm, Coef k,
       if (epi == 3) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 3, CB, true>), Gp, nt, lds, c->stream, PT_ARGS);
       else SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 4, CB, true>), Gp, nt, lds, c->stream, PT_ARGS);
     }
-  } else if (epi == 0) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 0, CB, false>), Gp, nt, lds, c->stream, PT_ARGS);
+  } else if (epi == 0) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 0, CB, false>), dim3(Gp, nvec), nt, lds, c->stream, PT_ARGS);
   else if (epi == 1) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 1, CB, false>), Gp, nt, lds, c->stream, PT_ARGS);
   else if (epi == 2) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 2, CB, false>), Gp, nt, lds, c->stream, PT_ARGS);
   else if (epi == 3) SUCEM_LAUNCH((k_mf_patch<R, ORDER, NFD, 3, CB, false>), Gp, nt, lds, c->stream, PT_ARGS);
@@ -1028,7 +1039,7 @@ SpmvCfg pt_cfg(const Space* s, int cb, int G) {
 
 template <typename R>
 void pt_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const void* x, void* y,
-              const void* w, int epi, const RedSite& rs, const SpmvCfg& f) {
+              const void* w, int epi, const RedSite& rs, const SpmvCfg& f, int nvec) {
   using C = typename C2<R>::T;
   const Space* s = sys->space;
   const int slot = cb_slot(f.U);
@@ -1042,26 +1053,30 @@ void pt_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const 
               "bad patch operator launch configuration");
   SUCEM_CHECK(pt_fits<R>(s, f.U), SUCEM_ERR_UNSUPPORTED,
               "the patch operator needs more LDS per workgroup than the device has");
-  SUCEM_CHECK((int64_t)sys->pt_part.n >= pm.npe, SUCEM_ERR_INVALID, "patch operator not prepared");
+  SUCEM_CHECK(nvec == 1 || (epi == 0 && nvec > 0 && nvec <= 65535), SUCEM_ERR_INTERNAL,
+              "several vectors without an epilogue only");
+  SUCEM_CHECK((int64_t)sys->pt_part.n * (int64_t)sizeof(double2) >=
+                  nvec * pm.npe * (int64_t)sizeof(C),
+              SUCEM_ERR_INVALID, "patch operator not prepared");
   if (s->order == 2) {
-    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
-    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
-    else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
-    else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
+    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
+    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
+    else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
+    else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
   } else {
     SUCEM_CHECK(f.U == 256, SUCEM_ERR_UNSUPPORTED, "order-1 patches hold 256 cells");
-    launch_patch<R, 1, 3, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt);
+    launch_patch<R, 1, 3, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
   }
   const int npd = (int)pm.npd;
 #define PS_ARGS npd, Gg, Gt, Gp, pm.qptr.p, pm.qdof.p, (const C*)sys->pt_part.p, mask, (C*)y, \
-                (const C*)w, rs
-  if (epi == 0) SUCEM_LAUNCH((k_mf_psum<R, 0>), Gg, TB, 0, c->stream, PS_ARGS);
+                (const C*)w, rs, s->ndofs, pm.npe
+  if (epi == 0) SUCEM_LAUNCH((k_mf_psum<R, 0>), dim3(Gg, nvec), TB, 0, c->stream, PS_ARGS);
   else if (epi == 1) SUCEM_LAUNCH((k_mf_psum<R, 1>), Gg, TB, 0, c->stream, PS_ARGS);
   else SUCEM_LAUNCH((k_mf_psum<R, 2>), Gg, TB, 0, c->stream, PS_ARGS);
 #undef PS_ARGS
 }
 template void pt_apply<float>(Context*, const System*, Coef, const uint8_t*, const void*, void*,
-                              const void*, int, const RedSite&, const SpmvCfg&);
+                              const void*, int, const RedSite&, const SpmvCfg&, int);
 
 int pt_deferred_parts(const System* sys, const SpmvCfg& f) {
   if (f.mf != 2 || !sys->pt_ready) return 0;
@@ -1110,6 +1125,27 @@ const int32_t* pt_qcode(const System* sys, const SpmvCfg& f) {
 }
 const void* pt_partials(const System* sys) { return sys->pt_part.p; }
 template void pt_apply<double>(Context*, const System*, Coef, const uint8_t*, const void*, void*,
-                               const void*, int, const RedSite&, const SpmvCfg&);
+                               const void*, int, const RedSite&, const SpmvCfg&, int);
+
+template <typename R>
+int pt_vectors(Context* c, const System* sys, const SpmvCfg& f, int64_t nvec) {
+  const PatchMaps& pm = pt_maps(sys->space, f.U);
+  const int64_t one = std::max<int64_t>(pm.npe, 1) * (int64_t)sizeof(typename C2<R>::T);
+  const int64_t have = (int64_t)sys->pt_part.n * (int64_t)sizeof(double2);
+  // a captured call allocates nothing: it takes what fits the buffer as it is
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess) (void)hipGetLastError();
+  const bool grow = cap == hipStreamCaptureStatusNone;
+  const int64_t fit = (grow ? std::max(have, int64_t(64) << 20) : have) / one;
+  const int nv = (int)std::max<int64_t>(1, std::min<int64_t>({nvec, fit, 64}));
+  if (nv * one > have) {
+    System* ms = const_cast<System*>(sys);
+    ms->pt_part.release_synced();
+    ms->pt_part.alloc((size_t)((nv * one + 15) / 16));
+  }
+  return nv;
+}
+template int pt_vectors<float>(Context*, const System*, const SpmvCfg&, int64_t);
+template int pt_vectors<double>(Context*, const System*, const SpmvCfg&, int64_t);
 
 }  // namespace sucem

@@ -89,3 +89,23 @@ def test_paired_solve_on_small_patches():
     r, bb = (bd - y).cpu().numpy(), b
     assert np.linalg.norm(r.real) <= 1.1e-11 * np.linalg.norm(bb.real)
     assert np.linalg.norm(r.imag) <= 1.1e-11 * np.linalg.norm(bb.imag)
+
+
+@pytest.mark.parametrize("n,order", [((7, 3, 1), 2), ((7, 6, 5), 2), ((9, 9, 8), 1)])
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("nvec", [2, 65, 70])
+def test_vectors_of_one_call_equal_single_calls(n, order, precision, nvec):
+    """Vectors that share a launch (up to 64) give the results of one call each, bit for bit."""
+    import torch
+    from sucemfem.Utilities.Workloads import DeviceProblem
+    torch.cuda.set_device(0)
+    p = DeviceProblem(n, np.array(n) * 0.05, order, 7, (1.0, 2.2, 4.4), 3)
+    dt = torch.complex128 if precision == 64 else torch.complex64
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    x = torch.randn(nvec, p.ndofs, dtype=dt, device="cuda", generator=g)
+    y, one = torch.zeros_like(x), torch.zeros_like(x)
+    p.apply(15.0, x, y, precision=precision, nvec=nvec)
+    for v in range(nvec):
+        p.apply(15.0, x[v], one[v], precision=precision)
+    assert torch.equal(y, one)
