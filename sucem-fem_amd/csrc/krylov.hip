@@ -120,6 +120,74 @@ __global__ void k_copy(int n, int G, const C* src, C* dst) {
   for (int i = rr.start + threadIdx.x; i < rr.end; i += TB) dst[i] = src[i];
 }
 
+// Sum of the G <= FOLD_MAX block partials part[0, G), in every block the same and bit for bit
+// what k_finalize gets: the kernel that needs a scalar then forms it itself, and the
+// one-block launch between producer and consumer (4.4 us, as long as the kernels around it on
+// small systems) is saved.  Beyond FOLD_MAX partials, reading them in every block would cost
+// more than that launch.
+constexpr int FOLD_MAX = 1024;
+__device__ __forceinline__ double2 sum_parts(const double2* part, int G) {
+  constexpr int W = TB / 64, Q = FOLD_MAX / TB;   // waves, segments of 64 per wave
+  __shared__ double2 seg[FOLD_MAX / 64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double2 v[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int i = (q * W + w) * 64 + lane;
+    v[q] = i < G ? part[i] : make_double2(0.0, 0.0);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    v[q] = make_double2(group_sum<64>(v[q].x), group_sum<64>(v[q].y));
+    if (lane == 0) seg[q * W + w] = v[q];
+  }
+  __syncthreads();
+  double2 s = seg[0];
+#pragma unroll
+  for (int i = 1; i < FOLD_MAX / 64; ++i) { s.x += seg[i].x; s.y += seg[i].y; }
+  return s;
+}
+
+// The scalars of a step formed by the consuming kernels (fold): every block gets the same
+// value, and block 0 stores what later kernels read.  Slots that the same kernel's blocks
+// read are never written: rho for the next alpha is in S_RHO_NEXT, and becomes S_RHO, the
+// previous rho that beta divides by, with alpha.
+__device__ __forceinline__ double2 fold_alpha(const RedSite& rs, int G) {
+  const double2 s0 = sum_parts(rs.part, G), rho = scal2(rs.scal, S_RHO_NEXT);
+  const double2 al = cdiv0(rho, s0);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    rs.scal[S_ALPHA] = al.x; rs.scal[S_ALPHA + 1] = al.y;
+    rs.scal[S_RHO] = rho.x; rs.scal[S_RHO + 1] = rho.y;
+  }
+  return al;
+}
+__device__ __forceinline__ double2 fold_omega(const RedSite& rs, int G) {
+  const double2 s0 = sum_parts(rs.part, G), s1 = sum_parts(rs.part + G, G);
+  const double2 om = s1.x == 0.0 ? make_double2(0.0, 0.0)
+                                 : make_double2(s0.x / s1.x, -s0.y / s1.x);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    rs.scal[S_OMEGA] = om.x; rs.scal[S_OMEGA + 1] = om.y;
+  }
+  return om;
+}
+__device__ __forceinline__ double2 fold_beta(const RedSite& rs, int G, bool bicg) {
+  double* sc = rs.scal;
+  const double2 s0 = sum_parts(rs.part, G);
+  double2 be = cdiv0(s0, scal2(sc, S_RHO));
+  if (bicg) be = cmuld(be, cdiv0(scal2(sc, S_ALPHA), scal2(sc, S_OMEGA)));
+  if (blockIdx.x == 0) {
+    const double2 s1 = sum_parts(rs.part + G, G);
+    if (threadIdx.x == 0) {
+      sc[S_BETA] = be.x; sc[S_BETA + 1] = be.y;
+      sc[S_RHO_NEXT] = s0.x; sc[S_RHO_NEXT + 1] = s0.y;
+      sc[S_RR] = s1.x;
+      if (rs.hist) rs.hist[rs.it] = sqrt(s1.x);
+    }
+  }
+  return be;
+}
+
 // ---- COCG -------------------------------------------------------------------
 // p = dinv r
 template <typename C>
@@ -128,12 +196,13 @@ __global__ void k_cocg_start(int n, int G, const C* dinv, const C* r, C* p) {
   for (int i = rr.start + threadIdx.x; i < rr.end; i += TB) p[i] = cmul(dinv[i], r[i]);
 }
 
-// x += alpha p ; r -= alpha q ; reduce rho' = r.(dinv r) and |r|^2 (-> beta)
+// x += alpha p ; r -= alpha q ; reduce rho' = r.(dinv r) and |r|^2 (-> beta).  Ga > 0: alpha
+// from the operator's Ga partials in ra (fold_alpha).
 template <typename C>
 __global__ __launch_bounds__(TB) void k_cocg_xr(int n, int G, const double* scal, C* x, C* r,
                                                 const C* p, const C* q, const C* dinv,
-                                                RedSite rs) {
-  const C a = from_d<C>(scal2(scal, S_ALPHA));
+                                                RedSite rs, int Ga, RedSite ra) {
+  const C a = from_d<C>(Ga > 0 ? fold_alpha(ra, Ga) : scal2(scal, S_ALPHA));
   Range rr = block_rows(n, G);
   double2 nr = make_double2(0, 0), n2 = make_double2(0, 0);
   for (int i = rr.start + threadIdx.x; i < rr.end; i += TB) {
@@ -279,10 +348,11 @@ __global__ void k_cocg_pz(int n, int G, const double* scal, const C* z, C* p) {
   }
 }
 
-// p = dinv r + beta p
+// p = dinv r + beta p.  Gb > 0: beta from the Gb partials of the last x/r update (fold_beta).
 template <typename C>
-__global__ void k_cocg_p(int n, int G, const double* scal, const C* dinv, const C* r, C* p) {
-  const C b = from_d<C>(scal2(scal, S_BETA));
+__global__ __launch_bounds__(TB) void k_cocg_p(int n, int G, const double* scal, const C* dinv,
+                                               const C* r, C* p, int Gb, RedSite rb) {
+  const C b = from_d<C>(Gb > 0 ? fold_beta(rb, Gb, false) : scal2(scal, S_BETA));
   Range rr = block_rows(n, G);
   for (int i = rr.start + threadIdx.x; i < rr.end; i += TB) {
     const C z = cmul(dinv[i], r[i]);
@@ -292,11 +362,14 @@ __global__ void k_cocg_p(int n, int G, const double* scal, const C* dinv, const 
 }
 
 // ---- BiCGStab (preconditioned; SciPy's formulation) ----------------------------
-// p = r + beta (p - omega v) (p = r on a restart) ; phat = dinv p
+// p = r + beta (p - omega v) (p = r on a restart) ; phat = dinv p.  Gb > 0: beta from the Gb
+// partials of the last x/r update (fold_beta).
 template <typename C>
-__global__ void k_bicg_p(int n, int G, int restart, const double* scal, const C* r, C* p,
-                         const C* v, const C* dinv, C* phat) {
-  const C b = from_d<C>(scal2(scal, S_BETA)), om = from_d<C>(scal2(scal, S_OMEGA));
+__global__ __launch_bounds__(TB) void k_bicg_p(int n, int G, int restart, const double* scal,
+                                               const C* r, C* p, const C* v, const C* dinv,
+                                               C* phat, int Gb, RedSite rb) {
+  const C om = from_d<C>(scal2(scal, S_OMEGA));
+  const C b = from_d<C>(Gb > 0 ? fold_beta(rb, Gb, true) : scal2(scal, S_BETA));
   Range rr = block_rows(n, G);
   for (int i = rr.start + threadIdx.x; i < rr.end; i += TB) {
     const C ri = r[i];
@@ -312,11 +385,12 @@ __global__ void k_bicg_p(int n, int G, int restart, const double* scal, const C*
   }
 }
 
-// s = r - alpha v ; shat = dinv s
+// s = r - alpha v ; shat = dinv s.  Ga > 0: alpha from the operator's Ga partials in ra.
 template <typename C>
-__global__ void k_bicg_s(int n, int G, const double* scal, const C* r, const C* v, const C* dinv,
-                         C* s, C* shat) {
-  const C a = from_d<C>(scal2(scal, S_ALPHA));
+__global__ __launch_bounds__(TB) void k_bicg_s(int n, int G, const double* scal, const C* r,
+                                               const C* v, const C* dinv, C* s, C* shat, int Ga,
+                                               RedSite ra) {
+  const C a = from_d<C>(Ga > 0 ? fold_alpha(ra, Ga) : scal2(scal, S_ALPHA));
   Range rr = block_rows(n, G);
   for (int i = rr.start + threadIdx.x; i < rr.end; i += TB) {
     const C av = cmul(a, v[i]), ri = r[i];
@@ -326,12 +400,15 @@ __global__ void k_bicg_s(int n, int G, const double* scal, const C* r, const C* 
   }
 }
 
-// x += alpha phat + omega shat ; r = s - omega t ; reduce conj(rt).r and |r|^2 (-> beta)
+// x += alpha phat + omega shat ; r = s - omega t ; reduce conj(rt).r and |r|^2 (-> beta).
+// Go > 0: omega from the operator's Go partials in ro.
 template <typename C>
 __global__ __launch_bounds__(TB) void k_bicg_x(int n, int G, const double* scal, C* x, C* r,
                                                const C* s, const C* t, const C* phat,
-                                               const C* shat, const C* rt, RedSite rs) {
-  const C o = from_d<C>(scal2(scal, S_OMEGA)), a = from_d<C>(scal2(scal, S_ALPHA));
+                                               const C* shat, const C* rt, RedSite rs, int Go,
+                                               RedSite ro) {
+  const C o = from_d<C>(Go > 0 ? fold_omega(ro, Go) : scal2(scal, S_OMEGA));
+  const C a = from_d<C>(scal2(scal, S_ALPHA));
   Range rr = block_rows(n, G);
   double2 nr = make_double2(0, 0), n2 = make_double2(0, 0);
   for (int i = rr.start + threadIdx.x; i < rr.end; i += TB) {
@@ -645,12 +722,28 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
   // reduction epilogue, not the one-block finalisation) is bracketed by two events on the
   // solve's stream; the pair is read back after the interval's host check has synchronised.
   OpTimer timer;
+  // Jacobi COCG and BiCGStab form their scalars in the consuming kernels where the partials
+  // are few (fold_alpha and the others): Ga of the operator, Gf of the vector kernels, or
+  // both 0 (the folded and the separate forms keep rho in different slots).
+  // beta is left to the next p update except before a host check, which reads the history
+  // entry that comes with it (`due_b`).  BiCGStab with Jacobi on 4,125 rows: 8 launches of an
+  // iteration become 5, 24.8 -> BICGUS us.
+  const bool fold = !grad && op.flo.parts() <= FOLD_MAX && G <= FOLD_MAX;
+  const int Ga = fold ? op.flo.parts() : 0, Gf = fold ? G : 0;
+  int due_b = 0;
+  RedSite last_b{};
+  auto update_done = [&](const RedSite& rs) {
+    const bool check = (it + 1) % o.check_every == 0 || it + 1 == o.max_iter;
+    due_b = check ? 0 : Gf;
+    if (due_b) last_b = rs;
+    else finish_reduction(c, rs, G);
+  };
   auto apply_epi = [&](const void* xv, void* yv, const void* wv, int epi, const RedSite& rs) {
     const bool sample = it >= o.check_every && it % o.check_every == 0;
     if (sample) timer.start(c);
     op.apply_lo(xv, yv, wv, epi, rs);
     if (sample) timer.stop(c);
-    finish_reduction(c, rs, op.flo.parts());
+    if (Ga == 0) finish_reduction(c, rs, op.flo.parts());
   };
   // grid of the preconditioner's z kernel in that loop (4 blocks per CU: 23.4 against
   // 24.7 us per FP32 application with the 8 of the other vector kernels, which lose more
@@ -696,22 +789,26 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
       SUCEM_LAUNCH((k_cocg_pz<C>), G, TB, 0, c->stream, n, G, scal.p, z.p, p.p);
       st.spmv_lo += 1;
     } else if (cocg) {
-      apply_epi(p.p, q.p, p.p, 1, site(SITE_SPMV1, FIN_COCG_ALPHA));
+      const RedSite ra = site(SITE_SPMV1, FIN_COCG_ALPHA), rb = site(SITE_UPDATE, FIN_COCG_BETA, it);
+      apply_epi(p.p, q.p, p.p, 1, ra);
       SUCEM_LAUNCH((k_cocg_xr<C>), G, TB, 0, c->stream, n, G, scal.p, xlo, r.p, p.p, q.p, dinv.p,
-                   site(SITE_UPDATE, FIN_COCG_BETA, it));
-      finish_reduction(c, site(SITE_UPDATE, FIN_COCG_BETA, it), G);
-      SUCEM_LAUNCH((k_cocg_p<C>), G, TB, 0, c->stream, n, G, scal.p, dinv.p, r.p, p.p);
+                   rb, Ga, ra);
+      update_done(rb);
+      SUCEM_LAUNCH((k_cocg_p<C>), G, TB, 0, c->stream, n, G, scal.p, dinv.p, r.p, p.p, due_b, rb);
       st.spmv_lo += 1;
     } else {
       SUCEM_LAUNCH((k_bicg_p<C>), G, TB, 0, c->stream, n, G, restart, scal.p, r.p, p.p, v.p, dinv.p,
-                   phat.p);
+                   phat.p, due_b, last_b);
       restart = 0;
-      apply_epi(phat.p, v.p, rt.p, 2, site(SITE_SPMV1, FIN_BICG_ALPHA));
-      SUCEM_LAUNCH((k_bicg_s<C>), G, TB, 0, c->stream, n, G, scal.p, r.p, v.p, dinv.p, s.p, shat.p);
-      apply_epi(shat.p, t.p, s.p, 2, site(SITE_SPMV2, FIN_BICG_OMEGA));
+      const RedSite ra = site(SITE_SPMV1, FIN_BICG_ALPHA), ro = site(SITE_SPMV2, FIN_BICG_OMEGA);
+      const RedSite rb = site(SITE_UPDATE, FIN_BICG_BETA, it);
+      apply_epi(phat.p, v.p, rt.p, 2, ra);
+      SUCEM_LAUNCH((k_bicg_s<C>), G, TB, 0, c->stream, n, G, scal.p, r.p, v.p, dinv.p, s.p, shat.p,
+                   Ga, ra);
+      apply_epi(shat.p, t.p, s.p, 2, ro);
       SUCEM_LAUNCH((k_bicg_x<C>), G, TB, 0, c->stream, n, G, scal.p, xlo, r.p, s.p, t.p, phat.p,
-                   shat.p, rt.p, site(SITE_UPDATE, FIN_BICG_BETA, it));
-      finish_reduction(c, site(SITE_UPDATE, FIN_BICG_BETA, it), G);
+                   shat.p, rt.p, rb, Ga, ro);
+      update_done(rb);
       st.spmv_lo += 2;
     }
     const bool check = ((it + 1) % o.check_every) == 0 || it + 1 == o.max_iter;
