@@ -1,5 +1,6 @@
 // extern "C" entry points of libsucem_hip (declared in include/sucem_hip.h).
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -25,6 +26,32 @@ double* Context::host_scratch(size_t count) {
     pinned_n = want;
   }
   return pinned;
+}
+
+double* Context::next_mail(unsigned long long& seq) {
+  if (!mail_h) {
+    SUCEM_HIP(hipHostMalloc((void**)&mail_h, 64, hipHostMallocMapped | hipHostMallocCoherent));
+    std::memset(mail_h, 0, 64);
+    SUCEM_HIP(hipHostGetDevicePointer((void**)&mail_d, mail_h, 0));
+  }
+  seq = ++mail_seq;
+  return mail_d;
+}
+
+double Context::wait_mail() {
+  const auto* word = reinterpret_cast<const unsigned long long*>(mail_h + 1);
+  auto arrived = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) == mail_seq; };
+  // a short interval's message is watched for; a long one's (or a device error) is left to
+  // the stream
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+  while (!arrived() && std::chrono::steady_clock::now() < until) __builtin_ia32_pause();
+  if (!arrived()) {
+    sync();
+    SUCEM_CHECK(arrived(), SUCEM_ERR_INTERNAL, "a kernel did not report its value");
+  }
+  double v;
+  __atomic_load(mail_h, &v, __ATOMIC_RELAXED);
+  return v;
 }
 
 // ---- device memory pools (common.hpp) ---------------------------------------------------
@@ -218,6 +245,7 @@ int sucem_ctx_destroy(sucem_ctx* ctx) {
     (void)hipStreamDestroy(c.aux_stream);
   }
   if (c.pinned) (void)hipHostFree(c.pinned);
+  if (c.mail_h) (void)hipHostFree(c.mail_h);
   if (c.own_stream) (void)hipStreamDestroy(c.stream);
   c.pool->close();
   if (current_pool() == c.pool) current_pool().reset();

@@ -177,6 +177,14 @@ struct Context {
     current_pool() = pool;
   }
   double* host_scratch(size_t n);
+  // One value from a kernel to the host without a copy: next_mail numbers the message and
+  // gives the kernel its address in pinned memory (a value and a sequence number), wait_mail
+  // waits until that message has arrived and returns its value.
+  double* mail_h = nullptr;   // host and device view of the two words
+  double* mail_d = nullptr;
+  unsigned long long mail_seq = 0;
+  double* next_mail(unsigned long long& seq);
+  double wait_mail();
 };
 
 // typed view of workspace slot k holding `count` elements

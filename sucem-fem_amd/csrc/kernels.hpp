@@ -205,7 +205,21 @@ struct RedSite {
   int mode;
   int it;
   int paired = 0;     // two real systems packed as real and imaginary parts (see pmul)
+  // where the host waits for the value this site ends with (|r|, or the true |b - A x|^2):
+  // the value and behind it seq, in pinned memory (null: nobody waits)
+  double* host = nullptr;
+  unsigned long long seq = 0;
 };
+
+// A value for the waiting host (Context::wait_mail), by one thread.  It is there as soon as it
+// is written; a copy behind the kernel would take a launch and its completion (about 15 us
+// for every host check).
+__device__ __forceinline__ void post(const RedSite& rs, double v) {
+  if (!rs.host) return;
+  __hip_atomic_store(rs.host, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(rs.host + 1), rs.seq, __ATOMIC_RELEASE,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Paired recursions: the larger of the two systems' squared residual norms s.x, s.y, each
 // relative to its |b|^2 (a system with b = 0 counts as solved).
@@ -231,11 +245,13 @@ __device__ __forceinline__ void finalize(const RedSite& rs, double2 s0, double2 
       sc[S_RHO_NEXT] = s0.x; sc[S_RHO_NEXT + 1] = s0.y;
       sc[S_RR] = s1.x;
       if (rs.hist) rs.hist[rs.it] = sqrt(s1.x);
+      post(rs, sqrt(s1.x));
       break;
     case FIN_RESID:   // paired: S_TRUE holds the larger relative square (see prel2)
       sc[S_TRUE] = rs.paired ? prel2(sc, s0) : s0.x;
       sc[S_RHO] = s1.x; sc[S_RHO + 1] = s1.y;
       sc[S_RHO_NEXT] = s1.x; sc[S_RHO_NEXT + 1] = s1.y;
+      post(rs, sc[S_TRUE]);
       break;
     case FIN_NORM:
       sc[S_BNORM] = s0.x;
@@ -259,6 +275,7 @@ __device__ __forceinline__ void finalize(const RedSite& rs, double2 s0, double2 
       sc[S_RHO_NEXT] = s0.x; sc[S_RHO_NEXT + 1] = s0.y;
       sc[S_RR] = s1.x;
       if (rs.hist) rs.hist[rs.it] = sqrt(s1.x);
+      post(rs, sqrt(s1.x));
       break;
     }
     default:

@@ -326,6 +326,7 @@ __global__ __launch_bounds__(TB) void k_cocg_pz_b(int n, int G, int Gr, RedSite 
       // paired: the larger of the two relative residuals, squared (see prel2)
       sc[S_RR] = pr ? prel2(sc, s1) : s1.x;
       if (rs.hist) rs.hist[rs.it] = sqrt(sc[S_RR]);
+      post(rs, sqrt(sc[S_RR]));
     }
   }
   const C b = from_d<C>(be);
@@ -574,7 +575,12 @@ struct OpTimer {
   void harvest() {
     if (!pending) return;
     float ms = 0.f;
-    SUCEM_HIP(hipEventElapsedTime(&ms, e0, e1));
+    const hipError_t e = hipEventElapsedTime(&ms, e0, e1);
+    if (e == hipErrorNotReady) {   // done, but not yet seen to be: at the next check
+      (void)hipGetLastError();
+      return;
+    }
+    SUCEM_HIP(e);
     pending = false;
     total_ms += ms;
     ++samples;
@@ -635,6 +641,12 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
     r.mode = mode;
     r.it = it;
     r.paired = paired ? 1 : 0;
+    return r;
+  };
+
+  // the same site with its value sent to the host (c->wait_mail())
+  auto mailed = [&](RedSite r) {
+    r.host = c->next_mail(r.seq);
     return r;
   };
 
@@ -727,7 +739,7 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
   // both 0 (the folded and the separate forms keep rho in different slots).
   // beta is left to the next p update except before a host check, which reads the history
   // entry that comes with it (`due_b`).  BiCGStab with Jacobi on 4,125 rows: 8 launches of an
-  // iteration become 5, 24.8 -> BICGUS us.
+  // iteration become 5, 24.8 -> 21.5 us.
   const bool fold = !grad && op.flo.parts() <= FOLD_MAX && G <= FOLD_MAX;
   const int Ga = fold ? op.flo.parts() : 0, Gf = fold ? G : 0;
   int due_b = 0;
@@ -736,7 +748,7 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
     const bool check = (it + 1) % o.check_every == 0 || it + 1 == o.max_iter;
     due_b = check ? 0 : Gf;
     if (due_b) last_b = rs;
-    else finish_reduction(c, rs, G);
+    else finish_reduction(c, check ? mailed(rs) : rs, G);
   };
   auto apply_epi = [&](const void* xv, void* yv, const void* wv, int epi, const RedSite& rs) {
     const bool sample = it >= o.check_every && it % o.check_every == 0;
@@ -779,13 +791,17 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
         due.Gr = Gz;
         due.rb = rb;
       } else {
-        SUCEM_LAUNCH((k_cocg_pz_b<C>), G, TB, 0, c->stream, n, G, Gz, rb, z.p, pc);
+        const bool check = (it + 1) % o.check_every == 0 || it + 1 == o.max_iter;
+        SUCEM_LAUNCH((k_cocg_pz_b<C>), G, TB, 0, c->stream, n, G, Gz, check ? mailed(rb) : rb,
+                     z.p, pc);
       }
       st.spmv_lo += 1;
     } else if (cocg && grad) {
       apply_epi(p.p, q.p, p.p, 1, site(SITE_SPMV1, FIN_COCG_ALPHA));
       SUCEM_LAUNCH((k_cocg_xr_plain<C>), G, TB, 0, c->stream, n, G, scal.p, xlo, r.p, p.p, q.p);
-      precondition(site(SITE_UPDATE, FIN_COCG_BETA, it));
+      const bool check = (it + 1) % o.check_every == 0 || it + 1 == o.max_iter;
+      const RedSite rb = site(SITE_UPDATE, FIN_COCG_BETA, it);
+      precondition(check ? mailed(rb) : rb);
       SUCEM_LAUNCH((k_cocg_pz<C>), G, TB, 0, c->stream, n, G, scal.p, z.p, p.p);
       st.spmv_lo += 1;
     } else if (cocg) {
@@ -813,7 +829,7 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
     }
     const bool check = ((it + 1) % o.check_every) == 0 || it + 1 == o.max_iter;
     if (!check) continue;
-    rel = read_scalar(c, hist.p + it) / bnorm;
+    rel = c->wait_mail() / bnorm;
     timer.harvest();
     if (!std::isfinite(rel)) {
       st.status = -1;   // breakdown
@@ -863,8 +879,8 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
     st.reliable_updates += 1;
     SUCEM_LAUNCH((k_residual<C>), G, TB, 0, c->stream, n, G, b, ax.p, op.mask, dinv.p, r.p,
                  cocg ? 1 : 0, site(SITE_RESID, FIN_RESID));
-    finish_reduction(c, site(SITE_RESID, FIN_RESID), G);
-    const double true_rel = std::sqrt(read_scalar(c, scal.p + S_TRUE)) / bnorm;
+    finish_reduction(c, mailed(site(SITE_RESID, FIN_RESID)), G);
+    const double true_rel = std::sqrt(c->wait_mail()) / bnorm;
     if (log_level >= 3)
       std::fprintf(stderr, "[sucem krylov] it %d: recursion %.3e, true %.3e%s (cycle %d)\n",
                    it + 1, rel, true_rel, cut ? " cut" : "", cyc);
