@@ -103,16 +103,16 @@ template <int M>
 __device__ __forceinline__ double lane_xor(double x) {
   return __hiloint2double(lane_xor<M>(__double2hiint(x)), lane_xor<M>(__double2loint(x)));
 }
-// Sum over aligned groups of L lanes, the same in every lane of a group; the order of a
-// butterfly from distance L / 2 down to 1.
-template <int L, typename R>
+// Sum over the lanes of aligned groups of L that are MIN apart, the same in all of them; the
+// order of a butterfly from distance L / 2 down to MIN.
+template <int L, int MIN = 1, typename R>
 __device__ __forceinline__ R group_sum(R x) {
-  if constexpr (L >= 64) x += lane_xor<32>(x);
-  if constexpr (L >= 32) x += lane_xor<16>(x);
-  if constexpr (L >= 16) x += lane_xor<8>(x);
-  if constexpr (L >= 8) x += lane_xor<4>(x);
-  if constexpr (L >= 4) x += lane_xor<2>(x);
-  if constexpr (L >= 2) x += lane_xor<1>(x);
+  if constexpr (L >= 64 && MIN <= 32) x += lane_xor<32>(x);
+  if constexpr (L >= 32 && MIN <= 16) x += lane_xor<16>(x);
+  if constexpr (L >= 16 && MIN <= 8) x += lane_xor<8>(x);
+  if constexpr (L >= 8 && MIN <= 4) x += lane_xor<4>(x);
+  if constexpr (L >= 4 && MIN <= 2) x += lane_xor<2>(x);
+  if constexpr (L >= 2 && MIN <= 1) x += lane_xor<1>(x);
   return x;
 }
 

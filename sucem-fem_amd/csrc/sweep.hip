@@ -14,15 +14,22 @@
 //                and runs the gather / element product / segment-sum phases of the patch
 //                operator for each system in turn (the per-system coefficients ct_j, c0_j
 //                scale the same registers), plus the block partials of p_j.q_j;
-//   k_sw_psum    rows of the DOFs shared by several patches (sums of partial sums);
-//   k_sw_alpha   one block: alpha_j = rho_j / (p_j.q_j) (0 for a finished system);
-//   k_sw_xr      x_j += alpha_j p_j, r_j -= alpha_j q_j;
+//   k_sw_xr_fold alpha_j = rho_j / (p_j.q_j) (0 for a finished system), summed from the
+//                operator's partials in every block; x_j += alpha_j p_j, r_j -= alpha_j q_j, with
+//                the rows of DOFs shared by several patches as the sums of their partial sums;
 //   k_sw_aux_t   vertex (and order-2 edge-node) rows of G^T r_j and Pi^T r_j, lanes =
 //                (system, incidence stride), so a row's gathers read whole [row][NB] lines;
 //   k_sw_aux_z   z_j = D_j^-1 r_j + theta G W_j G^T r_j + Pi V_j Pi^T r_j, partials of
 //                r_j.z_j and |r_j|^2;
-//   k_sw_beta    one block: beta_j, rho_j, |r_j| into a ring of the check interval;
-//   k_sw_pz      p_j = z_j + beta_j p_j.
+//   k_sw_pz_fold beta_j from those partials in every block, p_j = z_j + beta_j p_j; |r_j| into a
+//                ring of the check interval.
+//
+// Meshes of more than 2,048 patches, or with a DOF in more than 15 of them, run the shared
+// rows, alpha and beta as launches of their own (k_sw_psum, k_sw_alpha, k_sw_beta) around
+// k_sw_xr and k_sw_pz: every block summing that many partials would cost more than the three
+// launches.  Iteration with eight / five launches, us, FP32 / FP64, groups of 2: 48,000
+// order-1 cells 45.7 / 49.6 -> 32.4 / 34.4; 384,000 90.0 / 112.1 -> 73.5 / 94.6; 48,000
+// order-2 cells 105.8 / 121.8 -> 88.7 / 101.2 (the operator's batched loads included).
 //
 // The check interval's iterations (fixed launches, device-resident scalars) are captured
 // once per solve in a hipGraph on a library stream and replayed; between replays the host
@@ -45,9 +52,12 @@ namespace sucem {
 namespace {
 
 constexpr int TB = 256;
-constexpr int UBS = 8;       // patch DOFs per thread per gather / segment-sum batch
-constexpr int SW = 8;        // per-system scalars: rho (2), alpha (2), beta (2), spare (2)
-constexpr int SW_RHO = 0, SW_ALPHA = 2, SW_BETA = 4;
+// patch DOFs per thread per gather / segment-sum batch (one batch on the Kuhn meshes)
+constexpr int sw_batch(int order) { return order == 1 ? 3 : 8; }
+constexpr int SW = 8;        // per-system scalars: rho (2), alpha (2), beta (2), next rho (2)
+// SW_RHO: the previous rho, which beta divides by; SW_NEXT: rho for the next alpha (kernels
+// that form a scalar in every block do not write the slot that their blocks read)
+constexpr int SW_RHO = 0, SW_ALPHA = 2, SW_BETA = 4, SW_NEXT = 6;
 
 struct Rows { int start, end; };
 __device__ __forceinline__ Rows sw_rows(int n, int G) {
@@ -59,23 +69,33 @@ __device__ __forceinline__ Rows sw_rows(int n, int G) {
   return r;
 }
 
-// Per-system block sums: every thread holds a value of system tid % NB; thread t < NB
-// returns the block's sum for system t (fixed tree).  Contains barriers.
+// Per-system block sums of two values: every thread holds values of system tid % NB; thread
+// t < NB gets the block's sums for system t (fixed tree: the waves' lanes first, then a
+// butterfly over the lanes of a system).  Contains barriers.
 template <int NB>
-__device__ __forceinline__ double2 block_sum_nb(double2 v) {
-  __shared__ double2 red[TB];
+__device__ __forceinline__ void block_sum_nb(double2& a, double2& b) {
+  __shared__ double2 red[2][TB];
   const int t = threadIdx.x;
   __syncthreads();
-  red[t] = v;
+  red[0][t] = a;
+  red[1][t] = b;
   __syncthreads();
-  for (int step = TB / 2; step >= NB; step >>= 1) {
-    if (t < step) {
-      red[t].x += red[t + step].x;
-      red[t].y += red[t + step].y;
-    }
-    __syncthreads();
+  if (t < 64) {
+    auto total = [&](const double2* v) {
+      const double2 p = v[t], q = v[t + 64], r = v[t + 128], s = v[t + 192];
+      const double2 z = make_double2((p.x + r.x) + (q.x + s.x), (p.y + r.y) + (q.y + s.y));
+      return make_double2(group_sum<64, NB>(z.x), group_sum<64, NB>(z.y));
+    };
+    a = total(red[0]);
+    b = total(red[1]);
   }
-  return red[t < NB ? t : 0];
+}
+
+template <int NB>
+__device__ __forceinline__ double2 block_sum_nb(double2 v) {
+  double2 none = make_double2(0.0, 0.0);
+  block_sum_nb<NB>(v, none);
+  return v;
 }
 
 // ---- operator -------------------------------------------------------------------
@@ -85,10 +105,7 @@ __device__ __forceinline__ void block_sum_multi(double2 (&v)[NBL]) {
   __shared__ double2 red[CB / 64][NBL];
 #pragma unroll
   for (int jj = 0; jj < NBL; ++jj)
-    for (int o = 32; o > 0; o >>= 1) {
-      v[jj].x += __shfl_xor(v[jj].x, o);
-      v[jj].y += __shfl_xor(v[jj].y, o);
-    }
+    v[jj] = make_double2(group_sum<64>(v[jj].x), group_sum<64>(v[jj].y));
   const int w = threadIdx.x >> 6;
   __syncthreads();
   if ((threadIdx.x & 63) == 0)
@@ -112,7 +129,7 @@ __device__ __forceinline__ void block_sum_multi(double2 (&v)[NBL]) {
 // kco = {ct_0..ct_NB-1, c0_0..c0_NB-1} (cs = 1).  part: partial sums [slot][NB]; dp: with
 // EPI, block partials of p_j.q_j at dp[j Gp + lb].
 template <typename R, int ORDER, int NFD, int NB, int NBL, int CB, bool EPI>
-__global__ __launch_bounds__(CB) void k_sw_patch(
+__global__ __launch_bounds__(CB, ORDER == 1 || sizeof(R) == 4 ? 2 : 1) void k_sw_patch(
     int64_t np, int Gp, int64_t nc, int64_t nbf, int lds_main, const R* __restrict__ coef,
     const uint32_t* __restrict__ lp, const int32_t* __restrict__ uptr,
     const int32_t* __restrict__ pdof, const uint16_t* __restrict__ pseg,
@@ -127,6 +144,7 @@ __global__ __launch_bounds__(CB) void k_sw_patch(
   static_assert(NB % NBL == 0, "groups of NBL systems");
   constexpr int NLOC = MfTab<ORDER>::NLOC;
   constexpr int KK = NFD * NFD;
+  constexpr int UBS = sw_batch(ORDER);
   extern __shared__ double2 smem_[];
   C* sm = reinterpret_cast<C*>(smem_);
   const int lb = xcd_block(Gp);
@@ -156,22 +174,24 @@ __global__ __launch_bounds__(CB) void k_sw_patch(
 #pragma unroll
     for (int jj = 0; jj < NBL; ++jj) d1[jj] = make_double2(0.0, 0.0);
     if (live) {
+      // (indexes past the end are clamped, not branched around: a predicated load holds up the
+      // ones behind it)
       for (int j0 = 0; j0 < nu; j0 += UBS * CB) {
         int dv[UBS];
 #pragma unroll
-        for (int q = 0; q < UBS; ++q) {
-          const int jj = j0 + q * CB + threadIdx.x;
-          dv[q] = jj < nu ? pdof[u0 + jj] : -1;
-        }
+        for (int q = 0; q < UBS; ++q)
+          dv[q] = pdof[u0 + min(j0 + q * CB + (int)threadIdx.x, nu - 1)];
+        C xv[UBS][NBL];
+#pragma unroll
+        for (int q = 0; q < UBS; ++q)
+#pragma unroll
+          for (int jj = 0; jj < NBL; ++jj) xv[q][jj] = x[(int64_t)dv[q] * NB + jb + jj];
 #pragma unroll
         for (int q = 0; q < UBS; ++q) {
           const int u = j0 + q * CB + threadIdx.x;
-          if (dv[q] >= 0) {
-            C xv[NBL];
+          if (u < nu) {
 #pragma unroll
-            for (int jj = 0; jj < NBL; ++jj) xv[jj] = x[(int64_t)dv[q] * NB + jb + jj];
-#pragma unroll
-            for (int jj = 0; jj < NBL; ++jj) sm[u * NBL + jj] = xv[jj];
+            for (int jj = 0; jj < NBL; ++jj) sm[u * NBL + jj] = xv[q][jj];
           }
         }
       }
@@ -241,20 +261,36 @@ __global__ __launch_bounds__(CB) void k_sw_patch(
     }
     __syncthreads();
     if (live) {
+      int tq = threadIdx.x;   // opaque, so that the gather's ids are not held in registers
+      asm volatile("" : "+v"(tq));
       for (int j0 = 0; j0 < nu; j0 += UBS * CB) {
         int lo[UBS], hi[UBS], out[UBS], dv[UBS];
 #pragma unroll
         for (int q = 0; q < UBS; ++q) {
-          const int jj = j0 + q * CB + threadIdx.x;
-          const bool in = jj < nu;
-          lo[q] = (in && jj) ? (int)pseg[u0 + jj - 1] : 0;
-          hi[q] = in ? (int)pseg[u0 + jj] : 0;
-          out[q] = in ? pout[u0 + jj] : 0;
-          dv[q] = in ? pdof[u0 + jj] : 0;
+          const int jj = min(j0 + q * CB + tq, nu - 1);
+          lo[q] = jj ? (int)pseg[u0 + jj - 1] : 0;
+          hi[q] = (int)pseg[u0 + jj];
+          out[q] = pout[u0 + jj];
+          dv[q] = pdof[u0 + jj];
+        }
+        // the epilogue's x and the mask bytes are in flight while the segments are summed
+        C xe[EPI ? UBS : 1][NBL];
+        if constexpr (EPI) {
+#pragma unroll
+          for (int q = 0; q < UBS; ++q)
+#pragma unroll
+            for (int jj = 0; jj < NBL; ++jj) xe[q][jj] = x[(int64_t)dv[q] * NB + jb + jj];
+        }
+        uint8_t off[UBS];
+#pragma unroll
+        for (int q = 0; q < UBS; ++q) off[q] = 0;
+        if (mask) {
+#pragma unroll
+          for (int q = 0; q < UBS; ++q) off[q] = mask[dv[q]];
         }
 #pragma unroll
         for (int q = 0; q < UBS; ++q) {
-          if (hi[q] == 0) continue;   // not an entry of this patch (segments are never empty)
+          if (j0 + q * CB + tq >= nu) continue;   // not an entry of this patch
           C v[NBL];
 #pragma unroll
           for (int jj = 0; jj < NBL; ++jj) v[jj] = mk(R(0), R(0));
@@ -266,22 +302,16 @@ __global__ __launch_bounds__(CB) void k_sw_patch(
               v[jj].y += s.y;
             }
           }
-          const bool masked = out[q] < 0 && mask && mask[dv[q]];
+          const bool own = out[q] < 0;
+          C* dst = own ? y + (int64_t)dv[q] * NB + jb : part + (int64_t)out[q] * NB + jb;
 #pragma unroll
           for (int jj = 0; jj < NBL; ++jj) {
-            C w = v[jj];
-            if (out[q] >= 0) {
-              part[(int64_t)out[q] * NB + jb + jj] = w;
-            } else {
-              if (masked) w = mk(R(0), R(0));
-              y[(int64_t)dv[q] * NB + jb + jj] = w;
-            }
+            const C w = own && off[q] ? mk(R(0), R(0)) : v[jj];
+            dst[jj] = w;
             if constexpr (EPI) {
               // p.Ap over the finished rows and the partial sums (linear in q; p is zero
               // on masked rows)
-              const double2 xd = to_d(x[(int64_t)dv[q] * NB + jb + jj]), yd = to_d(w);
-              d1[jj].x += xd.x * yd.x - xd.y * yd.y;
-              d1[jj].y += xd.x * yd.y + xd.y * yd.x;
+              dot_acc(d1[jj], to_d(xe[q][jj]), to_d(w), false);
             }
           }
         }
@@ -347,11 +377,49 @@ __device__ __forceinline__ double2 wave_sum_partials(const double2* __restrict__
   }
   double2 v = make_double2((s[0].x + s[1].x) + (s[2].x + s[3].x),
                            (s[0].y + s[1].y) + (s[2].y + s[3].y));
-  for (int o = 32; o > 0; o >>= 1) {
-    v.x += __shfl_xor(v.x, o);
-    v.y += __shfl_xor(v.y, o);
+  return make_double2(group_sum<64>(v.x), group_sum<64>(v.y));
+}
+
+// The sum of the block partials of the thread's system (tid % NB), dp[j G + b], formed by
+// every block of the kernel that needs it.  All four waves share the work (one wave per
+// system, as in the one-block kernels below, leaves the others waiting for its chain of
+// loads), eight loads in flight each; fixed order.
+template <int NB>
+__device__ __forceinline__ double2 sw_fold(const double2* __restrict__ dp, int G) {
+  constexpr int W = TB / 64, WS = NB < W ? W / NB : 1;   // waves, waves per system
+  constexpr int U = 8, STEP = 64 * WS;
+  __shared__ double2 tot[W][NB < W ? 1 : NB / W];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < (NB < W ? 1 : NB / W); ++m) {
+    const int j = NB < W ? w / WS : m * W + w;
+    const int first = NB < W ? (w % WS) * 64 + lane : lane;
+    const double2* a = dp + (int64_t)j * G;
+    double2 s = make_double2(0.0, 0.0);
+    for (int b0 = 0; b0 < G; b0 += U * STEP) {
+      double2 v[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const int b = b0 + k * STEP + first;
+        v[k] = b < G ? a[b] : make_double2(0.0, 0.0);
+      }
+#pragma unroll
+      for (int k = 0; k < U; ++k) { s.x += v[k].x; s.y += v[k].y; }
+    }
+    s = make_double2(group_sum<64>(s.x), group_sum<64>(s.y));
+    if (lane == 0) tot[w][m] = s;
   }
-  return v;
+  __syncthreads();
+  const int j = threadIdx.x % NB;
+  if constexpr (NB >= W) return tot[j % W][j / W];
+  double2 r = tot[j * WS][0];
+#pragma unroll
+  for (int k = 1; k < WS; ++k) {
+    r.x += tot[(j * WS + k) % W][0].x;
+    r.y += tot[(j * WS + k) % W][0].y;
+  }
+  return r;
 }
 
 template <int NB>
@@ -386,13 +454,13 @@ __global__ __launch_bounds__(64 * NB) void k_sw_beta(int G, const double2* __res
       s[SW_BETA] = be.x;
       s[SW_BETA + 1] = be.y;
       if (on) {
-        s[SW_RHO] = s0.x;
-        s[SW_RHO + 1] = s0.y;
+        s[SW_RHO] = s[SW_NEXT] = s0.x;
+        s[SW_RHO + 1] = s[SW_NEXT + 1] = s0.y;
       }
       ring[k * NB + j] = sqrt(s1.x);
     } else if (sel[j]) {
-      s[SW_RHO] = s0.x;
-      s[SW_RHO + 1] = s0.y;
+      s[SW_RHO] = s[SW_NEXT] = s0.x;
+      s[SW_RHO + 1] = s[SW_NEXT + 1] = s0.y;
     }
   }
 }
@@ -425,6 +493,93 @@ __global__ __launch_bounds__(TB) void k_sw_xr(int n, int G, const double* __rest
     ri.x -= aq.x; ri.y -= aq.y;
     x[e] = xi;
     r[e] = ri;
+  }
+}
+
+// The x/r update after k_sw_patch alone: alpha_j from the operator's Gp partials in every
+// block, and a shared row's q as the sum of its partial sums (qcode, as k_cocg_xr_def_a), in
+// place of k_sw_psum and k_sw_alpha.  Block 0 stores alpha and moves the next rho to SW_RHO.
+template <typename R, int NB>
+__global__ __launch_bounds__(TB) void k_sw_xr_fold(int n, int G, int Gp,
+                                                   const double2* __restrict__ dp,
+                                                   const int* __restrict__ act, double* sc,
+                                                   const int32_t* __restrict__ qcode,
+                                                   const typename C2<R>::T* __restrict__ part,
+                                                   const uint8_t* __restrict__ mask,
+                                                   typename C2<R>::T* __restrict__ x,
+                                                   typename C2<R>::T* __restrict__ r,
+                                                   const typename C2<R>::T* __restrict__ p,
+                                                   const typename C2<R>::T* __restrict__ q) {
+  using C = typename C2<R>::T;
+  const Rows rr = sw_rows(n, G);
+  const int j = threadIdx.x % NB;
+  const double2 s = sw_fold<NB>(dp, Gp), rho = scal2(sc + j * SW, SW_NEXT);
+  const double2 al = act[j] ? cdiv0(rho, s) : make_double2(0, 0);
+  if (blockIdx.x == 0 && threadIdx.x < NB) {
+    double* o = sc + j * SW;
+    o[SW_ALPHA] = al.x;
+    o[SW_ALPHA + 1] = al.y;
+    o[SW_RHO] = rho.x;
+    o[SW_RHO + 1] = rho.y;
+  }
+  const C a = from_d<C>(al);
+  for (int64_t e = (int64_t)rr.start * NB + threadIdx.x; e < (int64_t)rr.end * NB; e += TB) {
+    const int i = (int)(e / NB);
+    const int code = qcode[i];
+    C qi;
+    if (code < 0) {
+      qi = q[e];
+    } else {
+      qi = mk(R(0), R(0));
+      const int q0 = code >> 4, q1 = q0 + (code & 15);
+      for (int t = q0; t < q1; ++t) {
+        const C v = part[(int64_t)t * NB + j];
+        qi.x += v.x;
+        qi.y += v.y;
+      }
+      if (mask && mask[i]) qi = mk(R(0), R(0));
+    }
+    const C ap = cmul(a, p[e]), aq = cmul(a, qi);
+    C xi = x[e], ri = r[e];
+    xi.x += ap.x; xi.y += ap.y;
+    ri.x -= aq.x; ri.y -= aq.y;
+    x[e] = xi;
+    r[e] = ri;
+  }
+}
+
+// p_j = z_j + beta_j p_j with beta_j from the preconditioner's G partials in every block, in
+// place of k_sw_beta; block 0 stores beta, the next rho and |r_j| in the ring.
+template <typename R, int NB>
+__global__ __launch_bounds__(TB) void k_sw_pz_fold(int n, int G, int Gz,
+                                                   const double2* __restrict__ dp,
+                                                   const int* __restrict__ act, double* sc,
+                                                   double* __restrict__ ring, int k,
+                                                   const typename C2<R>::T* __restrict__ z,
+                                                   typename C2<R>::T* __restrict__ p) {
+  using C = typename C2<R>::T;
+  const Rows rr = sw_rows(n, G);
+  const int j = threadIdx.x % NB;
+  const double2 s0 = sw_fold<NB>(dp, Gz);
+  const bool on = act[j] != 0;
+  const double2 be = on ? cdiv0(s0, scal2(sc + j * SW, SW_RHO)) : make_double2(0, 0);
+  if (blockIdx.x == 0) {
+    const double2 s1 = sw_fold<NB>(dp + (int64_t)NB * Gz, Gz);
+    if (threadIdx.x < NB) {
+      double* o = sc + j * SW;
+      o[SW_BETA] = be.x;
+      o[SW_BETA + 1] = be.y;
+      if (on) {
+        o[SW_NEXT] = s0.x;
+        o[SW_NEXT + 1] = s0.y;
+      }
+      ring[k * NB + j] = sqrt(s1.x);
+    }
+  }
+  const C b = from_d<C>(be);
+  for (int64_t e = (int64_t)rr.start * NB + threadIdx.x; e < (int64_t)rr.end * NB; e += TB) {
+    const C bp = cmul(b, p[e]), zi = z[e];
+    p[e] = mk(zi.x + bp.x, zi.y + bp.y);
   }
 }
 
@@ -635,16 +790,10 @@ __device__ __forceinline__ void sw_vertex_rows(int64_t blk, int nv, int nE, R in
       }
     }
   }
+  g = mk(group_sum<L, NB>(g.x), group_sum<L, NB>(g.y));
 #pragma unroll
-  for (int o = L / 2; o >= NB; o >>= 1) {
-    g.x += __shfl_xor(g.x, o);
-    g.y += __shfl_xor(g.y, o);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      acc[d].x += __shfl_xor(acc[d].x, o);
-      acc[d].y += __shfl_xor(acc[d].y, o);
-    }
-  }
+  for (int d = 0; d < 3; ++d)
+    acc[d] = mk(group_sum<L, NB>(acc[d].x), group_sum<L, NB>(acc[d].y));
   if (lr == 0 && v < nv) {
     w[v * NB + j] = cmul(winv[v * NB + j], mk(inv_den * g.x, inv_den * g.y));
 #pragma unroll
@@ -681,11 +830,7 @@ __device__ __forceinline__ void sw_edge_rows(int64_t blk, int nv, int nE, R inv_
       else { g.x += R(4) * (r0.x + r1.x); g.y += R(4) * (r0.y + r1.y); }
     }
   }
-#pragma unroll
-  for (int o = L / 2; o >= NB; o >>= 1) {
-    g.x += __shfl_xor(g.x, o);
-    g.y += __shfl_xor(g.y, o);
-  }
+  g = mk(group_sum<L, NB>(g.x), group_sum<L, NB>(g.y));
   if (lr == 0 && e < nE)
     w[(nv + e) * NB + j] = cmul(winv[(nv + e) * NB + j], mk(inv_den * g.x, inv_den * g.y));
 }
@@ -807,10 +952,11 @@ __global__ __launch_bounds__(TB) void k_sw_aux_z(int n, int G, int nv, int nE, R
     d1.y += rd.x * zd.y + rd.y * zd.x;
     d2.x += rd.x * rd.x + rd.y * rd.y;
   }
-  d1 = block_sum_nb<NB>(d1);
-  if (threadIdx.x < NB) dp[(int64_t)threadIdx.x * G + xcd_block(G)] = d1;
-  d2 = block_sum_nb<NB>(d2);
-  if (threadIdx.x < NB) dp[(int64_t)(NB + threadIdx.x) * G + xcd_block(G)] = d2;
+  block_sum_nb<NB>(d1, d2);
+  if (threadIdx.x < NB) {
+    dp[(int64_t)threadIdx.x * G + xcd_block(G)] = d1;
+    dp[(int64_t)(NB + threadIdx.x) * G + xcd_block(G)] = d2;
+  }
 }
 
 // ---- host driver --------------------------------------------------------------------
@@ -837,6 +983,9 @@ struct Chunk {
   const PatchMaps* pm;
   const PatchMaps* pm64;
   int Gp, Gp64, Gq;
+  // scalars and shared rows in the consuming kernels: five launches per iteration for eight,
+  // where the operator's partials are few enough to be summed by every block
+  bool fold;
   // device arrays (workspace slots 48..)
   C *x, *r, *p, *q, *z, *dinv, *w, *winv, *u, *vinv, *part;
   double2 *x64, *b64, *ax, *dp;
@@ -864,8 +1013,9 @@ struct Chunk {
       else SUCEM_LAUNCH((k_sw_patch<R, ORDER, NFD, NB, NBL, 192, false>), Gp, 192, lds, st, SW_PT);
     }
 #undef SW_PT
-    SUCEM_LAUNCH((k_sw_psum<R, NB>), Gq, TB, 0, st, (int)pm->npd, Gq, pm->qptr.p, pm->qdof.p,
-                 (const C*)part, mask, yout);
+    if (!fold)
+      SUCEM_LAUNCH((k_sw_psum<R, NB>), Gq, TB, 0, st, (int)pm->npd, Gq, pm->qptr.p, pm->qdof.p,
+                   (const C*)part, mask, yout);
   }
 
   // FP64 operator on x64 -> ax (all systems): the same kernels in FP64 with the FP64 maps
@@ -904,6 +1054,15 @@ struct Chunk {
   // one COCG iteration of every running system; k = slot of |r_j| in the ring
   void iteration(int k) {
     launch_patch(p, q, true);
+    if (fold) {
+      SUCEM_LAUNCH((k_sw_xr_fold<R, NB>), G, TB, 0, st, n, G, Gp, (const double2*)dp,
+                   (const int*)act, sc, pm->qcode.p, (const C*)part, mask, x, r, (const C*)p,
+                   (const C*)q);
+      precondition();
+      SUCEM_LAUNCH((k_sw_pz_fold<R, NB>), G, TB, 0, st, n, G, Gz, (const double2*)dp,
+                   (const int*)act, sc, ring, k, (const C*)z, p);
+      return;
+    }
     SUCEM_LAUNCH((k_sw_alpha<NB>), 1, 64 * NB, 0, st, Gp, (const double2*)dp, (const int*)act, sc);
     SUCEM_LAUNCH((k_sw_xr<R, NB>), G, TB, 0, st, n, G, (const double*)sc, x, r, (const C*)p,
                  (const C*)q);
@@ -956,6 +1115,7 @@ void sweep_chunk(Context* c, System* sys, int nb, const double* k0, const double
               SUCEM_ERR_UNSUPPORTED, "the batched patch kernel needs more LDS than the device has");
   k.Gp = (int)((k.pm->np + 7) / 8 * 8);
   k.Gp64 = (int)((k.pm64->np + 7) / 8 * 8);
+  k.fold = k.Gp <= 2048 && k.pm->qcode.p != nullptr;
   k.Gq = op_grid(c, std::max<int64_t>(std::max(k.pm->npd, k.pm64->npd), 1), 16);
   k.G = op_grid(c, n, 8);
   k.Gz = op_grid(c, n, 4);
