@@ -147,6 +147,22 @@ __device__ __forceinline__ double2 block_sum(double2 v) {
   return a[0];
 }
 
+// This thread's sum of the block partials part[tid], part[tid + NT], ..., in that order, four
+// loads in flight (the partials were written by other XCDs, so each load is a long one).
+template <int NT>
+__device__ __forceinline__ double2 thread_parts(const double2* part, int G) {
+  double2 s = make_double2(0, 0);
+  for (int k0 = threadIdx.x; k0 < G; k0 += 4 * NT) {
+    double2 t[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) t[q] = part[min(k0 + q * NT, G - 1)];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (k0 + q * NT < G) { s.x += t[q].x; s.y += t[q].y; }
+  }
+  return s;
+}
+
 // Logical block index that gives each XCD a contiguous share of the rows
 // (blocks are dispatched round-robin over the 8 XCDs; G is a multiple of 8).
 __device__ __forceinline__ int xcd_block(int G) {

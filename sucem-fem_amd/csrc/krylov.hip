@@ -244,7 +244,10 @@ __global__ void k_cocg_xr_plain(int n, int G, const double* scal, C* x, C* r, co
 // order, so they agree bit for bit, and the one-block finalising launch between the two
 // kernels is saved.  (Moving x += alpha p into the p update, which reads p anyway, was
 // measured: this kernel 30.3 -> 23.4 us, the p update 12.2 -> 20.9 us per FP32 application
-// at 40^3 order 2, so not kept.)
+// at 40^3 order 2, so not kept.)  A thread's first row is loaded before the partials are
+// summed, so the two round trips overlap (q of a shared row too, unused: waiting for its
+// qcode would stall the sum): 33 x 29 x 31 boxes order 1 FP64 7.4 -> 6.4 us, 40^3 order 2
+// FP32 30.1 -> 29.1 us; k_cocg_pz_b the same way 11.8 -> 10.2 us.
 // rho is read from S_RHO_NEXT, which no block of this kernel writes; block 0 stores alpha
 // and copies that rho to S_RHO, which the next p update reads as the previous rho.
 template <typename C>
@@ -253,12 +256,16 @@ __global__ __launch_bounds__(TB) void k_cocg_xr_def_a(int n, int G, int Gd, RedS
                                                       const int32_t* __restrict__ qcode,
                                                       const C* __restrict__ part,
                                                       const uint8_t* __restrict__ mask) {
-  double2 s0 = make_double2(0, 0);
-  for (int k = threadIdx.x; k < Gd; k += TB) {
-    const double2 t = rs.part[k];
-    s0.x += t.x;
-    s0.y += t.y;
-  }
+  const Range rr = block_rows(n, G);
+  int i = rr.start + threadIdx.x, code = -1;
+  C qi, pi, xi, ri;
+  auto load = [&] {
+    if (i >= rr.end) return;
+    code = qcode[i];
+    qi = q[i]; pi = p[i]; xi = x[i]; ri = r[i];
+  };
+  load();   // while the partials arrive
+  double2 s0 = thread_parts<TB>(rs.part, Gd);
   s0 = block_sum<TB>(s0);
   const double2 rho = scal2(rs.scal, S_RHO_NEXT);
   const bool pr = rs.paired;
@@ -270,13 +277,8 @@ __global__ __launch_bounds__(TB) void k_cocg_xr_def_a(int n, int G, int Gd, RedS
     rs.scal[S_RHO + 1] = rho.y;
   }
   const C a = from_d<C>(al);
-  Range rr = block_rows(n, G);
-  for (int i = rr.start + threadIdx.x; i < rr.end; i += TB) {
-    const int code = qcode[i];
-    C qi;
-    if (code < 0) {
-      qi = q[i];
-    } else {
+  while (i < rr.end) {
+    if (code >= 0) {
       qi = mk(decltype(qi.x)(0), decltype(qi.x)(0));
       const int q0 = code >> 4, q1 = q0 + (code & 15);
       for (int j = q0; j < q1; ++j) {
@@ -286,13 +288,13 @@ __global__ __launch_bounds__(TB) void k_cocg_xr_def_a(int n, int G, int Gd, RedS
       }
       if (mask && mask[i]) qi = mk(decltype(qi.x)(0), decltype(qi.x)(0));
     }
-    const C pi = p[i];
     const C ap = pr ? pmul(a, pi) : cmul(a, pi), aq = pr ? pmul(a, qi) : cmul(a, qi);
-    C xi = x[i], ri = r[i];
     xi.x += ap.x; xi.y += ap.y;
     ri.x -= aq.x; ri.y -= aq.y;
     x[i] = xi;
     r[i] = ri;
+    i += TB;
+    load();
   }
 }
 
@@ -303,22 +305,19 @@ __global__ __launch_bounds__(TB) void k_cocg_xr_def_a(int n, int G, int Gd, RedS
 template <typename C>
 __global__ __launch_bounds__(TB) void k_cocg_pz_b(int n, int G, int Gr, RedSite rs, const C* z,
                                                   C* p) {
-  double2 s0 = make_double2(0, 0), s1 = make_double2(0, 0);
-  for (int k = threadIdx.x; k < Gr; k += TB) {
-    const double2 t = rs.part[k];
-    s0.x += t.x;
-    s0.y += t.y;
-  }
+  const Range rr = block_rows(n, G);
+  int i = rr.start + threadIdx.x;
+  C pi, zi;
+  auto load = [&] {
+    if (i < rr.end) { pi = p[i]; zi = z[i]; }
+  };
+  load();   // while the partials arrive
+  double2 s0 = thread_parts<TB>(rs.part, Gr), s1;
   s0 = block_sum<TB>(s0);
   const bool pr = rs.paired;
   const double2 be = pr ? pdiv0(s0, scal2(rs.scal, S_RHO)) : cdiv0(s0, scal2(rs.scal, S_RHO));
   if (blockIdx.x == 0) {
-    for (int k = threadIdx.x; k < Gr; k += TB) {
-      const double2 t = rs.part[Gr + k];
-      s1.x += t.x;
-      s1.y += t.y;
-    }
-    s1 = block_sum<TB>(s1);
+    s1 = block_sum<TB>(thread_parts<TB>(rs.part + Gr, Gr));
     if (threadIdx.x == 0) {
       double* sc = rs.scal;
       sc[S_BETA] = be.x; sc[S_BETA + 1] = be.y;
@@ -330,11 +329,11 @@ __global__ __launch_bounds__(TB) void k_cocg_pz_b(int n, int G, int Gr, RedSite 
     }
   }
   const C b = from_d<C>(be);
-  Range rr = block_rows(n, G);
-  for (int i = rr.start + threadIdx.x; i < rr.end; i += TB) {
-    const C pi = p[i], zi = z[i];
+  while (i < rr.end) {
     const C bp = pr ? pmul(b, pi) : cmul(b, pi);
     p[i] = mk(zi.x + bp.x, zi.y + bp.y);
+    i += TB;
+    load();
   }
 }
 

@@ -306,22 +306,12 @@ constexpr bool patch_updates(int order, int cb, bool fp32) {
 // S_RHO, the previous rho, is read by all blocks).  Contains barriers.
 template <int NT, bool PR>
 __device__ __forceinline__ double2 next_beta(const RedSite& rb, int Gr) {
-  double2 s0 = make_double2(0, 0), s1 = make_double2(0, 0);
-  for (int k = threadIdx.x; k < Gr; k += NT) {
-    const double2 t = rb.part[k];
-    s0.x += t.x;
-    s0.y += t.y;
-  }
+  double2 s0 = thread_parts<NT>(rb.part, Gr);
   const double2 rho = scal2(rb.scal, S_RHO);
   s0 = block_sum<NT>(s0);
   const double2 be = PR ? pdiv0(s0, rho) : cdiv0(s0, rho);
   if (blockIdx.x == 0) {
-    for (int k = threadIdx.x; k < Gr; k += NT) {
-      const double2 t = rb.part[Gr + k];
-      s1.x += t.x;
-      s1.y += t.y;
-    }
-    s1 = block_sum<NT>(s1);
+    const double2 s1 = block_sum<NT>(thread_parts<NT>(rb.part + Gr, Gr));
     if (threadIdx.x == 0) {
       double* sc = rb.scal;
       sc[S_BETA] = be.x; sc[S_BETA + 1] = be.y;

@@ -513,6 +513,16 @@ __global__ __launch_bounds__(TB) void k_sw_xr_fold(int n, int G, int Gp,
   using C = typename C2<R>::T;
   const Rows rr = sw_rows(n, G);
   const int j = threadIdx.x % NB;
+  int64_t e = (int64_t)rr.start * NB + threadIdx.x;
+  const int64_t e1 = (int64_t)rr.end * NB;
+  int code = -1;
+  C qi, pi, xi, ri;
+  auto load = [&] {
+    if (e >= e1) return;
+    code = qcode[e / NB];
+    qi = q[e]; pi = p[e]; xi = x[e]; ri = r[e];
+  };
+  load();   // while the partials arrive
   const double2 s = sw_fold<NB>(dp, Gp), rho = scal2(sc + j * SW, SW_NEXT);
   const double2 al = act[j] ? cdiv0(rho, s) : make_double2(0, 0);
   if (blockIdx.x == 0 && threadIdx.x < NB) {
@@ -523,13 +533,8 @@ __global__ __launch_bounds__(TB) void k_sw_xr_fold(int n, int G, int Gp,
     o[SW_RHO + 1] = rho.y;
   }
   const C a = from_d<C>(al);
-  for (int64_t e = (int64_t)rr.start * NB + threadIdx.x; e < (int64_t)rr.end * NB; e += TB) {
-    const int i = (int)(e / NB);
-    const int code = qcode[i];
-    C qi;
-    if (code < 0) {
-      qi = q[e];
-    } else {
+  while (e < e1) {
+    if (code >= 0) {
       qi = mk(R(0), R(0));
       const int q0 = code >> 4, q1 = q0 + (code & 15);
       for (int t = q0; t < q1; ++t) {
@@ -537,14 +542,15 @@ __global__ __launch_bounds__(TB) void k_sw_xr_fold(int n, int G, int Gp,
         qi.x += v.x;
         qi.y += v.y;
       }
-      if (mask && mask[i]) qi = mk(R(0), R(0));
+      if (mask && mask[e / NB]) qi = mk(R(0), R(0));
     }
-    const C ap = cmul(a, p[e]), aq = cmul(a, qi);
-    C xi = x[e], ri = r[e];
+    const C ap = cmul(a, pi), aq = cmul(a, qi);
     xi.x += ap.x; xi.y += ap.y;
     ri.x -= aq.x; ri.y -= aq.y;
     x[e] = xi;
     r[e] = ri;
+    e += TB;
+    load();
   }
 }
 
@@ -560,6 +566,13 @@ __global__ __launch_bounds__(TB) void k_sw_pz_fold(int n, int G, int Gz,
   using C = typename C2<R>::T;
   const Rows rr = sw_rows(n, G);
   const int j = threadIdx.x % NB;
+  int64_t e = (int64_t)rr.start * NB + threadIdx.x;
+  const int64_t e1 = (int64_t)rr.end * NB;
+  C pi, zi;
+  auto load = [&] {
+    if (e < e1) { pi = p[e]; zi = z[e]; }
+  };
+  load();   // while the partials arrive
   const double2 s0 = sw_fold<NB>(dp, Gz);
   const bool on = act[j] != 0;
   const double2 be = on ? cdiv0(s0, scal2(sc + j * SW, SW_RHO)) : make_double2(0, 0);
@@ -577,9 +590,11 @@ __global__ __launch_bounds__(TB) void k_sw_pz_fold(int n, int G, int Gz,
     }
   }
   const C b = from_d<C>(be);
-  for (int64_t e = (int64_t)rr.start * NB + threadIdx.x; e < (int64_t)rr.end * NB; e += TB) {
-    const C bp = cmul(b, p[e]), zi = z[e];
+  while (e < e1) {
+    const C bp = cmul(b, pi);
     p[e] = mk(zi.x + bp.x, zi.y + bp.y);
+    e += TB;
+    load();
   }
 }
 
@@ -727,6 +742,10 @@ __device__ __forceinline__ void sw_vertex_rows(int64_t blk, int nv, int nE, R in
                                                typename C2<R>::T* __restrict__ w,
                                                typename C2<R>::T* __restrict__ u) {
   using C = typename C2<R>::T;
+  // edges and faces that a lane takes together (as in aux_vertex_rows): 20^3 order-2 boxes,
+  // groups of 2, iteration with one at a time / in batches 88.2 / 83.5 us FP32, 101 / 95.3
+  // FP64; order 1 31.9 / 30.9 and 33.9 / 32.7
+  constexpr int KE = LR >= 8 ? 2 : 4, KF = sizeof(R) == 4 ? 5 : 3;
   constexpr int L = NB * LR;
   const int lane = threadIdx.x % L;
   const int j = lane % NB, lr = lane / NB;
@@ -739,53 +758,92 @@ __device__ __forceinline__ void sw_vertex_rows(int64_t blk, int nv, int nE, R in
     R xv[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) xv[d] = xyz[3 * v + d];
-    for (int q = ve_ptr[v] + lr; q < ve_ptr[v + 1]; q += LR) {
-      const int ent = ve_ent[q];
-      const int e = ent >> 1;
-      const bool second = ent & 1;
-      C sr;
-      if constexpr (ORDER == 2) {
-        const C r0 = r[(int64_t)(2 * e) * NB + j], r1 = r[(int64_t)(2 * e + 1) * NB + j];
-        const R g0 = second ? R(1) : R(-5), g1 = second ? R(5) : R(-1);
-        g.x += g0 * r0.x + g1 * r1.x;
-        g.y += g0 * r0.y + g1 * r1.y;
-        const R l0 = second ? R(1.0 / 3.0) : R(2.0 / 3.0), l1 = R(1) - l0;
-        sr = mk(l0 * r0.x + l1 * r1.x, l0 * r0.y + l1 * r1.y);
-      } else {
-        const C r0 = r[(int64_t)e * NB + j];
-        g.x += second ? r0.x : -r0.x;
-        g.y += second ? r0.y : -r0.y;
-        sr = mk(R(0.5) * r0.x, R(0.5) * r0.y);
-      }
-      const int o = edges[2 * e + (second ? 0 : 1)];
+    const int e0 = ve_ptr[v], e1 = ve_ptr[v + 1];
+    for (int q0 = e0 + lr; q0 < e1; q0 += KE * LR) {
+      int ent[KE], o[KE];
+      C ra[KE], rb[KE];
+      R xo[KE][3];
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const R xo = xyz[3 * o + d];
-        const R t = second ? xv[d] - xo : xo - xv[d];
-        acc[d].x += t * sr.x;
-        acc[d].y += t * sr.y;
+      for (int k = 0; k < KE; ++k) ent[k] = ve_ent[min(q0 + k * LR, e1 - 1)];
+#pragma unroll
+      for (int k = 0; k < KE; ++k) {
+        const int64_t e = ent[k] >> 1;
+        o[k] = edges[2 * e + ((ent[k] & 1) ? 0 : 1)];
+        ra[k] = r[(ORDER == 2 ? 2 * e : e) * NB + j];
+        if constexpr (ORDER == 2) rb[k] = r[(2 * e + 1) * NB + j];
+      }
+#pragma unroll
+      for (int k = 0; k < KE; ++k)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) xo[k][d] = xyz[3 * o[k] + d];
+#pragma unroll
+      for (int k = 0; k < KE; ++k) {
+        if (q0 + k * LR >= e1) continue;
+        const bool second = ent[k] & 1;
+        C sr;
+        if constexpr (ORDER == 2) {
+          const C r0 = ra[k], r1 = rb[k];
+          const R g0 = second ? R(1) : R(-5), g1 = second ? R(5) : R(-1);
+          g.x += g0 * r0.x + g1 * r1.x;
+          g.y += g0 * r0.y + g1 * r1.y;
+          const R l0 = second ? R(1.0 / 3.0) : R(2.0 / 3.0), l1 = R(1) - l0;
+          sr = mk(l0 * r0.x + l1 * r1.x, l0 * r0.y + l1 * r1.y);
+        } else {
+          const C r0 = ra[k];
+          g.x += second ? r0.x : -r0.x;
+          g.y += second ? r0.y : -r0.y;
+          sr = mk(R(0.5) * r0.x, R(0.5) * r0.y);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const R t = second ? xv[d] - xo[k][d] : xo[k][d] - xv[d];
+          acc[d].x += t * sr.x;
+          acc[d].y += t * sr.y;
+        }
       }
     }
     if constexpr (ORDER == 2) {
-      for (int q = vf_ptr[v] + lr; q < vf_ptr[v + 1]; q += LR) {
-        const int ent = vf_ent[q];
-        const int f = ent >> 2, pos = ent & 3;
-        const C r0 = r[(int64_t)(2 * nE + 2 * f) * NB + j];
-        const C r1 = r[(int64_t)(2 * nE + 2 * f + 1) * NB + j];
-        if (pos == 0) { g.x -= r0.x + r1.x; g.y -= r0.y + r1.y; }
-        else if (pos == 1) { g.x += r0.x; g.y += r0.y; }
-        else { g.x += r1.x; g.y += r1.y; }
-        const int o1 = faces[3 * f + (pos == 0 ? 1 : 0)], o2 = faces[3 * f + (pos == 2 ? 1 : 2)];
+      const int f0 = vf_ptr[v], f1 = vf_ptr[v + 1];
+      for (int q0 = f0 + lr; q0 < f1; q0 += KF * LR) {
+        int fent[KF], o1[KF], o2[KF];
+        C ra[KF], rb[KF];
+        R y1[KF][3], y2[KF][3];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const R y1 = xyz[3 * o1 + d], y2 = xyz[3 * o2 + d];
-          const R xp = pos == 0 ? xv[d] : y1;
-          const R xq = pos == 0 ? y1 : (pos == 1 ? xv[d] : y2);
-          const R xr = pos == 2 ? xv[d] : y2;
-          const R t0 = (xq - xp) * R(1.0 / 3.0);
-          const R t1 = (xr - xp) * R(1.0 / 3.0);
-          acc[d].x += t0 * r0.x + t1 * r1.x;
-          acc[d].y += t0 * r0.y + t1 * r1.y;
+        for (int k = 0; k < KF; ++k) fent[k] = vf_ent[min(q0 + k * LR, f1 - 1)];
+#pragma unroll
+        for (int k = 0; k < KF; ++k) {
+          const int64_t f = fent[k] >> 2;
+          const int pos = fent[k] & 3;
+          o1[k] = faces[3 * f + (pos == 0 ? 1 : 0)];
+          o2[k] = faces[3 * f + (pos == 2 ? 1 : 2)];
+          ra[k] = r[(2 * nE + 2 * f) * NB + j];
+          rb[k] = r[(2 * nE + 2 * f + 1) * NB + j];
+        }
+#pragma unroll
+        for (int k = 0; k < KF; ++k)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            y1[k][d] = xyz[3 * o1[k] + d];
+            y2[k][d] = xyz[3 * o2[k] + d];
+          }
+#pragma unroll
+        for (int k = 0; k < KF; ++k) {
+          if (q0 + k * LR >= f1) continue;
+          const int pos = fent[k] & 3;
+          const C r0 = ra[k], r1 = rb[k];
+          if (pos == 0) { g.x -= r0.x + r1.x; g.y -= r0.y + r1.y; }
+          else if (pos == 1) { g.x += r0.x; g.y += r0.y; }
+          else { g.x += r1.x; g.y += r1.y; }
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            const R xp = pos == 0 ? xv[d] : y1[k][d];
+            const R xq = pos == 0 ? y1[k][d] : (pos == 1 ? xv[d] : y2[k][d]);
+            const R xr = pos == 2 ? xv[d] : y2[k][d];
+            const R t0 = (xq - xp) * R(1.0 / 3.0);
+            const R t1 = (xr - xp) * R(1.0 / 3.0);
+            acc[d].x += t0 * r0.x + t1 * r1.x;
+            acc[d].y += t0 * r0.y + t1 * r1.y;
+          }
         }
       }
     }
@@ -810,6 +868,7 @@ __device__ __forceinline__ void sw_edge_rows(int64_t blk, int nv, int nE, R inv_
                                              const typename C2<R>::T* __restrict__ winv,
                                              typename C2<R>::T* __restrict__ w) {
   using C = typename C2<R>::T;
+  constexpr int KF = 3;   // faces taken together
   constexpr int L = NB * LR;
   const int lane = threadIdx.x % L;
   const int j = lane % NB, lr = lane / NB;
@@ -820,14 +879,26 @@ __device__ __forceinline__ void sw_edge_rows(int64_t blk, int nv, int nE, R inv_
       const C r0 = r[(2 * e) * NB + j], r1 = r[(2 * e + 1) * NB + j];
       g = mk(R(4) * (r0.x - r1.x), R(4) * (r0.y - r1.y));
     }
-    for (int q = ef_ptr[e] + lr; q < ef_ptr[e + 1]; q += LR) {
-      const int ent = ef_ent[q];
-      const int f = ent >> 2, pos = ent & 3;
-      const C r0 = r[(int64_t)(2 * nE + 2 * f) * NB + j];
-      const C r1 = r[(int64_t)(2 * nE + 2 * f + 1) * NB + j];
-      if (pos == 0) { g.x -= R(4) * r1.x; g.y -= R(4) * r1.y; }
-      else if (pos == 1) { g.x -= R(4) * r0.x; g.y -= R(4) * r0.y; }
-      else { g.x += R(4) * (r0.x + r1.x); g.y += R(4) * (r0.y + r1.y); }
+    const int f0 = ef_ptr[e], f1 = ef_ptr[e + 1];
+    for (int q0 = f0 + lr; q0 < f1; q0 += KF * LR) {
+      int ent[KF];
+      C ra[KF], rb[KF];
+#pragma unroll
+      for (int k = 0; k < KF; ++k) ent[k] = ef_ent[min(q0 + k * LR, f1 - 1)];
+#pragma unroll
+      for (int k = 0; k < KF; ++k) {
+        const int64_t f = ent[k] >> 2;
+        ra[k] = r[(2 * nE + 2 * f) * NB + j];
+        rb[k] = r[(2 * nE + 2 * f + 1) * NB + j];
+      }
+#pragma unroll
+      for (int k = 0; k < KF; ++k) {
+        if (q0 + k * LR >= f1) continue;
+        const int pos = ent[k] & 3;
+        if (pos == 0) { g.x -= R(4) * rb[k].x; g.y -= R(4) * rb[k].y; }
+        else if (pos == 1) { g.x -= R(4) * ra[k].x; g.y -= R(4) * ra[k].y; }
+        else { g.x += R(4) * (ra[k].x + rb[k].x); g.y += R(4) * (ra[k].y + rb[k].y); }
+      }
     }
   }
   g = mk(group_sum<L, NB>(g.x), group_sum<L, NB>(g.y));
