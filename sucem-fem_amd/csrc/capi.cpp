@@ -92,6 +92,16 @@ std::shared_ptr<MemPool> new_pool() {
   return p;
 }
 
+size_t pools_unused(int device) {
+  PoolList& l = pool_list();
+  std::lock_guard<std::mutex> hold(l.mu);
+  size_t n = 0;
+  for (auto& w : l.all)
+    if (auto q = w.lock())
+      if (q->device == device) n += q->unused();
+  return n;
+}
+
 void* device_alloc(size_t bytes) {
   void* p = nullptr;
   if (hipMalloc(&p, bytes) == hipSuccess) return p;
@@ -151,6 +161,11 @@ void MemPool::trim() {
     unused_ = 0;
   }
   for (auto& e : old) (void)hipFree(e.second);   // waits for the work that may still use it
+}
+
+size_t MemPool::unused() {
+  std::lock_guard<std::mutex> hold(mu_);
+  return unused_;
 }
 
 void MemPool::close() {
@@ -216,6 +231,7 @@ int sucem_ctx_create(int device, void* hip_stream, sucem_ctx** out) {
   auto* h = new sucem_ctx();
   Context& c = h->c;
   c.device = device;
+  c.pool->device = device;
   try {
     SUCEM_HIP(hipSetDevice(device));
     hipDeviceProp_t prop;
@@ -284,7 +300,7 @@ int sucem_ctx_mem_info(sucem_ctx* ctx, int64_t* free_h, int64_t* total_h) {
   ctx->c.use();
   size_t fr = 0, tot = 0;
   SUCEM_HIP(hipMemGetInfo(&fr, &tot));
-  *free_h = (int64_t)fr;
+  *free_h = (int64_t)(fr + pools_unused(ctx->c.device));
   *total_h = (int64_t)tot;
   API_END
 }

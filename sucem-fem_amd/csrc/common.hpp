@@ -60,6 +60,8 @@ class MemPool {
   void put(void* p, size_t size);
   void trim();    // everything unused back to the device
   void close();   // trim, and keep nothing from now on
+  size_t unused();
+  int device = -1;   // of its context
 
  private:
   std::mutex mu_;
@@ -70,6 +72,8 @@ class MemPool {
 // The pool of the context that this thread's current entry point runs on (Context::use).
 std::shared_ptr<MemPool>& current_pool();
 std::shared_ptr<MemPool> new_pool();
+// unused bytes of all pools on a device: memory that an allocation there can have
+size_t pools_unused(int device);
 // hipMalloc; when it fails, once more after every pool has given its unused blocks back
 void* device_alloc(size_t bytes);
 

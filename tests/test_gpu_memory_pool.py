@@ -78,3 +78,30 @@ def test_threads_with_contexts_of_their_own():
     for a, g in zip(alone, got):
         for x in g:
             assert np.array_equal(x, a)
+
+
+def test_unused_blocks_count_as_free_memory():
+    """Dropped buffers that the pool keeps stay available to admission by free memory: what a
+    20^3 order-2 set-up (several hundred MB) leaves behind changes the reported free bytes by
+    less than 64 MB (allocation granularity), and releasing the pool adds no more than that."""
+    import gc
+    import torch
+    from sucemfem import _hip
+    from sucemfem.Utilities.Workloads import DeviceProblem
+    from sucemfem.runtime import Context
+    torch.cuda.set_device(0)
+    ctx = Context()
+    ctx.synchronize()
+    before = _free(ctx)
+    p = DeviceProblem((20, 20, 20), 0.6, 2, 7, (1.0, 2.2, 4.4), 0, ctx=ctx)
+    ctx.synchronize()
+    assert before - _free(ctx) > (128 << 20)
+    del p
+    gc.collect()
+    ws = ctypes.c_int64()
+    _hip.call("sucem_ctx_workspace_bytes", ctx.handle, ctypes.byref(ws))
+    after = _free(ctx) + ws.value        # the workspace is reported on its own
+    _hip.call("sucem_ctx_release_workspace", ctx.handle)
+    print("free bytes:", before, after, _free(ctx), ws.value, flush=True)
+    assert abs(_free(ctx) - after) < (64 << 20)
+    assert abs(before - after) < (64 << 20)
