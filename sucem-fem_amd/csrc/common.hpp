@@ -134,7 +134,7 @@ struct DBuf {
 // free, which synchronises the device) nothing after the first.  A slot is used by one
 // routine at a time: the Krylov solver takes slots [0, 32) and 84, the eigen solver [32, 48) (it
 // calls the Krylov solver, so their ranges differ), the batched solver [48, 80), the point entry
-// points [80, 84).  Calls on one context run one at a time (one host thread per context).
+// points [80, 84), operator products of several vectors 85.  Calls on one context run one at a time (one host thread per context).
 struct Workspace {
   std::vector<DBuf<unsigned char>> slot;
   // device memory of at least `bytes` bytes in slot k (nullptr for 0 bytes); the contents

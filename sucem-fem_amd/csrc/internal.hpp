@@ -147,7 +147,11 @@ struct System {
   bool pt_ready = false;
   DBuf<double> pt_coef64, pt_face64;
   DBuf<float> pt_coef32, pt_face32;
+  // Partial sums of the shared DOFs, for one vector.  A captured product holds this address, so
+  // it does not move: where another patch size needs more, the earlier (at most three) buffers
+  // stay with the system.
   DBuf<double2> pt_part;
+  std::vector<DBuf<double2>> pt_part_old;
 };
 
 // Generic complex CSR matrix (user-supplied, e.g. from scipy).

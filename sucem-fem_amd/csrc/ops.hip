@@ -675,11 +675,11 @@ void system_apply(Context* c, const System* sys, Coef k, bool eliminate_pec, int
     // several vectors to a launch: on small and middle meshes one vector leaves most of the
     // device idle (three vectors, 178,000 order-1 cells in FP64: 52.4 -> 36.7 us)
     for (int64_t v = 0; v < nvec;) {
-      const int nv = pt_vectors<R>(c, sys, f, nvec - v);
+      const PtVectors pv = pt_vectors<R>(c, sys, f, nvec - v);
       pt_apply<R>(c, sys, k, eliminate_pec ? s->pec.p : nullptr,
                   (const char*)x + v * s->ndofs * bytes, (char*)y + v * s->ndofs * bytes, nullptr,
-                  0, none, f, nv);
-      v += nv;
+                  0, none, f, pv.nvec, pv.part);
+      v += pv.nvec;
     }
     return;
   }

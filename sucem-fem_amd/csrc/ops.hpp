@@ -34,11 +34,18 @@ void mf_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const 
 bool pt_prepare(Context* c, System* sys, int cb);
 template <typename R>
 void pt_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const void* x, void* y,
-              const void* w, int epi, const RedSite& rs, const SpmvCfg& f, int nvec = 1);
-// how many of nvec vectors (ndofs apart) one pt_apply without an epilogue takes, its
-// partial-sum buffer made large enough: as many as fit 64 MB of partial sums
+              const void* w, int epi, const RedSite& rs, const SpmvCfg& f, int nvec = 1,
+              void* part = nullptr);
+// How many of nvec vectors (ndofs apart) one pt_apply without an epilogue takes, and where
+// their partial sums go: as many as fit 64 MB in the context's workspace; one, through the
+// system's own buffer (null), in a captured call (which must hold no address that a later
+// call frees, and allocates nothing) and where the memory cannot be had.
+struct PtVectors {
+  int nvec = 1;
+  void* part = nullptr;
+};
 template <typename R>
-int pt_vectors(Context* c, const System* sys, const SpmvCfg& f, int64_t nvec);
+PtVectors pt_vectors(Context* c, const System* sys, const SpmvCfg& f, int64_t nvec);
 // Patch operator for COCG with the shared DOFs' partial sums left unsummed: y holds the
 // rows of DOFs that lie in one patch, the partial sums stay in the system's buffer (rows
 // marked by pt_qcode), and the epilogue is x.y (FP64: the sum of the element quadratic

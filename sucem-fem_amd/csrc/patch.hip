@@ -37,6 +37,7 @@
 namespace sucem {
 namespace {
 
+constexpr int kWsPtVectors = 85;   // workspace slot: partial sums of several vectors
 constexpr int TB = 256;    // threads of the set-up kernels and of k_mf_psum
 int cb_slot(int cb) { return cb == 128 ? 0 : (cb == 192 ? 1 : (cb == 256 ? 2 : (cb == 64 ? 3 : -1))); }
 
@@ -908,7 +909,8 @@ void pt_validate(Context* c, const Space* s, const PatchMaps& pm, const std::vec
 template <typename R, int ORDER, int NFD, int CB>
 void launch_patch(Context* c, const System* sys, const PatchMaps& pm, Coef k,
                   const uint8_t* mask, const void* x, void* y, const void* w, int epi,
-                  const RedSite& rs, int Gp, int Gt, const PtUpdate* up = nullptr, int nvec = 1) {
+                  const RedSite& rs, int Gp, int Gt, void* part, const PtUpdate* up = nullptr,
+                  int nvec = 1) {
   using C = typename C2<R>::T;
   const Space* s = sys->space;
   const R* coef;
@@ -927,7 +929,7 @@ void launch_patch(Context* c, const System* sys, const PatchMaps& pm, Coef k,
   const RedSite rb = up ? up->rb : RedSite{};
 #define PT_ARGS pm.np, Gp, Gt, s->mesh->nc, s->nbf, pm.lds, coef, pm.lp.p, pm.uptr.p, pm.dof.p, \
                 pm.seg.p, pm.out.p, pm.fptr.p, s->pt_fmeta.p, pm.fpos.p, hf, s->ref_face_dofs.p, \
-                s->ref_face.p, (R)k.s, (R)k.t, c0, mask, (const C*)x, (C*)y, (C*)sys->pt_part.p, \
+                s->ref_face.p, (R)k.s, (R)k.t, c0, mask, (const C*)x, (C*)y, (C*)part, \
                 (const C*)w, rs, z, pnew, Gr, rb, s->ndofs, pm.npe
   if (up) {
     SUCEM_CHECK((epi == 3 || epi == 4) && patch_updates(ORDER, CB, sizeof(R) == 4),
@@ -978,7 +980,7 @@ bool pt_prepare(Context* c, System* sys, int cb) {
     sys->pt_ready = true;
   }
   if ((int64_t)sys->pt_part.n < std::max<int64_t>(s->pt[slot].npe, 1)) {
-    sys->pt_part.release_synced();
+    if (sys->pt_part.p) sys->pt_part_old.push_back(std::move(sys->pt_part));
     sys->pt_part.alloc(std::max<int64_t>(s->pt[slot].npe, 1));
   }
   return true;
@@ -1029,7 +1031,8 @@ SpmvCfg pt_cfg(const Space* s, int cb, int G) {
 
 template <typename R>
 void pt_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const void* x, void* y,
-              const void* w, int epi, const RedSite& rs, const SpmvCfg& f, int nvec) {
+              const void* w, int epi, const RedSite& rs, const SpmvCfg& f, int nvec,
+              void* part) {
   using C = typename C2<R>::T;
   const Space* s = sys->space;
   const int slot = cb_slot(f.U);
@@ -1045,20 +1048,22 @@ void pt_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const 
               "the patch operator needs more LDS per workgroup than the device has");
   SUCEM_CHECK(nvec == 1 || (epi == 0 && nvec > 0 && nvec <= 65535), SUCEM_ERR_INTERNAL,
               "several vectors without an epilogue only");
-  SUCEM_CHECK((int64_t)sys->pt_part.n * (int64_t)sizeof(double2) >=
-                  nvec * pm.npe * (int64_t)sizeof(C),
-              SUCEM_ERR_INVALID, "patch operator not prepared");
+  if (!part) {
+    SUCEM_CHECK(nvec == 1 && (int64_t)sys->pt_part.n >= pm.npe, SUCEM_ERR_INVALID,
+                "patch operator not prepared");
+    part = sys->pt_part.p;
+  }
   if (s->order == 2) {
-    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
-    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
-    else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
-    else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
+    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, part, nullptr, nvec);
+    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, part, nullptr, nvec);
+    else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, part, nullptr, nvec);
+    else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, part, nullptr, nvec);
   } else {
     SUCEM_CHECK(f.U == 256, SUCEM_ERR_UNSUPPORTED, "order-1 patches hold 256 cells");
-    launch_patch<R, 1, 3, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, nullptr, nvec);
+    launch_patch<R, 1, 3, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gt, part, nullptr, nvec);
   }
   const int npd = (int)pm.npd;
-#define PS_ARGS npd, Gg, Gt, Gp, pm.qptr.p, pm.qdof.p, (const C*)sys->pt_part.p, mask, (C*)y, \
+#define PS_ARGS npd, Gg, Gt, Gp, pm.qptr.p, pm.qdof.p, (const C*)part, mask, (C*)y, \
                 (const C*)w, rs, s->ndofs, pm.npe
   if (epi == 0) SUCEM_LAUNCH((k_mf_psum<R, 0>), dim3(Gg, nvec), TB, 0, c->stream, PS_ARGS);
   else if (epi == 1) SUCEM_LAUNCH((k_mf_psum<R, 1>), Gg, TB, 0, c->stream, PS_ARGS);
@@ -1066,7 +1071,7 @@ void pt_apply(Context* c, const System* sys, Coef k, const uint8_t* mask, const 
 #undef PS_ARGS
 }
 template void pt_apply<float>(Context*, const System*, Coef, const uint8_t*, const void*, void*,
-                              const void*, int, const RedSite&, const SpmvCfg&, int);
+                              const void*, int, const RedSite&, const SpmvCfg&, int, void*);
 
 int pt_deferred_parts(const System* sys, const SpmvCfg& f) {
   if (f.mf != 2 || !sys->pt_ready) return 0;
@@ -1088,12 +1093,12 @@ void pt_apply_deferred(Context* c, const System* sys, Coef k, const uint8_t* mas
   const PatchMaps& pm = sys->space->pt[cb_slot(f.U)];
   const int epi = rs.paired ? 4 : 3;
   if (sys->space->order == 2) {
-    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
-    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
-    else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
-    else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
+    if (f.U == 64) launch_patch<R, 2, 8, 64>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, sys->pt_part.p, up);
+    else if (f.U == 128) launch_patch<R, 2, 8, 128>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, sys->pt_part.p, up);
+    else if (f.U == 192) launch_patch<R, 2, 8, 192>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, sys->pt_part.p, up);
+    else launch_patch<R, 2, 8, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, sys->pt_part.p, up);
   } else {
-    launch_patch<R, 1, 3, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, up);
+    launch_patch<R, 1, 3, 256>(c, sys, pm, k, mask, x, y, w, epi, rs, Gp, Gp, sys->pt_part.p, up);
   }
 }
 template void pt_apply_deferred<float>(Context*, const System*, Coef, const uint8_t*,
@@ -1115,27 +1120,35 @@ const int32_t* pt_qcode(const System* sys, const SpmvCfg& f) {
 }
 const void* pt_partials(const System* sys) { return sys->pt_part.p; }
 template void pt_apply<double>(Context*, const System*, Coef, const uint8_t*, const void*, void*,
-                               const void*, int, const RedSite&, const SpmvCfg&, int);
+                               const void*, int, const RedSite&, const SpmvCfg&, int, void*);
 
 template <typename R>
-int pt_vectors(Context* c, const System* sys, const SpmvCfg& f, int64_t nvec) {
+PtVectors pt_vectors(Context* c, const System* sys, const SpmvCfg& f, int64_t nvec) {
   const PatchMaps& pm = pt_maps(sys->space, f.U);
   const int64_t one = std::max<int64_t>(pm.npe, 1) * (int64_t)sizeof(typename C2<R>::T);
-  const int64_t have = (int64_t)sys->pt_part.n * (int64_t)sizeof(double2);
-  // a captured call allocates nothing: it takes what fits the buffer as it is
+  PtVectors v;
+  const int64_t fit = std::min<int64_t>({nvec, (int64_t(64) << 20) / one, 64});
+  if (fit < 2) return v;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess) (void)hipGetLastError();
-  const bool grow = cap == hipStreamCaptureStatusNone;
-  const int64_t fit = (grow ? std::max(have, int64_t(64) << 20) : have) / one;
-  const int nv = (int)std::max<int64_t>(1, std::min<int64_t>({nvec, fit, 64}));
-  if (nv * one > have) {
-    System* ms = const_cast<System*>(sys);
-    ms->pt_part.release_synced();
-    ms->pt_part.alloc((size_t)((nv * one + 15) / 16));
+  if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return v;
   }
-  return nv;
+  if (cap != hipStreamCaptureStatusNone) return v;
+  // (a capture of another stream does not forbid this call: its products go to no graph)
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  try {
+    v.part = c->ws.get(kWsPtVectors, (size_t)(fit * one));
+    v.nvec = (int)fit;
+  } catch (const Error&) {   // one by one then, as without the memory
+    (void)hipGetLastError();
+  }
+  if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  else (void)hipGetLastError();
+  return v;
 }
-template int pt_vectors<float>(Context*, const System*, const SpmvCfg&, int64_t);
-template int pt_vectors<double>(Context*, const System*, const SpmvCfg&, int64_t);
+template PtVectors pt_vectors<float>(Context*, const System*, const SpmvCfg&, int64_t);
+template PtVectors pt_vectors<double>(Context*, const System*, const SpmvCfg&, int64_t);
 
 }  // namespace sucem
