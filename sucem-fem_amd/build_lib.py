@@ -17,7 +17,7 @@ OUT_DIR = os.path.join(HERE, "sucemfem", "_native")
 OBJ_DIR = os.path.join(HERE, "_build")
 LIB = os.path.join(OUT_DIR, "libsucem_hip.so")
 
-SOURCES = ["refdata.cpp", "capi.cpp", "mesh_space.hip", "assemble.hip", "ops.hip", "krylov.hip", "eigen.hip",
+SOURCES = ["refdata.cpp", "mempool.cpp", "capi.cpp", "mesh_space.hip", "assemble.hip", "ops.hip", "krylov.hip", "eigen.hip",
            "hiptmair.hip", "batch.hip", "postproc.hip", "matfree.hip", "patch.hip", "sweep.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

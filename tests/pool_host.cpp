@@ -1,0 +1,162 @@
+// The device memory pools (csrc/mempool.cpp) over a counted stand-in for the device: one named
+// check per run, exit code 0 when it holds.  Built and run by tests/test_pool_host.py.
+#include <cstdlib>
+#include <map>
+#include <set>
+
+#include "mempool.cpp"
+
+namespace {
+
+struct Device {
+  size_t capacity = size_t(64) << 30, used = 0, next = 4096;
+  std::map<size_t, size_t> blocks;   // address -> bytes
+  int mallocs = 0, frees = 0;
+  hipError_t last = hipSuccess;
+} dev;
+
+hipError_t fail(hipError_t e) { return dev.last = e; }
+
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t bytes) {
+  if (dev.used + bytes > dev.capacity) return fail(hipErrorOutOfMemory);
+  ++dev.mallocs;
+  *p = (void*)dev.next;
+  dev.blocks[dev.next] = bytes;
+  dev.next += bytes + 4096;
+  dev.used += bytes;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  auto it = dev.blocks.find((size_t)p);
+  if (it == dev.blocks.end()) std::abort();   // freed twice, or never allocated
+  ++dev.frees;
+  dev.used -= it->second;
+  dev.blocks.erase(it);
+  return hipSuccess;
+}
+hipError_t hipGetLastError(void) {
+  const hipError_t e = dev.last;
+  dev.last = hipSuccess;
+  return e;
+}
+hipError_t hipMemGetInfo(size_t* f, size_t* t) {
+  *f = dev.capacity - dev.used;
+  *t = dev.capacity;
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "stand-in error"; }
+}
+
+using namespace sucem;
+
+namespace {
+
+constexpr size_t MB = size_t(1) << 20, GB = size_t(1) << 30;
+
+struct Fixture {
+  std::shared_ptr<MemPool> pool = new_pool();
+  Fixture() {
+    pool->device = 0;
+    current_pool() = pool;
+  }
+};
+
+#define CHECK(cond)                                               \
+  do {                                                            \
+    if (!(cond)) {                                                \
+      std::printf("line %d: %s is false\n", __LINE__, #cond);     \
+      return 1;                                                   \
+    }                                                             \
+  } while (0)
+
+// blocks come back from the pool, and only to a request of about their size
+int reuse() {
+  Fixture f;
+  void* p;
+  {
+    DBuf<char> a(10 * MB);
+    p = a.p;
+  }
+  CHECK(f.pool->unused() >= 10 * MB && dev.frees == 0);
+  {
+    DBuf<char> a(10 * MB);
+    CHECK(a.p == p && dev.mallocs == 1 && f.pool->unused() == 0);
+    DBuf<char> b(8 * MB);
+    CHECK(dev.mallocs == 2);
+  }
+  DBuf<char> c(5 * MB);   // neither 10 nor 8 MB for 5
+  CHECK(dev.mallocs == 3);
+  return 0;
+}
+
+// at most kMax bytes stay in a pool, beyond that blocks go back to the device
+int cap() {
+  Fixture f;
+  {
+    std::vector<DBuf<char>> a;
+    for (int i = 0; i < 12; ++i) a.emplace_back(512 * MB);
+    CHECK(dev.used >= 6 * GB);
+  }
+  CHECK(f.pool->unused() <= MemPool::kMax && f.pool->unused() > MemPool::kMax - 640 * MB);
+  CHECK(dev.used == f.pool->unused());
+  {
+    DBuf<char> big(MemPool::kMax + 1);
+  }
+  CHECK(dev.used == f.pool->unused() && f.pool->unused() <= MemPool::kMax);
+  return 0;
+}
+
+// trim and close give everything back; a closed pool keeps nothing
+int trim() {
+  Fixture f;
+  {
+    DBuf<char> a(MB), b(3 * MB);
+  }
+  CHECK(f.pool->unused() > 0);
+  f.pool->trim();
+  CHECK(f.pool->unused() == 0 && dev.used == 0);
+  DBuf<char> late(2 * MB);
+  f.pool->close();
+  late.release();
+  CHECK(dev.used == 0 && f.pool->unused() == 0);
+  return 0;
+}
+
+// a failed allocation empties every pool of the process and is tried again
+int full_device() {
+  Fixture f;
+  auto other = new_pool();
+  other->device = 0;
+  {
+    DBuf<char> a(2 * GB);
+    current_pool() = other;
+    DBuf<char> b(GB);
+  }
+  CHECK(f.pool->unused() + other->unused() >= 3 * GB);
+  dev.capacity = 6 * GB;
+  current_pool() = f.pool;
+  DBuf<char> big(5 * GB);
+  CHECK(f.pool->unused() == 0 && other->unused() == 0 && dev.last == hipSuccess);
+  bool thrown = false;
+  try {
+    DBuf<char> more(5 * GB);
+  } catch (const Error& e) {
+    thrown = e.code == SUCEM_ERR_OOM;
+  }
+  CHECK(thrown);
+  return 0;
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::map<std::string, int (*)()> checks = {
+      {"reuse", reuse}, {"cap", cap}, {"trim", trim}, {"full_device", full_device}};
+  auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
+  if (it == checks.end()) return 2;
+  return it->second();
+}

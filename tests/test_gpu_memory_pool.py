@@ -29,6 +29,19 @@ def _solve(ctx, n, order, seed):
     return x.cpu().numpy()
 
 
+def _raw():
+    """Free device memory as the device reports it: idle blocks of a pool are not in it."""
+    import gc
+    import torch
+    gc.collect()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    return torch.cuda.mem_get_info()[0]
+
+
+SLACK = 64 << 20     # granularity of the device's allocations
+
+
 def test_repeated_meshes_do_not_grow_and_release_gives_back():
     import torch
     from sucemfem import _hip
@@ -36,16 +49,59 @@ def test_repeated_meshes_do_not_grow_and_release_gives_back():
     torch.cuda.set_device(0)
     ctx = Context()
     ref = _solve(ctx, (9, 8, 7), 2, 0)
-    after = _free(ctx)
-    for n, order, seed in (((9, 8, 7), 2, 0), ((8, 8, 8), 2, 1), ((12, 9, 10), 1, 2)) * 4:
-        x = _solve(ctx, n, order, seed)
-        if (n, order, seed) == ((9, 8, 7), 2, 0):
-            assert np.array_equal(x, ref)       # reused memory changes nothing
-    # a second and third size add at most their own buffers, not one set per repetition
-    assert after - _free(ctx) < (1 << 30)
-    held = _free(ctx)
+    sizes = ((9, 8, 7), 2, 0), ((8, 8, 8), 2, 1), ((12, 9, 10), 1, 2)
+    start = None
+    for k in range(5):
+        for n, order, seed in sizes:
+            x = _solve(ctx, n, order, seed)
+            if (n, order, seed) == ((9, 8, 7), 2, 0):
+                assert np.array_equal(x, ref)       # reused memory changes nothing
+        if k == 0:
+            start = _raw()
+    # once every size has been seen, repetitions take nothing more
+    assert start - _raw() <= SLACK
+    ws = ctypes.c_int64()
+    _hip.call("sucem_ctx_workspace_bytes", ctx.handle, ctypes.byref(ws))
+    held = _raw()
     _hip.call("sucem_ctx_release_workspace", ctx.handle)
-    assert _free(ctx) > held
+    assert _raw() - held >= ws.value
+    _hip.call("sucem_ctx_workspace_bytes", ctx.handle, ctypes.byref(ws))
+    assert ws.value == 0
+
+
+def test_idle_blocks_are_bounded_and_go_back():
+    """What a 20^3 order-2 problem leaves in the pool (several hundred MB, at most 4 GB), in
+    free memory as the device reports it: no more after repetitions, nothing after the release
+    and nothing after the context."""
+    import torch
+    from sucemfem import _hip
+    from sucemfem.Utilities.Workloads import DeviceProblem
+    from sucemfem.runtime import Context
+    torch.cuda.set_device(0)
+
+    def build(ctx):
+        p = DeviceProblem((20, 20, 20), 0.6, 2, 7, (1.0, 2.2, 4.4), 0, ctx=ctx)
+        ctx.synchronize()
+        del p
+
+    ctx = Context()
+    build(ctx)                                    # code and tables of the library
+    _hip.call("sucem_ctx_release_workspace", ctx.handle)
+    before = _raw()
+    build(ctx)
+    ws = ctypes.c_int64()
+    _hip.call("sucem_ctx_workspace_bytes", ctx.handle, ctypes.byref(ws))
+    idle = before - _raw() - ws.value
+    assert (128 << 20) < idle <= (4 << 30) + SLACK
+    for _ in range(3):
+        build(ctx)
+    assert before - _raw() - ws.value <= idle + SLACK
+    _hip.call("sucem_ctx_release_workspace", ctx.handle)
+    assert abs(before - _raw()) <= SLACK
+    build(ctx)
+    assert before - _raw() > (128 << 20)
+    del ctx
+    assert before - _raw() <= SLACK
 
 
 def test_threads_with_contexts_of_their_own():
