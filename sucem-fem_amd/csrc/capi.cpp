@@ -318,7 +318,7 @@ int sucem_mesh_destroy(sucem_mesh* m) {
   API_BEGIN
   if (!m) return SUCEM_OK;
   (void)hipSetDevice(m->m.ctx->device);
-  (void)hipDeviceSynchronize();   // other contexts' streams may still read it
+  const DeviceWait wait;   // other contexts' streams may still read it
   delete m;
   API_END
 }
@@ -405,7 +405,7 @@ int sucem_space_destroy(sucem_space* s) {
   API_BEGIN
   if (!s) return SUCEM_OK;
   (void)hipSetDevice(s->s.ctx->device);
-  (void)hipDeviceSynchronize();   // other contexts' streams may still read it
+  const DeviceWait wait;   // other contexts' streams may still read it
   delete s;
   API_END
 }
@@ -473,7 +473,7 @@ int sucem_system_destroy(sucem_system* sys) {
   API_BEGIN
   if (!sys) return SUCEM_OK;
   (void)hipSetDevice(sys->s.ctx->device);
-  (void)hipDeviceSynchronize();   // other contexts' streams may still read it
+  const DeviceWait wait;   // other contexts' streams may still read it
   delete sys;
   API_END
 }
@@ -999,7 +999,7 @@ int sucem_csr_destroy(sucem_csr* A) {
   API_BEGIN
   if (!A) return SUCEM_OK;
   (void)hipSetDevice(A->a.ctx->device);
-  (void)hipDeviceSynchronize();   // other contexts' streams may still read it
+  const DeviceWait wait;   // other contexts' streams may still read it
   delete A;
   API_END
 }

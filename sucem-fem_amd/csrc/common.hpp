@@ -46,9 +46,9 @@ void set_last_error(const std::string& msg);
 //
 // A block that is put back may still be in use by work queued on its context's stream, so it
 // is only handed out to that context (whose stream orders the new use behind the old one).
-// Whoever frees memory that other streams may use waits for the device first, as hipFree
-// does: the destroy entry points, and members replaced while their owner lives (see
-// DBuf::release_synced).  At most kMax bytes stay unused in one pool; blocks go back to the
+// Whoever frees memory that other streams may use has the device waited for first, as hipFree
+// does: the destroy entry points (DeviceWait) and members replaced while their owner lives
+// (DBuf::release_synced).  At most kMax bytes stay unused in one pool; blocks go back to the
 // device beyond that, when the context's workspace is released, when an allocation fails
 // (all pools give way), and with the context (buffers that outlive it free directly).
 class MemPool {
@@ -76,6 +76,24 @@ std::shared_ptr<MemPool> new_pool();
 size_t pools_unused(int device);
 // hipMalloc; when it fails, once more after every pool has given its unused blocks back
 void* device_alloc(size_t bytes);
+// hipFree (which waits for all work on the device); a refusal leaves no error behind for the
+// thread's next launch to report
+bool device_free(void* p);
+
+// Waits until the device's queued work is done, before buffers that any stream may use go back
+// to their pools.  Through hipFree of a small block (1.2 us on an idle device): a
+// hipDeviceSynchronize ends every stream capture of the process, that of another thread's
+// batched sweep among them.  Where even that is refused, the buffers that this thread releases
+// while the object lives go to the device instead, which orders them itself.
+class DeviceWait {
+ public:
+  DeviceWait();
+  ~DeviceWait() { bypass_pools() = before_; }
+  static bool& bypass_pools();   // of this thread
+
+ private:
+  bool before_;
+};
 
 // Owning device allocation.
 template <typename T>
@@ -114,16 +132,17 @@ struct DBuf {
   }
   void release() {
     if (p) {
-      if (pool) pool->put(p, size);
-      else (void)hipFree(p);
+      if (pool && !DeviceWait::bypass_pools()) pool->put(p, size);
+      else (void)device_free(p);
     }
     p = nullptr;
     n = size = 0;
     pool.reset();
   }
-  // release of memory that work on another context's stream may still use
+  // release of memory that work on another context's stream may still use: to the device,
+  // which waits for it
   void release_synced() {
-    if (p && pool) (void)hipDeviceSynchronize();
+    pool.reset();
     release();
   }
   size_t bytes() const { return n * sizeof(T); }

@@ -70,6 +70,23 @@ void* device_alloc(size_t bytes) {
   return p;
 }
 
+bool device_free(void* p) {
+  if (hipFree(p) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+DeviceWait::DeviceWait() : before_(bypass_pools()) {
+  void* p = nullptr;
+  if (hipMalloc(&p, 256) != hipSuccess) (void)hipGetLastError();
+  if (!p || !device_free(p)) bypass_pools() = true;
+}
+
+bool& DeviceWait::bypass_pools() {
+  static thread_local bool b = false;
+  return b;
+}
+
 MemPool::~MemPool() { trim(); }
 
 void* MemPool::take(size_t bytes, size_t& got) {
@@ -102,7 +119,7 @@ void MemPool::put(void* p, size_t size) {
       }
     }
   }
-  (void)hipFree(p);
+  (void)device_free(p);
 }
 
 void MemPool::trim() {
@@ -112,7 +129,7 @@ void MemPool::trim() {
     old.swap(free_);
     unused_ = 0;
   }
-  for (auto& e : old) (void)hipFree(e.second);   // waits for the work that may still use it
+  for (auto& e : old) (void)device_free(e.second);   // waits for the work that may still use it
 }
 
 size_t MemPool::unused() {

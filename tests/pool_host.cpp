@@ -12,6 +12,7 @@ struct Device {
   size_t capacity = size_t(64) << 30, used = 0, next = 4096;
   std::map<size_t, size_t> blocks;   // address -> bytes
   int mallocs = 0, frees = 0;
+  bool refuse = false;   // as under another stream's global capture
   hipError_t last = hipSuccess;
 } dev;
 
@@ -21,6 +22,7 @@ hipError_t fail(hipError_t e) { return dev.last = e; }
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t bytes) {
+  if (dev.refuse) return fail(hipErrorStreamCaptureUnsupported);
   if (dev.used + bytes > dev.capacity) return fail(hipErrorOutOfMemory);
   ++dev.mallocs;
   *p = (void*)dev.next;
@@ -30,6 +32,7 @@ hipError_t hipMalloc(void** p, size_t bytes) {
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {
+  if (dev.refuse) return fail(hipErrorStreamCaptureUnsupported);
   auto it = dev.blocks.find((size_t)p);
   if (it == dev.blocks.end()) std::abort();   // freed twice, or never allocated
   ++dev.frees;
@@ -47,7 +50,8 @@ hipError_t hipMemGetInfo(size_t* f, size_t* t) {
   *t = dev.capacity;
   return hipSuccess;
 }
-hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+// ends every capture of the process: nothing here may call it
+hipError_t hipDeviceSynchronize(void) { std::abort(); }
 const char* hipGetErrorString(hipError_t) { return "stand-in error"; }
 }
 
@@ -151,11 +155,46 @@ int full_device() {
   return 0;
 }
 
+// blocks are pooled after a wait for the device; where the wait is refused they never reach a
+// pool, and no error is left for the next launch
+int wait() {
+  Fixture f;
+  DBuf<char> a(MB), b(MB), c(MB);
+  {
+    const int frees = dev.frees;
+    const DeviceWait w;
+    CHECK(dev.frees == frees + 1);   // hipFree waits
+    a.release();
+  }
+  CHECK(f.pool->unused() >= MB);
+  const size_t idle = f.pool->unused();
+  {
+    dev.refuse = true;
+    const DeviceWait w;
+    b.release();
+  }
+  CHECK(f.pool->unused() == idle && dev.last == hipSuccess);
+  dev.refuse = false;
+  {
+    const DeviceWait w;
+  }
+  {
+    const int frees = dev.frees;
+    c.release_synced();
+    CHECK(dev.frees == frees + 1 && f.pool->unused() == idle && !c.p);
+  }
+  DBuf<char> d(2 * MB);
+  d.release();   // the refusal is over
+  CHECK(f.pool->unused() > idle);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, int (*)()> checks = {
-      {"reuse", reuse}, {"cap", cap}, {"trim", trim}, {"full_device", full_device}};
+      {"reuse", reuse}, {"cap", cap}, {"trim", trim}, {"full_device", full_device},
+      {"wait", wait}};
   auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   return it->second();

@@ -161,3 +161,94 @@ def test_unused_blocks_count_as_free_memory():
     print("free bytes:", before, after, _free(ctx), ws.value, flush=True)
     assert abs(_free(ctx) - after) < (64 << 20)
     assert abs(before - after) < (64 << 20)
+
+
+def test_objects_dropped_by_another_thread_during_a_capture():
+    """A thread that drops a mesh, its space and its system leaves a capture of another thread
+    alone (the batched sweep captures its iterations), and the next launch reports nothing."""
+    import torch
+    from sucemfem.Utilities.Workloads import DeviceProblem
+    from sucemfem.runtime import Context
+    torch.cuda.set_device(0)
+    errs = []
+
+    def drop():
+        try:
+            torch.cuda.set_device(0)
+            s = torch.cuda.Stream()
+            with torch.cuda.stream(s):
+                ctx = Context(stream=s)
+                for _ in range(2):
+                    p = DeviceProblem((3, 4, 2), 0.1, 2, 7, (1.0, 2.2, 4.4), 0, ctx=ctx)
+                    x = torch.ones(p.ndofs, dtype=torch.complex128, device="cuda")
+                    y = torch.zeros_like(x)
+                    del p
+                    p = DeviceProblem((2, 2, 2), 0.1, 1, 7, (1.0, 2.2, 4.4), 0, ctx=ctx)
+                    p.apply(3.0, x[:p.ndofs], y[:p.ndofs], precision=64)
+                    del p
+        except Exception as e:  # noqa: BLE001 - reported below
+            errs.append(e)
+
+    w = torch.ones(16, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream(), capture_error_mode="relaxed"):
+        t = threading.Thread(target=drop)
+        t.start()
+        t.join()
+        w.add_(1.0)
+    g.replay()
+    torch.cuda.synchronize()
+    assert not errs, errs
+    assert torch.all(w == 2.0)
+
+
+def test_sweeps_beside_a_thread_that_drops_problems():
+    """Batched sweeps (whose iterations are captured) on one thread while another one builds
+    and drops problems: the sweeps' solutions are those of a sweep alone."""
+    import torch
+    from sucemfem.Utilities.Workloads import DeviceProblem
+    from sucemfem.runtime import Context
+    torch.cuda.set_device(0)
+    k0s = np.linspace(0.5, 12.0, 4)
+
+    def problem(ctx, n, order):
+        return DeviceProblem(n, np.array(n) * 0.03, order, 7, (1.0, 2.2, 4.4), 3, ctx=ctx)
+
+    s1 = torch.cuda.Stream()
+    with torch.cuda.stream(s1):
+        p = problem(Context(stream=s1), (6, 5, 4), 1)
+        g = torch.Generator(device="cuda")
+        g.manual_seed(0)
+        B = torch.randn(4, p.ndofs, dtype=torch.complex128, device="cuda", generator=g)
+        ref, X = torch.zeros_like(B), torch.zeros_like(B)
+        p.solve_sweep(k0s, B, ref, precision=64, tol=1e-10, width=2, use_graph=True)
+    s1.synchronize()
+    stop, errs = threading.Event(), []
+
+    def churn():
+        try:
+            torch.cuda.set_device(0)
+            s2 = torch.cuda.Stream()
+            with torch.cuda.stream(s2):
+                ctx = Context(stream=s2)
+                while not stop.is_set():
+                    q = problem(ctx, (3, 4, 2), 2)
+                    del q
+        except Exception as e:  # noqa: BLE001 - reported below
+            errs.append(e)
+
+    t = threading.Thread(target=churn)
+    t.start()
+    try:
+        with torch.cuda.stream(s1):
+            for _ in range(20):
+                X.zero_()
+                st = p.solve_sweep(k0s, B, X, precision=64, tol=1e-10, width=2, use_graph=True)
+                s1.synchronize()
+                assert all(q["status"] == 0 for q in st)
+                assert torch.equal(X, ref)
+    finally:
+        stop.set()
+        t.join()
+    assert not errs, errs
