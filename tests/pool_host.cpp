@@ -155,6 +155,39 @@ int full_device() {
   return 0;
 }
 
+// what a buffer takes from the device: at most an eighth more than its size (512 bytes for the
+// smallest), the size itself beyond what a pool can keep, also when a kept block is handed out
+int rounding() {
+  Fixture f;
+  for (size_t n : {size_t(1), size_t(511), size_t(4096), size_t(4097), size_t(8191), size_t(8193),
+                   size_t(1000003), 16 * MB + 1, 3 * GB + 12345, MemPool::kMax}) {
+    const size_t used = dev.used;
+    DBuf<char> a(n);
+    const size_t took = dev.used - used;
+    CHECK(took >= n && took - n <= std::max(n / 8, size_t(511)));
+    a.release();
+    f.pool->trim();
+  }
+  {
+    const size_t used = dev.used;
+    DBuf<char> a(MemPool::kMax + 1);
+    CHECK(dev.used - used == MemPool::kMax + 1);
+  }
+  for (size_t n = 100; n < 64 * MB; n = n * 5 / 4 + 1) {   // blocks of every class, kept
+    DBuf<char> a(n);
+  }
+  for (size_t n = 4096; n < 40 * MB; n = n * 9 / 8 + 7) {
+    DBuf<char> a(n);
+    CHECK(a.size >= n && a.size - n <= n / 8);
+  }
+  f.pool->trim();
+  // a request for what is left gets it although its rounded size does not fit
+  dev.capacity = dev.used + 9 * MB + 4;
+  DBuf<char> exact(9 * MB + 4);
+  CHECK(exact.p && exact.size == 9 * MB + 4 && dev.last == hipSuccess);
+  return 0;
+}
+
 // blocks are pooled after a wait for the device; where the wait is refused they never reach a
 // pool, and no error is left for the next launch
 int wait() {
@@ -194,7 +227,7 @@ int wait() {
 int main(int argc, char** argv) {
   const std::map<std::string, int (*)()> checks = {
       {"reuse", reuse}, {"cap", cap}, {"trim", trim}, {"full_device", full_device},
-      {"wait", wait}};
+      {"wait", wait}, {"rounding", rounding}};
   auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   return it->second();

@@ -252,3 +252,27 @@ def test_sweeps_beside_a_thread_that_drops_problems():
         stop.set()
         t.join()
     assert not errs, errs
+
+
+@pytest.mark.parametrize("mb,extra", [(9, 4), (1000, 12345)])
+def test_what_a_buffer_takes_from_the_device(mb, extra):
+    """An allocation takes at most an eighth more than its size from the device (whose own
+    granularity, 2 MB, comes on top)."""
+    import torch
+    from sucemfem import _hip
+    from sucemfem.runtime import Context
+    torch.cuda.set_device(0)
+    ctx = Context()
+    # a matrix of nnz values keeps nnz (4 + 16 + 8) bytes and 8 (n + 1) of row pointers and
+    # diagonals: one row holds them all
+    nnz = ((mb << 20) + extra) // 16
+    ptr = np.array([0, nnz], np.int64)
+    col = np.zeros(nnz, np.int32)
+    val = np.ones(nnz, np.complex128)
+    h = _hip.out_handle()
+    before = _raw()
+    _hip.call("sucem_csr_create", ctx.handle, 1, nnz, _hip.ptr(ptr), _hip.ptr(col), _hip.ptr(val),
+              ctypes.byref(h))
+    took = before - _raw()
+    _hip.call("sucem_csr_destroy", h)
+    assert 28 * nnz - (2 << 20) <= took <= 28 * nnz * 9 // 8 + (8 << 20), (took, 28 * nnz)
