@@ -151,12 +151,14 @@ int sucem_ctx_create(int device, void* hip_stream, sucem_ctx** out);
 int sucem_ctx_destroy(sucem_ctx* ctx);
 int sucem_ctx_synchronize(sucem_ctx* ctx);
 /* Device bytes held by the context's workspace; release frees it (the next solve
- * allocates again) and the unused blocks of the context's buffer pool (at most 4 GB).  (No reference counterpart: memory accounting for serving.) */
+ * allocates again) and the unused blocks of the context's buffer pool (the pools of a device
+ * keep at most 4 GB together).  (No reference counterpart: memory accounting for serving.) */
 int sucem_ctx_workspace_bytes(sucem_ctx* ctx, int64_t* bytes_h);
 int sucem_ctx_release_workspace(sucem_ctx* ctx);
-/* Free and total device memory of the context's device (hipMemGetInfo; free with the
- * unused blocks of the contexts' pools, which give way to allocations).  (No reference
- * counterpart: admission of requests by device memory.) */
+/* Free and total device memory of the context's device (hipMemGetInfo), after the unused
+ * blocks of the device's pools have been given back: what any allocation can have, the
+ * library's or another's.  Waits for the device's queued work if there were any.  (No
+ * reference counterpart: admission of requests by device memory.) */
 int sucem_ctx_mem_info(sucem_ctx* ctx, int64_t* free_h, int64_t* total_h);
 
 /* ---- mesh (replaces the DOLFIN Mesh handed to EMProblem.set_mesh, EMProblem.py:49-54) ---- */

@@ -176,9 +176,10 @@ int sucem_ctx_mem_info(sucem_ctx* ctx, int64_t* free_h, int64_t* total_h) {
   API_BEGIN
   NOT_NULL(ctx); NOT_NULL(free_h); NOT_NULL(total_h);
   ctx->c.use();
+  trim_pools(ctx->c.device);
   size_t fr = 0, tot = 0;
   SUCEM_HIP(hipMemGetInfo(&fr, &tot));
-  *free_h = (int64_t)(fr + pools_unused(ctx->c.device));
+  *free_h = (int64_t)fr;
   *total_h = (int64_t)tot;
   API_END
 }

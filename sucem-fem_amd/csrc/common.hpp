@@ -48,9 +48,12 @@ void set_last_error(const std::string& msg);
 // is only handed out to that context (whose stream orders the new use behind the old one).
 // Whoever frees memory that other streams may use has the device waited for first, as hipFree
 // does: the destroy entry points (DeviceWait) and members replaced while their owner lives
-// (DBuf::release_synced).  At most kMax bytes stay unused in one pool; blocks go back to the
-// device beyond that, when the context's workspace is released, when an allocation fails
-// (all pools give way), and with the context (buffers that outlive it free directly).
+// (DBuf::release_synced).  All pools of a device together keep at most kMax bytes unused, and
+// at most an eighth of the memory that would be free without them: allocations outside the
+// library (torch's) cannot make a pool give way.  Blocks go back to the device beyond that,
+// when the context's workspace is released, when free memory is asked for, when an allocation
+// of the library fails (all pools give way), and with the context (buffers that outlive it
+// free directly).
 class MemPool {
  public:
   static constexpr size_t kMax = size_t(4) << 30;
@@ -64,26 +67,49 @@ class MemPool {
   int device = -1;   // of its context
 
  private:
+  bool may_keep(size_t size);
   std::mutex mu_;
   std::multimap<size_t, void*> free_;
   size_t unused_ = 0;
+  // the device's free memory is looked at again (5 us) after kLook bytes more have come back
+  static constexpr size_t kLook = size_t(64) << 20;
+  size_t limit_ = 0, since_look_ = kLook;
   bool closed_ = false;
 };
 // The pool of the context that this thread's current entry point runs on (Context::use).
 std::shared_ptr<MemPool>& current_pool();
 std::shared_ptr<MemPool> new_pool();
-// unused bytes of all pools on a device: memory that an allocation there can have
-size_t pools_unused(int device);
+// every pool of a device gives its unused blocks back
+void trim_pools(int device);
 // hipMalloc; when it fails, once more after every pool has given its unused blocks back
 void* device_alloc(size_t bytes);
 // hipFree (which waits for all work on the device); a refusal leaves no error behind for the
 // thread's next launch to report
 bool device_free(void* p);
 
+// While it lives, this thread's allocations and frees are neither refused because of another
+// stream's capture nor end it (they belong to no graph).
+class BesideCaptures {
+ public:
+  BesideCaptures() {
+    if (hipThreadExchangeStreamCaptureMode(&mode_) != hipSuccess) {
+      (void)hipGetLastError();
+      changed_ = false;
+    }
+  }
+  ~BesideCaptures() {
+    if (changed_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+  }
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+  bool changed_ = true;
+};
+
 // Waits until the device's queued work is done, before buffers that any stream may use go back
 // to their pools.  Through hipFree of a small block (1.2 us on an idle device): a
 // hipDeviceSynchronize ends every stream capture of the process, that of another thread's
-// batched sweep among them.  Where even that is refused, the buffers that this thread releases
+// batched sweep among them.  Should that be refused, the buffers that this thread releases
 // while the object lives go to the device instead, which orders them itself.
 class DeviceWait {
  public:

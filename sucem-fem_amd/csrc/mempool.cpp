@@ -1,5 +1,6 @@
 // Device memory pools (declared in common.hpp).
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <new>
 
@@ -47,39 +48,48 @@ std::shared_ptr<MemPool> new_pool() {
   return p;
 }
 
-size_t pools_unused(int device) {
+namespace {
+
+std::vector<std::shared_ptr<MemPool>> live_pools() {
   PoolList& l = pool_list();
   std::lock_guard<std::mutex> hold(l.mu);
-  size_t n = 0;
+  std::vector<std::shared_ptr<MemPool>> pools;
   for (auto& w : l.all)
-    if (auto q = w.lock())
-      if (q->device == device) n += q->unused();
-  return n;
+    if (auto q = w.lock()) pools.push_back(q);
+  return pools;
+}
+
+// unused bytes of all pools of a device
+std::atomic<size_t>& kept_on(int device) {
+  static std::atomic<size_t> kept[256];
+  return kept[(unsigned)device % 256];
+}
+
+}  // namespace
+
+void trim_pools(int device) {
+  for (auto& q : live_pools())
+    if (q->device == device) q->trim();
 }
 
 void* device_alloc(size_t bytes) {
   void* p = nullptr;
   if (hipMalloc(&p, bytes) == hipSuccess) return p;
   (void)hipGetLastError();
-  std::vector<std::shared_ptr<MemPool>> pools;
-  {
-    PoolList& l = pool_list();
-    std::lock_guard<std::mutex> hold(l.mu);
-    for (auto& w : l.all)
-      if (auto q = w.lock()) pools.push_back(q);
-  }
-  for (auto& q : pools) q->trim();
+  for (auto& q : live_pools()) q->trim();
   SUCEM_HIP(hipMalloc(&p, bytes));
   return p;
 }
 
 bool device_free(void* p) {
+  const BesideCaptures beside;
   if (hipFree(p) == hipSuccess) return true;
   (void)hipGetLastError();
   return false;
 }
 
 DeviceWait::DeviceWait() : before_(bypass_pools()) {
+  const BesideCaptures beside;
   void* p = nullptr;
   if (hipMalloc(&p, 256) != hipSuccess) (void)hipGetLastError();
   if (!p || !device_free(p)) bypass_pools() = true;
@@ -101,6 +111,7 @@ void* MemPool::take(size_t bytes, size_t& got) {
       void* p = it->second;
       got = it->first;
       unused_ -= got;
+      kept_on(device) -= got;
       free_.erase(it);
       return p;
     }
@@ -121,10 +132,11 @@ void* MemPool::take(size_t bytes, size_t& got) {
 void MemPool::put(void* p, size_t size) {
   {
     std::lock_guard<std::mutex> hold(mu_);
-    if (!closed_ && unused_ + size <= kMax) {
+    if (!closed_ && may_keep(size)) {
       try {
         free_.emplace(size, p);
         unused_ += size;
+        kept_on(device) += size;
         return;
       } catch (const std::bad_alloc&) {   // (destructors call this) back to the device
       }
@@ -133,12 +145,32 @@ void MemPool::put(void* p, size_t size) {
   (void)device_free(p);
 }
 
+bool MemPool::may_keep(size_t size) {
+  if (size > kMax) return false;
+  since_look_ += size;
+  const size_t kept = kept_on(device);
+  if (since_look_ >= kLook) {
+    int current = -1;
+    size_t free_now = 0, total = 0;
+    if (hipGetDevice(&current) != hipSuccess || current != device ||
+        hipMemGetInfo(&free_now, &total) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    limit_ = std::min(kMax, (free_now + kept) / 8);
+    since_look_ = 0;
+  }
+  return kept + size <= limit_;
+}
+
 void MemPool::trim() {
   std::multimap<size_t, void*> old;
   {
     std::lock_guard<std::mutex> hold(mu_);
     old.swap(free_);
+    kept_on(device) -= unused_;
     unused_ = 0;
+    since_look_ = kLook;
   }
   for (auto& e : old) (void)device_free(e.second);   // waits for the work that may still use it
 }

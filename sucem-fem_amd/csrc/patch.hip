@@ -1136,16 +1136,13 @@ PtVectors pt_vectors(Context* c, const System* sys, const SpmvCfg& f, int64_t nv
   }
   if (cap != hipStreamCaptureStatusNone) return v;
   // (a capture of another stream does not forbid this call: its products go to no graph)
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  const BesideCaptures beside;
   try {
     v.part = c->ws.get(kWsPtVectors, (size_t)(fit * one));
     v.nvec = (int)fit;
   } catch (const Error&) {   // one by one then, as without the memory
     (void)hipGetLastError();
   }
-  if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
-  else (void)hipGetLastError();
   return v;
 }
 template PtVectors pt_vectors<float>(Context*, const System*, const SpmvCfg&, int64_t);

@@ -108,7 +108,8 @@ def footprint_bytes(req):
 
 
 def device_free_bytes(device=None):
-    """Free device memory (hipMemGetInfo through the library), or None without a device."""
+    """Free device memory (hipMemGetInfo through the library, once its pools have given their
+    unused buffers back), or None without a device."""
     try:
         import torch
         if not torch.cuda.is_available():
@@ -267,6 +268,15 @@ def device_executor(tol=1e-8, max_iter=50000, precision=64, eig_tol=1e-8, eig_in
         return local.stream, local.context
 
     def run(req):
+        try:
+            return attempt(req)
+        except torch.cuda.OutOfMemoryError:
+            # buffers that the slots' finished requests left in the library's pools do not give
+            # way to torch by themselves
+            device_free_bytes()
+        return attempt(req)
+
+    def attempt(req):
         stream, context = ctx()
         with torch.cuda.stream(stream):
             if req.kind == 'eigen':

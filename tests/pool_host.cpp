@@ -9,10 +9,11 @@
 namespace {
 
 struct Device {
-  size_t capacity = size_t(64) << 30, used = 0, next = 4096;
+  size_t capacity = size_t(288) << 30, used = 0, next = 4096;
   std::map<size_t, size_t> blocks;   // address -> bytes
   int mallocs = 0, frees = 0;
   bool refuse = false;   // as under another stream's global capture
+  hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;   // of the thread
   hipError_t last = hipSuccess;
 } dev;
 
@@ -48,6 +49,14 @@ hipError_t hipGetLastError(void) {
 hipError_t hipMemGetInfo(size_t* f, size_t* t) {
   *f = dev.capacity - dev.used;
   *t = dev.capacity;
+  return hipSuccess;
+}
+hipError_t hipGetDevice(int* d) {
+  *d = 0;
+  return hipSuccess;
+}
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
+  std::swap(*m, dev.mode);
   return hipSuccess;
 }
 // ends every capture of the process: nothing here may call it
@@ -188,6 +197,46 @@ int rounding() {
   return 0;
 }
 
+// the pools of a device keep kMax bytes together, and little of a device that is nearly full
+int shared_cap() {
+  Fixture f;
+  std::vector<std::shared_ptr<MemPool>> pools;
+  size_t kept = 0;
+  for (int i = 0; i < 3; ++i) {
+    pools.push_back(new_pool());
+    pools.back()->device = 0;
+    current_pool() = pools.back();
+    std::vector<DBuf<char>> a;
+    for (int j = 0; j < 5; ++j) a.emplace_back(512 * MB);
+    a.clear();
+    kept += pools.back()->unused();
+  }
+  CHECK(kept <= MemPool::kMax && kept > MemPool::kMax - 512 * MB && dev.used == kept);
+  trim_pools(0);
+  CHECK(dev.used == 0);
+  for (auto& q : pools) CHECK(q->unused() == 0);
+  // 8 GB free: an eighth of them may be kept, whatever is asked for
+  dev.capacity = 8 * GB;
+  for (int round = 0; round < 3; ++round) {
+    std::vector<DBuf<char>> a;
+    for (int j = 0; j < 40; ++j) a.emplace_back(96 * MB);
+    a.clear();
+    CHECK(dev.used <= GB && dev.used >= GB / 2);
+  }
+  // memory that others take lowers it at the next look
+  dev.capacity = dev.used + 2 * GB;
+  for (int round = 0; round < 3; ++round) {
+    std::vector<DBuf<char>> a;
+    for (int j = 0; j < 20; ++j) a.emplace_back(96 * MB);
+  }
+  CHECK(dev.used <= GB);
+  pools.clear();
+  current_pool().reset();
+  f.pool.reset();
+  CHECK(dev.used == 0 && dev.mode == hipStreamCaptureModeGlobal);
+  return 0;
+}
+
 // blocks are pooled after a wait for the device; where the wait is refused they never reach a
 // pool, and no error is left for the next launch
 int wait() {
@@ -227,7 +276,8 @@ int wait() {
 int main(int argc, char** argv) {
   const std::map<std::string, int (*)()> checks = {
       {"reuse", reuse}, {"cap", cap}, {"trim", trim}, {"full_device", full_device},
-      {"wait", wait}, {"rounding", rounding}};
+      {"wait", wait}, {"rounding", rounding},
+      {"shared_cap", shared_cap}};
   auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   return it->second();

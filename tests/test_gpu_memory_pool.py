@@ -163,36 +163,85 @@ def test_unused_blocks_count_as_free_memory():
     assert abs(before - after) < (64 << 20)
 
 
-def test_objects_dropped_by_another_thread_during_a_capture():
+def test_free_memory_is_what_any_allocation_can_have():
+    """The free memory reported to admission holds for torch too: the pools of every context
+    have given their idle blocks back by then."""
+    import torch
+    from sucemfem.Serving import device_free_bytes
+    from sucemfem.Utilities.Workloads import DeviceProblem
+    from sucemfem.runtime import Context
+    torch.cuda.set_device(0)
+    ctx = Context()
+    DeviceProblem((20, 20, 20), 0.6, 2, 7, (1.0, 2.2, 4.4), 0, ctx=ctx)
+    low = _raw()
+    told = device_free_bytes()
+    assert told - low > (128 << 20)
+    assert abs(_raw() - told) <= SLACK
+
+
+def test_request_survives_torch_running_out_of_memory(monkeypatch):
+    """A request whose vectors torch cannot allocate runs again once the pools' idle blocks are
+    free."""
+    import torch
+    from sucemfem.Serving import Request, Server, device_executor
+    from sucemfem.Utilities import Workloads
+    from sucemfem.runtime import Context
+    torch.cuda.set_device(0)
+    other = Context()
+    seen = []
+    rhs = Workloads.DeviceProblem.rhs_dipoles
+
+    def short_of_memory(self, *a, **kw):
+        if not seen:       # what another slot's request leaves behind
+            Workloads.DeviceProblem((20, 20, 20), 0.6, 2, 7, (1.0, 2.2, 4.4), 0, ctx=other)
+        seen.append(torch.cuda.mem_get_info()[0])
+        if len(seen) == 1:
+            raise torch.cuda.OutOfMemoryError("no memory for b")
+        return rhs(self, *a, **kw)
+
+    monkeypatch.setattr(Workloads.DeviceProblem, "rhs_dipoles", short_of_memory)
+    req = Request(0, "driven", (0.3, 0.2, 0.25), 4, 1, 0.0, freq=4e8)
+    (r,), _ = Server(device_executor(), slots=1).run([req], realtime=False)
+    assert r.status == "done", r.error
+    assert len(seen) == 2 and seen[1] - seen[0] > (128 << 20)
+
+
+@pytest.mark.parametrize("mode", ["relaxed", "global"])
+def test_objects_dropped_by_another_thread_during_a_capture(mode):
     """A thread that drops a mesh, its space and its system leaves a capture of another thread
-    alone (the batched sweep captures its iterations), and the next launch reports nothing."""
+    alone (the batched sweep captures its iterations), and the next launch reports nothing.
+    Free memory can be asked for as well."""
     import torch
     from sucemfem.Utilities.Workloads import DeviceProblem
     from sucemfem.runtime import Context
     torch.cuda.set_device(0)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        ctx = Context(stream=s)
+        ps = [DeviceProblem((3, 4, 2), 0.1, 2, 7, (1.0, 2.2, 4.4), 0, ctx=ctx),
+              DeviceProblem((2, 2, 2), 0.1, 1, 7, (1.0, 2.2, 4.4), 0, ctx=ctx)]
+        x = torch.ones(ps[1].ndofs, dtype=torch.complex128, device="cuda")
+        y, ref = torch.zeros_like(x), torch.zeros_like(x)
+        ps[1].apply(3.0, x, ref, precision=64)
     errs = []
 
     def drop():
         try:
             torch.cuda.set_device(0)
-            s = torch.cuda.Stream()
-            with torch.cuda.stream(s):
-                ctx = Context(stream=s)
-                for _ in range(2):
-                    p = DeviceProblem((3, 4, 2), 0.1, 2, 7, (1.0, 2.2, 4.4), 0, ctx=ctx)
-                    x = torch.ones(p.ndofs, dtype=torch.complex128, device="cuda")
-                    y = torch.zeros_like(x)
-                    del p
-                    p = DeviceProblem((2, 2, 2), 0.1, 1, 7, (1.0, 2.2, 4.4), 0, ctx=ctx)
-                    p.apply(3.0, x[:p.ndofs], y[:p.ndofs], precision=64)
-                    del p
+            del ps[0]
+            ps[0].apply(3.0, x, y, precision=64)
+            assert _free(ctx) > 0
+            if mode == "relaxed":
+                with torch.cuda.stream(s):
+                    DeviceProblem((2, 3, 2), 0.1, 2, 7, (1.0, 2.2, 4.4), 0, ctx=ctx)
+            del ps[0]
         except Exception as e:  # noqa: BLE001 - reported below
             errs.append(e)
 
     w = torch.ones(16, device="cuda")
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g, stream=torch.cuda.Stream(), capture_error_mode="relaxed"):
+    with torch.cuda.graph(g, stream=torch.cuda.Stream(), capture_error_mode=mode):
         t = threading.Thread(target=drop)
         t.start()
         t.join()
@@ -201,6 +250,7 @@ def test_objects_dropped_by_another_thread_during_a_capture():
     torch.cuda.synchronize()
     assert not errs, errs
     assert torch.all(w == 2.0)
+    assert torch.equal(y, ref)
 
 
 def test_sweeps_beside_a_thread_that_drops_problems():
