@@ -236,7 +236,7 @@ int sucem_system_tune(sucem_ctx* ctx, sucem_system* sys, int precision, int reps
  * 2 matrix-free per patch), lanes (4, 8, 16, 32; matrix-free: lanes per row of its gather,
  * 1 or 4, or 0 for one row per thread staged through LDS; patch: ignored), loads (1, 2, 4;
  * matrix-free: 1 = element rows in one pass, 2 = half the rows at a time; patch: cells
- * per patch, 128, 192 or 256 (order 1: 256)),
+ * per patch, 64, 128, 192 or 256 (order 1: 256)),
  * blocks (multiple of 8; patch: grid of the shared-DOF kernel)}.
  * Calls on one system must not overlap (the matrix-free element buffer is per system). */
 int sucem_system_set_spmv(sucem_ctx* ctx, sucem_system* sys, int precision, const int* cfg4_h);

@@ -422,9 +422,10 @@ int sucem_assemble(sucem_ctx* ctx, sucem_space* s, unsigned which, sucem_system*
   try {
     assemble_system(c, &s->s, &h->s, which);
     // default operator: matrix-free wherever it applies (5-8x faster than the tuned
-    // assembled CSR on a 2.5M-DOF order-2 system), in its patch form (patches of 256
-    // cells for FP32 and 192 for FP64 at order 2, 256 at order 1) where the device holds
-    // the patch's LDS, else per cell; sucem_system_tune / _set_spmv override
+    // assembled CSR on a 2.5M-DOF order-2 system), in its patch form (patches of 64 cells
+    // on small meshes, else 256 for FP32 and 192 for FP64 at order 2, 256 at order 1: see
+    // pt_default_cb) where the device holds the patch's LDS, else per cell;
+    // sucem_system_tune / _set_spmv override
     const unsigned st = SUCEM_MAT_S | SUCEM_MAT_T;
     if ((which & st) == st && (s->s.nloc == 6 || s->s.nloc == 20)) {
       mf_prepare(c, &h->s);
@@ -520,8 +521,10 @@ int sucem_system_set_spmv(sucem_ctx* ctx, sucem_system* sys, int precision, cons
   Context* c = &ctx->c;
   c->use();
   if (f.mf == 2) {
-    SUCEM_CHECK(f.U == 128 || f.U == 192 || f.U == 256, SUCEM_ERR_INVALID,
-                "patch operator: loads (cells per patch) must be 128, 192 or 256");
+    SUCEM_CHECK(f.U == 128 || f.U == 192 || f.U == 256 ||
+                    (f.U == 64 && sys->s.space->order == 2),
+                SUCEM_ERR_INVALID,
+                "patch operator: loads (cells per patch) must be 64 (order 2), 128, 192 or 256");
     SUCEM_CHECK(sys->s.space->order == 2 || f.U == 256, SUCEM_ERR_UNSUPPORTED,
                 "patch operator: order-1 patches hold 256 cells");
     SUCEM_CHECK(pt_prepare(c, &sys->s, f.U), SUCEM_ERR_UNSUPPORTED,
@@ -555,8 +558,8 @@ int sucem_system_set_spmv(sucem_ctx* ctx, sucem_system* sys, int precision, cons
 int sucem_system_patch_info(sucem_ctx* ctx, sucem_system* sys, int cb, int64_t* info6_h) {
   API_BEGIN
   NOT_NULL(ctx); NOT_NULL(sys); NOT_NULL(info6_h);
-  SUCEM_CHECK(cb == 128 || cb == 192 || cb == 256, SUCEM_ERR_INVALID,
-              "cells per patch must be 128, 192 or 256");
+  SUCEM_CHECK(cb == 128 || cb == 192 || cb == 256 || (cb == 64 && sys->s.space->order == 2),
+              SUCEM_ERR_INVALID, "cells per patch must be 64 (order 2), 128, 192 or 256");
   Context* c = &ctx->c;
   c->use();
   SUCEM_CHECK(pt_prepare(c, &sys->s, cb), SUCEM_ERR_UNSUPPORTED,

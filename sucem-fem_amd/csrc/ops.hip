@@ -525,9 +525,9 @@ SpmvCfg sys_cfg(Context* c, const System* sys) {
   const SpmvCfg& t = sys->cfg[sizeof(R) == 4 ? 0 : 1];
   if (t.L > 0 || t.mf) return t;
   // Nothing tuned or set: the patch operator (what the autotuner picks on the driven
-  // cubes, 8-10x faster than the assembled CSR operator), with the patch size it picks
-  // (FP64 order 2: 192 cells, else 256), when the space suits it; the choice is kept on
-  // the system (its maps and coefficients are lazily built caches of the system).
+  // cubes, 8-10x faster than the assembled CSR operator), with the patch size that suits the
+  // mesh (pt_default_cb), when the space suits it; the choice is kept on the system (its
+  // maps and coefficients are lazily built caches of the system).
   System* ms = const_cast<System*>(sys);
   const int cb = pt_default_cb<R>(sys->space);
   if (sys->space->nloc == 6 || sys->space->nloc == 20) {
@@ -611,7 +611,7 @@ SpmvCfg tune_sys(Context* c, System* sys, int reps) {
           time_cfg(f);
         }
     // patch operator: element products summed per patch of cells in LDS + shared-DOF sums
-    for (int cb : {128, 192, 256}) {
+    for (int cb : {64, 128, 192, 256}) {
       if ((s->order == 1 && cb != 256) || !pt_prepare(c, sys, cb) || !pt_fits<R>(s, cb)) continue;
       const int64_t npd = pt_maps(s, cb).npd;
       for (int pc : {4, 16}) {

@@ -3,8 +3,8 @@
 // The per-cell form (matfree.hip) writes every element product to HBM and reads it back
 // in a second kernel that sums each DOF's products.  Here the cells are ordered along a
 // Morton curve of their centroids and cut into patches of CB consecutive cells (compact
-// clusters of the mesh; CB = 128, 192 or 256, chosen by the autotuner, or 64 on small
-// meshes), one workgroup per patch:
+// clusters of the mesh; CB = 64, 128, 192 or 256, by default after the mesh's size, see
+// pt_default_cb), one workgroup per patch:
 //
 //  1. the patch's DOFs ("patch DOFs": the union of its cells' DOFs, ~1.4 per DOF of the
 //     mesh) are gathered from x into LDS once;

@@ -187,7 +187,8 @@ class DeviceProblem(object):
         """Select the operator explicitly (see ``tune``): matrix_free 0 (assembled CSR: lanes
         per row, loads per lane), 1 (per-cell element products: lanes per gather row 0, 1, 4;
         loads 1 = whole element, 2 = half the rows at a time) or 2 (patches: loads = cells
-        per patch, 128, 192 or 256); blocks = grid of the row / shared-DOF kernel."""
+        per patch, 64, 128, 192 or 256; order 1: 256); blocks = grid of the row / shared-DOF
+        kernel."""
         cfg = np.array([matrix_free, lanes, loads, blocks], np.int32)
         _hip.call("sucem_system_set_spmv", self.ctx.handle, self.system.handle.h, int(precision),
                   _hip.ptr(cfg))
