@@ -123,9 +123,13 @@ __global__ void k_copy(int n, int G, const C* src, C* dst) {
 // Sum of the G <= FOLD_MAX block partials part[0, G), in every block the same and bit for bit
 // what k_finalize gets: the kernel that needs a scalar then forms it itself, and the
 // one-block launch between producer and consumer (4.4 us, as long as the kernels around it on
-// small systems) is saved.  Beyond FOLD_MAX partials, reading them in every block would cost
-// more than that launch.
-constexpr int FOLD_MAX = 1024;
+// small systems) is saved.  Beyond FOLD_MAX partials (64 rows each), reading them in every
+// block would cost more than that launch; BiCGStab, whose omega and beta take two sums each,
+// is there at FOLD_MAX_BICG.  Jacobi iteration with separate launches / folded, 11 entries per
+// row, FP64, us (runs differ by up to 1 us): COCG 2,000 rows 15.8 / 14.5, 30,000 17.8 / 14.7,
+// 48,000 18.4 / 17.0, 65,000 19.3 / 18.4; BiCGStab 25.9 / 24.8, 27.7 / 25.1, 29.5 / 30.0,
+// 31.4 / 33.6.
+constexpr int FOLD_MAX = 1024, FOLD_MAX_BICG = 768;
 __device__ __forceinline__ double2 sum_parts(const double2* part, int G) {
   constexpr int W = TB / 64, Q = FOLD_MAX / TB;   // waves, segments of 64 per wave
   __shared__ double2 seg[FOLD_MAX / 64];
@@ -739,7 +743,8 @@ void krylov(Op& op, const double2* b, double2* x, const SolveOpts& o, SolveStats
   // beta is left to the next p update except before a host check, which reads the history
   // entry that comes with it (`due_b`).  BiCGStab with Jacobi on 4,125 rows: 8 launches of an
   // iteration become 5, 24.8 -> 21.5 us.
-  const bool fold = !grad && op.flo.parts() <= FOLD_MAX && G <= FOLD_MAX;
+  const int fold_max = cocg ? FOLD_MAX : FOLD_MAX_BICG;
+  const bool fold = !grad && op.flo.parts() <= fold_max && G <= fold_max;
   const int Ga = fold ? op.flo.parts() : 0, Gf = fold ? G : 0;
   int due_b = 0;
   RedSite last_b{};

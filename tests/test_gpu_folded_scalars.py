@@ -7,11 +7,11 @@ import scipy.sparse as sp
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 7, 64, 65, 4097, 66000])
+@pytest.mark.parametrize("n", [1, 7, 64, 65, 4097, 49152, 49153, 65537, 66000])
 @pytest.mark.parametrize("precision", [64, 32])
 def test_check_interval_and_solution(n, precision):
     """Diagonally dominant complex systems (66,000 rows: too many partials, the separate
-    launches).  The histories of the first iterations are those of check_every = 1 (its
+    launches; BiCGStab uses those from 49,153 rows on).  The histories of the first iterations are those of check_every = 1 (its
     scalars come from the finalising kernel every time): the sums are equal bit for bit, the
     two or three roundings of a scalar's formula may be contracted differently in another
     kernel (1e-16 each, 1e-12 over six iterations of a well-conditioned system).  The
