@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
@@ -71,9 +72,11 @@ class MemPool {
   std::mutex mu_;
   std::multimap<size_t, void*> free_;
   size_t unused_ = 0;
-  // the device's free memory is looked at again (5 us) after kLook bytes more have come back
-  static constexpr size_t kLook = size_t(64) << 20;
-  size_t limit_ = 0, since_look_ = kLook;
+  // The device's free memory is looked at again after kLookMs: a look takes 5 to 11 us, and
+  // one for every 64 MB that came back made up 3 % of a far-field transform.
+  static constexpr int kLookMs = 50;
+  size_t limit_ = 0;
+  std::chrono::steady_clock::time_point looked_{};
   bool closed_ = false;
 };
 // The pool of the context that this thread's current entry point runs on (Context::use).

@@ -147,9 +147,9 @@ void MemPool::put(void* p, size_t size) {
 
 bool MemPool::may_keep(size_t size) {
   if (size > kMax) return false;
-  since_look_ += size;
   const size_t kept = kept_on(device);
-  if (since_look_ >= kLook) {
+  const auto now = std::chrono::steady_clock::now();
+  if (now - looked_ >= std::chrono::milliseconds(kLookMs)) {
     int current = -1;
     size_t free_now = 0, total = 0;
     if (hipGetDevice(&current) != hipSuccess || current != device ||
@@ -158,7 +158,7 @@ bool MemPool::may_keep(size_t size) {
       return false;
     }
     limit_ = std::min(kMax, (free_now + kept) / 8);
-    since_look_ = 0;
+    looked_ = now;
   }
   return kept + size <= limit_;
 }
@@ -170,7 +170,7 @@ void MemPool::trim() {
     old.swap(free_);
     kept_on(device) -= unused_;
     unused_ = 0;
-    since_look_ = kLook;
+    looked_ = {};
   }
   for (auto& e : old) (void)device_free(e.second);   // waits for the work that may still use it
 }
