@@ -195,7 +195,9 @@ __global__ void k_csr_identity_dinv(int64_t n, const uint8_t* mask, typename C2<
 // bounding box, so that only points in it meet the cells themselves: one box test per 64
 // cell-point pairs instead of 64 tetrahedron tests (which bound this kernel by FP64
 // arithmetic).  The box is enlarged far beyond the tolerance and the rounding of the
-// tetrahedron test.  51,840 cells, 1,200 to 4,000 points: 586 -> 113 us.
+// tetrahedron test.  51,840 cells, 1,200 to 4,000 points: 586 -> 113 us; cells in random order,
+// whose boxes are the whole mesh's, gain less (a call with 4,000 points 1,012 -> 636 us, against
+// 860 -> 70 us in order).
 __global__ __launch_bounds__(TB) void k_locate(int64_t nc, const double* xyz, const int32_t* cells,
                                                int64_t n, const double* pts, double tol,
                                                int32_t* out) {

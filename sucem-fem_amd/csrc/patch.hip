@@ -1002,8 +1002,11 @@ template bool pt_fits<double>(const Space*, int);
 // workgroup per CU, and the operator is then one workgroup's chain of loads.  Operator in
 // the solve, 256 / 192 cells (FP32 / FP64) against 64, us: 6,468 cells 19.8 / 22.8 -> 12.5 /
 // 13.9; 29,172 cells 20.9 / 24.5 -> 14.7 / 17.2; 82,944 cells 24.6 / 29.9 against 23.8 /
-// 34.3; 162,000 cells 30.3 / 48.0 against 34.7 / 52.2.  Order 1 gains nothing (48,000
-// cells: 9.8 / 10.3 against 10.5 / 11.1).
+// 34.3; 162,000 cells 30.3 / 48.0 against 34.7 / 52.2.  Around the limit, whole iterations of
+// the solve: 48,000 cells 42.2 / 46.9 against 34.9 / 47.6; 58,212 cells 42.6 / 54.3 against
+// 39.8 / 52.0; 69,696 cells 46.0 / 56.4 against 43.5 / 58.0: FP64 is even from 48,000 cells on
+// and FP32 gains up to 70,000, so one limit serves both where neither loses.  Order 1 gains
+// nothing (48,000 cells: 9.8 / 10.3 against 10.5 / 11.1).
 constexpr int64_t kSmallCells = 50000;
 template <typename R>
 int pt_default_cb(const Space* s) {

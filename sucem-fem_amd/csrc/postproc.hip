@@ -186,6 +186,9 @@ __device__ inline void cross_c(const double n[3], const double2 v[3], double2 ou
 // on how many are asked for.  part[(q nd + d) 2 NC + k]: the sums of chunk q.
 // 264,000 points, 181 directions: 597 us (one block row per direction) -> 110 us; the
 // boundary DOFs' sums of the variational form, which ran over all cells, 783 -> 39 us.
+// FF_FEW: a surface transform (79,200 points) of 4 / 16 / 17 / 32 / 48 / 181 directions takes
+// 120 / 123 / 137 / 139 / 159 / 328 us with k_ff_few and 134 / 136 / 137 / 136 / 138 / 209 us
+// with k_ff_sums.
 constexpr int FF_TILE = 64, FF_SL = 4, FF_DL = TB / FF_SL, FF_CHUNKS = 1024, FF_FEW = 16;
 
 // NC = 6: w (n x H), w (n x E) of the boundary samples

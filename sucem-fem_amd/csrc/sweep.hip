@@ -26,10 +26,15 @@
 //
 // Meshes of more than 2,048 patches, or with a DOF in more than 15 of them, run the shared
 // rows, alpha and beta as launches of their own (k_sw_psum, k_sw_alpha, k_sw_beta) around
-// k_sw_xr and k_sw_pz: every block summing that many partials would cost more than the three
-// launches.  Iteration with eight / five launches, us, FP32 / FP64, groups of 2: 48,000
-// order-1 cells 45.7 / 49.6 -> 32.4 / 34.4; 384,000 90.0 / 112.1 -> 73.5 / 94.6; 48,000
-// order-2 cells 105.8 / 121.8 -> 88.7 / 101.2 (the operator's batched loads included).
+// k_sw_xr and k_sw_pz: the sums that every block then forms grow with the patches.  Iteration
+// with eight / five launches, us, groups of 2 FP32, FP64, groups of 8 FP32, FP64 (order 1):
+//    48,000 cells   39.5 / 29.0   41.6 / 31.6   67.9 / 57.8   77.7 / 67.1
+//   196,608 cells   54.2 / 45.9   62.5 / 54.1   121 / 119     199 / 194
+//   384,000 cells   79.8 / 71.0   102 / 89      219 / 226     385 / 386
+//   522,720 cells   94.6 / 84.2   146 / 135     296 / 308     532 / 526   (2,042 patches)
+//   750,000 cells   120 / 110     203 / 192     410 / 436     772 / 763   (eight are run)
+// Groups of 2, which the tuner mostly picks, would gain beyond the limit too; groups of 8 in
+// FP32 lose from 384,000 cells on.
 //
 // The check interval's iterations (fixed launches, device-resident scalars) are captured
 // once per solve in a hipGraph on a library stream and replayed; between replays the host
