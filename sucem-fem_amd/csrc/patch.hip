@@ -343,6 +343,7 @@ __device__ __forceinline__ T at32(const T* base, uint32_t idx) {
 // bounds, destinations, epilogue operands and mask bytes of a whole batch are in flight
 // together, and the first two products of every segment are read before any is summed.
 // Per application in the solve at 40^3 order 2: FP32 60.9 -> 54.8 us, FP64 111 -> 97.8 us
+// without the p update (with it, below, the FP64 kernel takes 104 us)
 // (there the places that are read again instead of held also take the kernel from 274 to
 // 246 registers, one wave per SIMD to two); 17 x 22 x 13 boxes with the 64-cell patches
 // 24.4 -> 14.7 and 26.7 -> 17.2 us.
