@@ -51,10 +51,11 @@ void set_last_error(const std::string& msg);
 // does: the destroy entry points (DeviceWait) and members replaced while their owner lives
 // (DBuf::release_synced).  All pools of a device together keep at most kMax bytes unused, and
 // at most an eighth of the memory that would be free without them: allocations outside the
-// library (torch's) cannot make a pool give way.  Blocks go back to the device beyond that,
-// when the context's workspace is released, when free memory is asked for, when an allocation
-// of the library fails (all pools give way), and with the context (buffers that outlive it
-// free directly).
+// library (torch's) cannot make a pool give way.  Blocks go back to the device beyond that (those
+// first that nobody has asked for in a second: a program that went on to other meshes would
+// otherwise find the pools full of sizes that it no longer needs), when the context's workspace
+// is released, when free memory is asked for, when an allocation of the library fails (all
+// pools give way), and with the context (buffers that outlive it free directly).
 class MemPool {
  public:
   static constexpr size_t kMax = size_t(4) << 30;
@@ -68,15 +69,24 @@ class MemPool {
   int device = -1;   // of its context
 
  private:
-  bool may_keep(size_t size);
+  using Clock = std::chrono::steady_clock;
+  struct Block {
+    void* p;
+    Clock::time_point since;
+  };
+  bool keep(void* p, size_t size, Clock::time_point now);
+  bool drop_idle(Clock::time_point now);   // blocks unused for kIdleMs; whether there were any
+  bool look(Clock::time_point now);        // limit_ up to date, if the device says so
+  static constexpr int kIdleMs = 1000;
   std::mutex mu_;
-  std::multimap<size_t, void*> free_;
+  std::multimap<size_t, Block> free_;
+  Clock::time_point oldest_{};             // no block has been unused for longer
   size_t unused_ = 0;
   // The device's free memory is looked at again after kLookMs: a look takes 5 to 11 us, and
   // one for every 64 MB that came back made up 3 % of a far-field transform.
   static constexpr int kLookMs = 50;
   size_t limit_ = 0;
-  std::chrono::steady_clock::time_point looked_{};
+  Clock::time_point looked_{};
   bool closed_ = false;
 };
 // The pool of the context that this thread's current entry point runs on (Context::use).

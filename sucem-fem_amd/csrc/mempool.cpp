@@ -108,7 +108,7 @@ void* MemPool::take(size_t bytes, size_t& got) {
     std::lock_guard<std::mutex> hold(mu_);
     auto it = free_.lower_bound(want);
     if (it != free_.end() && it->first <= std::max(want, bytes + bytes / 8)) {
-      void* p = it->second;
+      void* p = it->second.p;
       got = it->first;
       unused_ -= got;
       kept_on(device) -= got;
@@ -130,26 +130,62 @@ void* MemPool::take(size_t bytes, size_t& got) {
 }
 
 void MemPool::put(void* p, size_t size) {
-  {
-    std::lock_guard<std::mutex> hold(mu_);
-    if (!closed_ && may_keep(size)) {
-      try {
-        free_.emplace(size, p);
-        unused_ += size;
-        kept_on(device) += size;
-        return;
-      } catch (const std::bad_alloc&) {   // (destructors call this) back to the device
-      }
-    }
+  const auto now = Clock::now();
+  try {   // (destructors call this: what cannot be kept goes back to the device)
+    if (keep(p, size, now)) return;
+    bool dropped = false;
+    if (size <= kMax)
+      for (auto& q : live_pools())
+        if (q->device == device && q->drop_idle(now)) dropped = true;
+    if (dropped && keep(p, size, now)) return;
+  } catch (const std::bad_alloc&) {
   }
   (void)device_free(p);
 }
 
-bool MemPool::may_keep(size_t size) {
-  if (size > kMax) return false;
-  const size_t kept = kept_on(device);
-  const auto now = std::chrono::steady_clock::now();
+bool MemPool::keep(void* p, size_t size, Clock::time_point now) {
+  std::lock_guard<std::mutex> hold(mu_);
+  if (closed_ || size > kMax || !look(now)) return false;
+  if (kept_on(device).fetch_add(size) + size > limit_) {
+    kept_on(device) -= size;
+    return false;
+  }
+  try {
+    free_.emplace(size, Block{p, now});
+  } catch (const std::bad_alloc&) {
+    kept_on(device) -= size;
+    throw;
+  }
+  unused_ += size;
+  return true;
+}
+
+bool MemPool::drop_idle(Clock::time_point now) {
+  const auto old = now - std::chrono::milliseconds(kIdleMs);
+  std::vector<void*> drop;
+  {
+    std::lock_guard<std::mutex> hold(mu_);
+    if (oldest_ > old) return false;
+    oldest_ = now;
+    for (auto it = free_.begin(); it != free_.end();) {
+      if (it->second.since > old) {
+        oldest_ = std::min(oldest_, it->second.since);
+        ++it;
+        continue;
+      }
+      drop.push_back(it->second.p);
+      unused_ -= it->first;
+      kept_on(device) -= it->first;
+      it = free_.erase(it);
+    }
+  }
+  for (void* q : drop) (void)device_free(q);   // waits for the work that may still use it
+  return !drop.empty();
+}
+
+bool MemPool::look(Clock::time_point now) {
   if (now - looked_ >= std::chrono::milliseconds(kLookMs)) {
+    const size_t kept = kept_on(device);
     int current = -1;
     size_t free_now = 0, total = 0;
     if (hipGetDevice(&current) != hipSuccess || current != device ||
@@ -160,11 +196,11 @@ bool MemPool::may_keep(size_t size) {
     limit_ = std::min(kMax, (free_now + kept) / 8);
     looked_ = now;
   }
-  return kept + size <= limit_;
+  return true;
 }
 
 void MemPool::trim() {
-  std::multimap<size_t, void*> old;
+  std::multimap<size_t, Block> old;
   {
     std::lock_guard<std::mutex> hold(mu_);
     old.swap(free_);
@@ -172,7 +208,7 @@ void MemPool::trim() {
     unused_ = 0;
     looked_ = {};
   }
-  for (auto& e : old) (void)device_free(e.second);   // waits for the work that may still use it
+  for (auto& e : old) (void)device_free(e.second.p);   // waits for the work that may still use it
 }
 
 size_t MemPool::unused() {

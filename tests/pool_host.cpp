@@ -248,6 +248,32 @@ int shared_cap() {
   return 0;
 }
 
+// a full pool makes room by giving back what nobody has asked for in a second, its own and
+// other pools' blocks, and nothing younger
+int idle() {
+  Fixture f;
+  auto other = new_pool();
+  other->device = 0;
+  auto fill = [&](const std::shared_ptr<MemPool>& p, int n, size_t size) {
+    current_pool() = p;
+    std::vector<DBuf<char>> a;
+    for (int i = 0; i < n; ++i) a.emplace_back(size);
+  };
+  fill(f.pool, 4, 512 * MB);
+  fill(other, 4, 512 * MB);
+  CHECK(dev.used == 4 * GB && f.pool->unused() + other->unused() == 4 * GB);
+  fill(f.pool, 1, 96 * MB);
+  CHECK(dev.used == 4 * GB);   // full, and nothing is old: the block went back
+  std::this_thread::sleep_for(std::chrono::milliseconds(1100));
+  fill(other, 1, 512 * MB);    // in use again: young
+  fill(f.pool, 1, 96 * MB);
+  CHECK(f.pool->unused() == 96 * MB && other->unused() == 512 * MB);
+  CHECK(dev.used == 608 * MB);
+  fill(f.pool, 20, 160 * MB);
+  CHECK(dev.used <= 4 * GB && f.pool->unused() > 3 * GB && other->unused() == 512 * MB);
+  return 0;
+}
+
 // blocks are pooled after a wait for the device; where the wait is refused they never reach a
 // pool, and no error is left for the next launch
 int wait() {
@@ -288,7 +314,7 @@ int main(int argc, char** argv) {
   const std::map<std::string, int (*)()> checks = {
       {"reuse", reuse}, {"cap", cap}, {"trim", trim}, {"full_device", full_device},
       {"wait", wait}, {"rounding", rounding},
-      {"shared_cap", shared_cap}};
+      {"shared_cap", shared_cap}, {"idle", idle}};
   auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   return it->second();

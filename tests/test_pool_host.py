@@ -18,7 +18,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["reuse", "cap", "trim", "full_device", "wait", "rounding", "shared_cap"])
+@pytest.mark.parametrize("check", ["reuse", "cap", "trim", "full_device", "wait", "rounding", "shared_cap", "idle"])
 def test_pool(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
