@@ -319,7 +319,7 @@ int sucem_mesh_destroy(sucem_mesh* m) {
   API_BEGIN
   if (!m) return SUCEM_OK;
   (void)hipSetDevice(m->m.ctx->device);
-  const DeviceWait wait;   // other contexts' streams may still read it
+  const DeviceWait wait(m->m.ctx->stream);   // other contexts' streams may still read it
   delete m;
   API_END
 }
@@ -406,7 +406,7 @@ int sucem_space_destroy(sucem_space* s) {
   API_BEGIN
   if (!s) return SUCEM_OK;
   (void)hipSetDevice(s->s.ctx->device);
-  const DeviceWait wait;   // other contexts' streams may still read it
+  const DeviceWait wait(s->s.ctx->stream);   // other contexts' streams may still read it
   delete s;
   API_END
 }
@@ -475,7 +475,7 @@ int sucem_system_destroy(sucem_system* sys) {
   API_BEGIN
   if (!sys) return SUCEM_OK;
   (void)hipSetDevice(sys->s.ctx->device);
-  const DeviceWait wait;   // other contexts' streams may still read it
+  const DeviceWait wait(sys->s.ctx->stream);   // other contexts' streams may still read it
   delete sys;
   API_END
 }
@@ -1003,7 +1003,7 @@ int sucem_csr_destroy(sucem_csr* A) {
   API_BEGIN
   if (!A) return SUCEM_OK;
   (void)hipSetDevice(A->a.ctx->device);
-  const DeviceWait wait;   // other contexts' streams may still read it
+  const DeviceWait wait(A->a.ctx->stream);   // other contexts' streams may still read it
   delete A;
   API_END
 }

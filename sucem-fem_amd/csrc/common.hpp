@@ -120,13 +120,14 @@ class BesideCaptures {
 };
 
 // Waits until the device's queued work is done, before buffers that any stream may use go back
-// to their pools.  Through hipFree of a small block (1.2 us on an idle device): a
+// to their pools.  Through hipFree of a small block (1.2 us on an idle device, some 100 us behind
+// a stream that has not been waited for, so the owner's stream is waited for first): a
 // hipDeviceSynchronize ends every stream capture of the process, that of another thread's
 // batched sweep among them.  Should that be refused, the buffers that this thread releases
 // while the object lives go to the device instead, which orders them itself.
 class DeviceWait {
  public:
-  DeviceWait();
+  explicit DeviceWait(hipStream_t owners);
   ~DeviceWait() { bypass_pools() = before_; }
   static bool& bypass_pools();   // of this thread
 

@@ -88,8 +88,12 @@ bool device_free(void* p) {
   return false;
 }
 
-DeviceWait::DeviceWait() : before_(bypass_pools()) {
+DeviceWait::DeviceWait(hipStream_t owners) : before_(bypass_pools()) {
   const BesideCaptures beside;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(owners, &cap) != hipSuccess ||
+      (cap == hipStreamCaptureStatusNone && hipStreamSynchronize(owners) != hipSuccess))
+    (void)hipGetLastError();
   void* p = nullptr;
   if (hipMalloc(&p, 256) != hipSuccess) (void)hipGetLastError();
   if (!p || !device_free(p)) bypass_pools() = true;

@@ -42,6 +42,12 @@ hipError_t hipFree(void* p) {
   dev.blocks.erase(it);
   return hipSuccess;
 }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
+  if (dev.refuse) return fail(hipErrorStreamCaptureImplicit);
+  *s = hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError(void) {
   const hipError_t e = dev.last;
   dev.last = hipSuccess;
@@ -281,7 +287,7 @@ int wait() {
   DBuf<char> a(MB), b(MB), c(MB);
   {
     const int frees = dev.frees;
-    const DeviceWait w;
+    const DeviceWait w(nullptr);
     CHECK(dev.frees == frees + 1);   // hipFree waits
     a.release();
   }
@@ -289,13 +295,13 @@ int wait() {
   const size_t idle = f.pool->unused();
   {
     dev.refuse = true;
-    const DeviceWait w;
+    const DeviceWait w(nullptr);
     b.release();
   }
   CHECK(f.pool->unused() == idle && dev.last == hipSuccess);
   dev.refuse = false;
   {
-    const DeviceWait w;
+    const DeviceWait w(nullptr);
   }
   {
     const int frees = dev.frees;
