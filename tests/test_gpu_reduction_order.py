@@ -1,4 +1,4 @@
-"""Sums over lanes: the dot products behind COCG keep their butterfly order."""
+"""Sums over lanes, waves and blocks behind COCG's scalars: every row once."""
 import numpy as np
 import pytest
 
